@@ -189,7 +189,8 @@ def main():
     ap.add_argument("--no-batch", action="store_true", help="skip the batched 64-sample mix")
     ap.add_argument("--batch-samples", type=int, default=64)
     ap.add_argument("--batch-steps", type=int, default=1)
-    ap.add_argument("--no-graph", action="store_true", help="launch the batch's radix passes one by one")
+    ap.add_argument("--graph", action="store_true",
+                    help="the batch by radix passes replayed from a captured graph, instead of by minimizer bins")
     ap.add_argument("--no-serve", action="store_true", help="skip the served workload")
     ap.add_argument("--serve-jobs", type=int, default=200)
     ap.add_argument("--serve-engines", type=int, default=3)
@@ -269,6 +270,7 @@ def main():
     sc = plain["scan"]
     n = int(sc["tuples"])
     N = args.reads
+    by_bins = float(sc["ms_sort_gen"]) == 0  # the scan went by minimizer bins: no radix pass ran
     passes = int(sc["sort_passes"])
     pass_ms = float(sc["ms_sort_pass_avg"])
     per_pass_bytes = 2 * TUPLE_BYTES * n  # read and write 13 B per tuple
@@ -287,7 +289,10 @@ def main():
     else:  # enumerated tuples: one histogram read (k-mers), then every pass reads and writes them
         sort_bytes = n * (8 + 2 * full * TUPLE_BYTES) + local_bytes
     sort_ms = float(sc["ms_sort"])
-    traffic = measured_traffic(args.reads)
+    traffic = None if by_bins else measured_traffic(args.reads)
+    runs_ms = float(sc["ms_sort_local"])
+    # what building the runs cannot do without: the 2-bit and 'N' streams read once, a label per tuple written
+    runs_bytes = bases * 3 // 8 + 4 * n
 
     def stage(ms, nbytes, what):
         gbs = nbytes / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
@@ -307,6 +312,28 @@ def main():
         "union": stage(float(sc["ms_union"]), n // 4 + 4 * n, "run bitmaps and the labels (random parent "
                                                               "accesses not counted)"),
     }
+    roofline = {"bound": "hbm", "kernel": "onesweep_kernel (one radix scatter pass)", "achieved": achieved,
+                "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                "traffic": traffic["bytes"] if traffic else None,
+                "traffic_source": traffic["source"] if traffic else None,
+                "bytes_per_launch": per_pass_bytes, "launch_ms": pass_ms, "tuples": n}
+    sort = {"passes": passes, "digit_bits": 8, "tuple_bytes": TUPLE_BYTES, "algorithmic_bytes": sort_bytes,
+            "ms": sort_ms, "hbm_frac": sort_bytes / (sort_ms * 1e-3) / 1e12 / (HBM_PEAK_GBS / 1e3)
+            if sort_ms > 0 else 0.0}
+    if by_bins:
+        ms = float(sc["ms_enumerate"]) + sort_ms
+        gbs = runs_bytes / (runs_ms * 1e-3) / 1e9 if runs_ms > 0 else 0.0
+        stages = {
+            "bin_records": stage(float(sc["ms_enumerate"]), bases * 3 // 8, "2-bit and 'N' streams read"),
+            "bin_runs": stage(runs_ms, runs_bytes, "0.375 B per base read, 4 B per tuple written at most (the kernels "
+                                                   "that build the runs and evaluate the filter)"),
+            "refilter": stage(float(sc["ms_filter"]), 2 * N, "filtered and BAD flags"),
+            "union": stages["union"]}
+        roofline = {"bound": "lds", "kernel": "bin_runs_kernel (runs of equal k-mers in LDS tables, filter)",
+                    "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS, "traffic": None,
+                    "traffic_source": None, "bytes_per_launch": runs_bytes, "launch_ms": runs_ms, "tuples": n}
+        sort = {"passes": passes, "by": "minimizer bins (no radix pass)", "algorithmic_bytes": runs_bytes, "ms": ms,
+                "hbm_frac": runs_bytes / (ms * 1e-3) / 1e12 / (HBM_PEAK_GBS / 1e3) if ms > 0 else 0.0}
     out = {
         "metric": "reads partitioned/s at k=31 on 1 GPU (plain path); % HBM peak in sort",
         "value": plain["reads_per_s"],
@@ -323,14 +350,8 @@ def main():
         "config": {"workload": "200 genomes 1-5 Mb GC U(0.3,0.7) + 10x5 kb repeats; %d SE reads x 150 bp, 1%% error; "
                                "k=%d m=10, 16 chunks, S=1, T=1, plain" % (args.reads, args.k),
                    "reads": args.reads, "k": args.k, "chunks": args.chunks, "scans": 1, "segments": 1},
-        "roofline": {"bound": "hbm", "kernel": "onesweep_kernel (one radix scatter pass)", "achieved": achieved,
-                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": traffic["bytes"] if traffic else None,
-                     "traffic_source": traffic["source"] if traffic else None,
-                     "bytes_per_launch": per_pass_bytes, "launch_ms": pass_ms, "tuples": n},
-        "sort": {"passes": passes, "digit_bits": 8, "tuple_bytes": TUPLE_BYTES, "algorithmic_bytes": sort_bytes,
-                 "ms": sort_ms, "hbm_frac": sort_bytes / (sort_ms * 1e-3) / 1e12 / (HBM_PEAK_GBS / 1e3)
-                 if sort_ms > 0 else 0.0},
+        "roofline": roofline,
+        "sort": sort,
         "stages": stages,
         "stages_ms": {k: sc[k] for k in ("ms_enumerate", "ms_sort", "ms_sort_gen", "ms_sort_local", "ms_sort_count",
                                          "ms_filter", "ms_union")},
@@ -542,8 +563,7 @@ def batch_section(args, mp, torch, dev):
     del da
     torch.cuda.empty_cache()
 
-    # the batch's pass chain captured in a HIP graph by the warm-up step, replayed by the timed ones
-    bctx = mp.Context(k=args.k, sort_graph=not args.no_graph)
+    bctx = mp.Context(k=args.k, sort_graph=args.graph)
 
     def batch_step():
         bctx.batch_load_device(base, total, ofs)

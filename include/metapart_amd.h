@@ -80,6 +80,12 @@ typedef struct {
                              and replayed while the sort's shape and buffers repeat; 0: launched one by one */
 } mp_cfg;
 
+/* A scan with k = 20..31 and every field of mp_cfg that names a form of the
+ * radix sort at 0 groups its k-mers by minimizer bins instead of sorting them:
+ * ms_enumerate is then the making of the bins' records, ms_sort the grouping
+ * and the runs with the filter (ms_sort_local: that kernel), ms_filter the
+ * refilter, sort_long_groups the bins past one table, and the fields of the
+ * radix passes are 0 (ms_sort_gen = 0 tells the two apart). */
 typedef struct {
     uint64_t tuples;          /* tuples enumerated in the scan */
     uint64_t bad_labels;      /* labels marked BAD by the filter in this scan */

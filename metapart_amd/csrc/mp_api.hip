@@ -87,6 +87,8 @@ int mp_ctx_destroy(mp_ctx *ctx)
 const char *mp_last_error(const mp_ctx *ctx) { return ctx ? ctx->err.c_str() : "null context"; }
 uint64_t mp_ctx_device_bytes(const mp_ctx *ctx) { return ctx ? ctx->held : 0; }
 
+static int batch_sort(mp_ctx *ctx, uint64_t *n_out, std::vector<uint64_t> &tpos, int *passes, float *gen_ms);
+
 static int load_common(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *chunk_first_id, int C)
 {
     if (C <= 0 || !chunk_ofs) return ctx->fail(MP_EINVAL, "need at least one chunk");
@@ -95,6 +97,7 @@ static int load_common(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *c
     for (int c = 0; c < C; c++)
         if (chunk_ofs[c + 1] < chunk_ofs[c]) return ctx->fail(MP_EINVAL, "chunk offsets must not decrease");
     ctx->have_scan = false;
+    ctx->dump_lazy = false;
     ctx->finished = false;
     ctx->scans_done = 0;
     ctx->last_n = 0;
@@ -379,8 +382,34 @@ int mp_scan(mp_ctx *ctx, int s, uint64_t lo, uint64_t hi, const uint64_t *seg_bo
             return 0;
         }
     }
+    ctx->dump_lazy = false;
     hipEventRecord(ctx->ev[0], ctx->stream);
     uint64_t n = 0;
+    if (bins_apply(ctx, T)) {
+        BinJob job;
+        job.s = s;
+        job.lo = lo;
+        job.hi = hi;
+        job.bounds = seg_bounds;
+        job.T = T;
+        job.expected = expected_tuples;
+        bool done = false;
+        MP_TRY(bins_scan(ctx, job, &st, nullptr, &n, &done));
+        if (done) {
+            st.tuples = n;
+            if (stats) *stats = st;
+            ctx->last_n = n;
+            ctx->have_scan = true;
+            ctx->dump_lazy = true;
+            ctx->dump_scan = s;
+            ctx->dump_lo = lo;
+            ctx->dump_hi = hi;
+            ctx->dump_bounds.assign(seg_bounds, seg_bounds + T + 1);
+            ctx->scans_done++;
+            return 0;
+        }
+        memset(&st, 0, sizeof(st));
+    }
     // every k-mer: the first radix pass generates the tuples from the reads;
     // 3-minimizer k-mers (a per-read window state machine) are enumerated
     std::unique_ptr<GenSource> gen;
@@ -453,6 +482,33 @@ int mp_get_bad(mp_ctx *ctx, uint8_t *bad)
     return 0;
 }
 
+// The sorted tuples and zeroed runs of a scan that went by minimizer bins,
+// made when a dump asks for them: the scan's labels are the read ids (the
+// first scan) or the snapshot taken at its start.
+static int sort_for_dump(mp_ctx *ctx)
+{
+    uint64_t n = 0;
+    int passes = 0;
+    if (ctx->batch) {
+        std::vector<uint64_t> tpos;
+        float gen_ms = 0;
+        MP_TRY(batch_sort(ctx, &n, tpos, &passes, &gen_ms));
+        if (tpos != ctx->sample_tuples) return ctx->fail(MP_ECOUNT, "the sorted samples differ from the scan's");
+        MP_TRY(filter_zbits_groups(ctx, n, tpos.data(), ctx->C));
+    } else {
+        GenSource gen;
+        ctx->use_labsnap = ctx->dump_scan > 0;
+        int rc = gen_histograms(ctx, ctx->dump_scan, ctx->dump_lo, ctx->dump_hi, scan_pass_mask(ctx->cfg.k), false, &gen, &n);
+        if (!rc) rc = radix_sort_tuples(ctx, n, &passes, &gen);
+        ctx->use_labsnap = false;
+        MP_TRY(rc);
+        if (n != ctx->last_n) return ctx->fail(MP_ECOUNT, "the sorted tuples differ from the scan's");
+        MP_TRY(filter_zbits_scan(ctx, n, ctx->dump_bounds.data(), (int)ctx->dump_bounds.size() - 1));
+    }
+    ctx->dump_lazy = false;
+    return 0;
+}
+
 int mp_dump_tuples(mp_ctx *ctx, uint8_t *dst, uint64_t cap, uint64_t *n)
 {
     if (!ctx || !n) return MP_EINVAL;
@@ -462,6 +518,7 @@ int mp_dump_tuples(mp_ctx *ctx, uint8_t *dst, uint64_t cap, uint64_t *n)
     if (cap < ctx->last_n) return ctx->fail(MP_EINVAL, "dump buffer holds %llu tuples, need %llu",
                                             (unsigned long long)cap, (unsigned long long)ctx->last_n);
     MP_HIP(hipSetDevice(ctx->device));
+    if (ctx->dump_lazy) MP_TRY(sort_for_dump(ctx));
     const uint64_t m = ctx->last_n;
     std::vector<uint64_t> k(m);
     std::vector<uint32_t> l(m), z((m + 31) / 32 + 1);
@@ -547,22 +604,13 @@ int mp_batch_load_device(mp_ctx *ctx, const void *d_fq, uint64_t nbytes, int n, 
     return batch_after_load(ctx);
 }
 
-int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_stats, mp_finish_stats *finish_stats)
+// The batch's tuples sorted sample by sample: tpos takes the samples' tuple offsets.
+static int batch_sort(mp_ctx *ctx, uint64_t *n_out, std::vector<uint64_t> &tpos, int *passes, float *gen_ms)
 {
-    if (!ctx) return MP_EINVAL;
-    if (!ctx->batch) return ctx->fail(MP_ESTATE, "mp_batch_partition before mp_batch_load");
-    MP_HIP(hipSetDevice(ctx->device));
-    const uint64_t N = ctx->N;
     const int ns = ctx->C;
-    mp_scan_stats st;
-    memset(&st, 0, sizeof(st));
-    MP_TRY(iota_u32(ctx, (uint32_t *)ctx->parent.p, N));
-    MP_TRY(fill_u32(ctx, ctx->bad.p, 0, (N + 3) / 4));
-    MP_TRY(fill_u32(ctx, ctx->filtered.p, 0, (N + 3) / 4));
-    ctx->scans_done = 0;
-    hipEventRecord(ctx->ev[0], ctx->stream);
     uint64_t n = 0;
     std::unique_ptr<GenSource> gen;
+    tpos.assign(ns + 1, 0);
     // every sample sorted on its own (segmented passes, each sample's tuples
     // from its own position) unless the passes take look-back offsets
     const char *lbe = getenv("MP_SORT_LOOKBACK");
@@ -575,9 +623,6 @@ int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_s
         MP_TRY(gen_histograms(ctx, 0, 0, MP_NBUCKETS, scan_pass_mask(ctx->cfg.k), true, gen.get(), &n));
     }
     hipEventRecord(ctx->ev[1], ctx->stream);
-    std::vector<uint64_t> tpos(ns + 1, 0);
-    int passes = 0;
-    float gen_ms = 0.f;
     if (segmented && gen->gcnt && gen->gcnt_seg && gen->seg_tuples.size() == (size_t)ns) {
         for (int i = 0; i < ns; i++) {  // a plain run's range plan is degenerate without k-mers (mp_plan_ranges)
             if (gen->seg_tuples[i] == 0) return ctx->fail(MP_EPLAN, "sample %d has no k-mers to partition", i);
@@ -587,21 +632,21 @@ int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_s
         sg.ns = ns;
         sg.tpos = tpos.data();
         sg.wpos = ctx->seg_wpos.data();
-        MP_TRY(radix_sort_tuples(ctx, n, &passes, gen.get(), &sg));
-        gen_ms = ctx->sort_gen_ms;
+        MP_TRY(radix_sort_tuples(ctx, n, passes, gen.get(), &sg));
+        *gen_ms = ctx->sort_gen_ms;
     } else {
         // sort by (sample, k-mer, adj): the sample of a label is its chunk
         uint64_t *d_first = nullptr;
         MP_HIP(hipMallocAsync((void **)&d_first, sizeof(uint64_t) * (ns + 1), ctx->stream));
         MP_HIP(hipMemcpyAsync(d_first, ctx->chunk_ids.data(), sizeof(uint64_t) * (ns + 1), hipMemcpyHostToDevice,
                               ctx->stream));
-        int rc = radix_sort_tuples(ctx, n, &passes, gen.get());
-        gen_ms = gen ? ctx->sort_gen_ms : 0.f;
+        int rc = radix_sort_tuples(ctx, n, passes, gen.get());
+        *gen_ms = gen ? ctx->sort_gen_ms : 0.f;
         if (!rc) {  // then the sample of the label as the most significant digit
             int sp = 0;
             rc = radix_sort_generic(ctx, ctx->keys, ctx->lab, ctx->adj, &ctx->cur, n, 1u << 9, &sp, d_first, ns,
                                     tpos.data());
-            passes += sp;
+            *passes += sp;
         }
         MP_HIP(hipFreeAsync(d_first, ctx->stream));
         MP_TRY(rc);
@@ -617,26 +662,66 @@ int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_s
     }
     for (int i = 0; i < ns; i++)  // a plain run's range plan is degenerate without k-mers (mp_plan_ranges)
         if (tpos[i + 1] == tpos[i]) return ctx->fail(MP_EPLAN, "sample %d has no k-mers to partition", i);
-    hipEventRecord(ctx->ev[7], ctx->stream);
-    // one filter/union segment per sample, each its own quirk group
-    std::vector<uint64_t> grp(2 * (size_t)ns);
-    for (int i = 0; i < ns; i++) {
-        grp[2 * i] = tpos[i];
-        grp[2 * i + 1] = tpos[i + 1];
+    *n_out = n;
+    return 0;
+}
+
+int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_stats, mp_finish_stats *finish_stats)
+{
+    if (!ctx) return MP_EINVAL;
+    if (!ctx->batch) return ctx->fail(MP_ESTATE, "mp_batch_partition before mp_batch_load");
+    MP_HIP(hipSetDevice(ctx->device));
+    const uint64_t N = ctx->N;
+    const int ns = ctx->C;
+    mp_scan_stats st;
+    memset(&st, 0, sizeof(st));
+    MP_TRY(iota_u32(ctx, (uint32_t *)ctx->parent.p, N));
+    MP_TRY(fill_u32(ctx, ctx->bad.p, 0, (N + 3) / 4));
+    MP_TRY(fill_u32(ctx, ctx->filtered.p, 0, (N + 3) / 4));
+    ctx->scans_done = 0;
+    hipEventRecord(ctx->ev[0], ctx->stream);
+    uint64_t n = 0;
+    std::vector<uint64_t> tpos(ns + 1, 0);
+    int passes = 0;
+    float gen_ms = 0.f;
+    bool done = false;  // by minimizer bins: nothing left to sort, filter or join
+    ctx->dump_lazy = false;
+    if (bins_apply(ctx, ns)) {
+        BinJob job;
+        job.lo = 0;
+        job.hi = MP_NBUCKETS;
+        job.T = ns;
+        job.first = ctx->chunk_ids.data();
+        MP_TRY(bins_scan(ctx, job, &st, &tpos, &n, &done));
     }
-    MP_TRY(filter_union_groups(ctx, n, tpos.data(), ns, grp.data(), &st));
+    if (!done) {
+        memset(&st, 0, sizeof(st));
+        MP_TRY(batch_sort(ctx, &n, tpos, &passes, &gen_ms));
+    }
+    if (!done) {
+        hipEventRecord(ctx->ev[7], ctx->stream);
+        // one filter/union segment per sample, each its own quirk group
+        std::vector<uint64_t> grp(2 * (size_t)ns);
+        for (int i = 0; i < ns; i++) {
+            grp[2 * i] = tpos[i];
+            grp[2 * i + 1] = tpos[i + 1];
+        }
+        MP_TRY(filter_union_groups(ctx, n, tpos.data(), ns, grp.data(), &st));
+        st.sort_passes = passes;
+        st.ms_sort_pass_avg = ctx->sort_pass_avg;
+        st.ms_sort_hist = ctx->sort_hist_ms;
+        st.ms_sort_local = ctx->local_ms;
+        st.sort_long_groups = ctx->local_long;
+        st.sort_local_moved = ctx->local_moved;
+        st.ms_sort_gen = gen_ms;
+        st.ms_sort_count = ctx->sort_count_ms;
+        st.sort_graph = ctx->sort_graph_last;
+        hipEventElapsedTime(&st.ms_enumerate, ctx->ev[0], ctx->ev[1]);
+        hipEventElapsedTime(&st.ms_sort, ctx->ev[1], ctx->ev[7]);
+    }
     st.tuples = n;
-    st.sort_passes = passes;
-    st.ms_sort_pass_avg = ctx->sort_pass_avg;
-    st.ms_sort_hist = ctx->sort_hist_ms;
-    st.ms_sort_local = ctx->local_ms;
-    st.sort_long_groups = ctx->local_long;
-    st.sort_local_moved = ctx->local_moved;
-    st.ms_sort_gen = gen_ms;
-    st.ms_sort_count = ctx->sort_count_ms;
-    st.sort_graph = ctx->sort_graph_last;
-    hipEventElapsedTime(&st.ms_enumerate, ctx->ev[0], ctx->ev[1]);
-    hipEventElapsedTime(&st.ms_sort, ctx->ev[1], ctx->ev[7]);
+    ctx->dump_lazy = done;
+    ctx->dump_scan = 0;
     ctx->last_n = n;
     ctx->have_scan = true;
     ctx->scans_done = 1;

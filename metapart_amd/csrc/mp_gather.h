@@ -82,17 +82,20 @@ __device__ __forceinline__ uint32_t prefix_mask(uint32_t e, int k)
 struct PackSink {
     uint32_t *packed;  // the 2-bit stream as 32-bit halves
     uint16_t *nmask;   // the 'N' stream as 16-bit quarters
+    uint32_t *odd;     // set when a letter other than 'N' has bit 3 set (its neighbour class is not in the 2-bit code)
     __device__ void operator()(uint64_t x, const uint32_t b[4], uint32_t valid) const
     {
-        uint32_t code = 0, nb = 0;
+        uint32_t code = 0, nb = 0, b3 = 0;
 #pragma unroll
         for (int e = 0; e < 16; e++) {
             const uint32_t c = (b[e >> 2] >> (8 * (e & 3))) & 0xFF;
             if (e < (int)valid) {
                 code |= ((0x2310u >> (((c & 6) >> 1) * 4)) & 3) << (30 - 2 * e);
                 if (c == 'N') nb |= 1u << (15 - e);
+                b3 |= ((c >> 3) & 1) << (15 - e);
             }
         }
+        if (b3 != nb) atomicOr(odd, 1u);
         const uint64_t u = x >> 4;
         packed[2 * (u >> 1) + 1 - (u & 1)] = code;  // bases 0-15 of a word are its high half
         nmask[4 * (u >> 2) + 3 - (u & 3)] = (uint16_t)nb;

@@ -523,6 +523,8 @@ __device__ __forceinline__ bool is_bad(const uint64_t *bits, uint32_t x) { retur
 // labels, so the work is the label and BAD-bit reads, not the finds.
 constexpr int kUW = 4;  // bitmap words a wave takes per step, their loads in flight together
 
+// ALL: every run is joined (rs_bits unused; a scan by minimizer bins lists only those)
+template <bool ALL>
 __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *__restrict__ rs_bits,
                                                     const uint64_t *__restrict__ st_bits,
                                                     const uint64_t *__restrict__ badbits)
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *_
 #pragma unroll
         for (int u = 0; u < kUW; u++) {
             st[u] = w0 + u < nw ? st_bits[w0 + u] : 0;
-            rs[u] = w0 + u < nw ? rs_bits[w0 + u] : 0;
+            rs[u] = ALL ? ~0ull : w0 + u < nw ? rs_bits[w0 + u] : 0;
             lb[u] = G.lab[min((w0 + u) * 64 + lane, G.n - 1)];
         }
         // the run holding tuple w0 * 64 when it began before: its start and whether it is joined
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *_
             if (m) {
                 const int bit = 63 - __builtin_clzll(m);
                 cs = q * 64 + bit;
-                cjoin = (rs_bits[q] >> bit) & 1;
+                cjoin = ALL || ((rs_bits[q] >> bit) & 1);
             }
         }
         uint32_t b[kUW];
@@ -1069,7 +1071,7 @@ static int filter_union_core(mp_ctx *ctx, uint64_t n, const uint64_t *d_seg, int
         hipLaunchKernelGGL(bad_bits_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint8_t *)G.bad, N,
                            badbits);
         MP_HIP(hipGetLastError());
-        hipLaunchKernelGGL(union_kernel, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0, ctx->stream,
+        hipLaunchKernelGGL(union_kernel<false>, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0, ctx->stream,
                            G, (const uint64_t *)rs_bits, (const uint64_t *)st_bits, (const uint64_t *)badbits);
         MP_HIP(hipGetLastError());
     }
@@ -1277,7 +1279,7 @@ int two_sweep_scan(mp_ctx *ctx, const std::vector<uint64_t> &cuts, const uint64_
                            badbits);
         const uint64_t rwords = (n + 63) / 64 + 1;
         const uint64_t *rs_bits = (const uint64_t *)ctx->runbits.p;
-        hipLaunchKernelGGL(union_kernel, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0,
+        hipLaunchKernelGGL(union_kernel<false>, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0,
                            ctx->stream, G, rs_bits, rs_bits + rwords, (const uint64_t *)badbits);
         MP_HIP(hipGetLastError());
         hipEventRecord(ctx->ev[5], ctx->stream);
@@ -1301,6 +1303,90 @@ int two_sweep_scan(mp_ctx *ctx, const std::vector<uint64_t> &cuts, const uint64_
         st->parts = P;
     }
     return 0;
+}
+
+int refilter_reads(mp_ctx *ctx, unsigned long long *d_nbad)
+{
+    hipLaunchKernelGGL(refilter_kernel, dim3(stride_grid(ctx->N)), dim3(256), 0, ctx->stream, (uint8_t *)ctx->bad.p,
+                       (const uint8_t *)ctx->filtered.p, (uint32_t *)ctx->parent.p, ctx->N, d_nbad);
+    MP_HIP(hipGetLastError());
+    return 0;
+}
+
+int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, uint64_t n)
+{
+    const uint64_t N = ctx->N;
+    if (n) {
+        MP_TRY(ensure(ctx, ctx->scratch, ((N + 63) / 64 + 1) * sizeof(uint64_t)));
+        uint64_t *badbits = (uint64_t *)ctx->scratch.p;
+        hipLaunchKernelGGL(bad_bits_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint8_t *)ctx->bad.p, N,
+                           badbits);
+        GParams G{};
+        G.lab = lab;
+        G.n = n;
+        G.parent = (uint32_t *)ctx->parent.p;
+        hipLaunchKernelGGL(union_kernel<true>, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0,
+                           ctx->stream, G, (const uint64_t *)nullptr, st_bits, (const uint64_t *)badbits);
+        MP_HIP(hipGetLastError());
+    }
+    return compress_labels(ctx, (uint32_t *)ctx->parent.p, (const uint8_t *)ctx->bad.p, N);
+}
+
+// The zeroed runs alone, for a dump of tuples sorted after their scan: the
+// marks the kernel makes on the way repeat the scan's.
+int filter_zbits(mp_ctx *ctx, uint64_t n, const uint64_t *d_seg, int nseg)
+{
+    const uint64_t nwords = (n + 31) / 32 + 1, rwords = (n + 63) / 64 + 1;
+    MP_TRY(ensure(ctx, ctx->zbits, nwords * sizeof(uint32_t)));
+    MP_TRY(ensure(ctx, ctx->runbits, 2 * rwords * sizeof(uint64_t)));
+    MP_TRY(ensure(ctx, ctx->scratch, 4096));
+    MP_TRY(fill_u32(ctx, ctx->zbits.p, 0, nwords));
+    GParams G{};
+    G.keys = (const uint64_t *)ctx->keys[ctx->cur].p;
+    G.lab = (const uint32_t *)ctx->lab[ctx->cur].p;
+    G.adj = (const uint8_t *)ctx->adj[ctx->cur].p;
+    G.n = n;
+    G.seg = d_seg;
+    G.T = nseg;
+    G.bad = (uint8_t *)ctx->bad.p;
+    G.filtered = (uint8_t *)ctx->filtered.p;
+    G.zbits = (uint32_t *)ctx->zbits.p;
+    G.stats = (unsigned long long *)ctx->scratch.p;
+    if (!grid_fits((n + kFTile - 1) / kFTile, kFLanes))
+        return ctx->fail(MP_EINVAL, "filter over %llu tuples exceeds one dispatch: use more scans", (unsigned long long)n);
+    if (n) {
+        uint64_t *rs_bits = (uint64_t *)ctx->runbits.p;
+        hipLaunchKernelGGL(filter_tile_kernel, dim3((unsigned)((n + kFTile - 1) / kFTile)), dim3(kFLanes), 0,
+                           ctx->stream, G, rs_bits, rs_bits + rwords);
+        MP_HIP(hipGetLastError());
+    }
+    MP_HIP(hipStreamSynchronize(ctx->stream));
+    return 0;
+}
+
+int filter_zbits_scan(mp_ctx *ctx, uint64_t n, const uint64_t *seg_bounds, int T)
+{
+    uint64_t *d_small = nullptr;
+    MP_HIP(hipMallocAsync((void **)&d_small, 2 * (size_t)(T + 1) * sizeof(uint64_t), ctx->stream));
+    uint64_t *d_bounds = d_small, *d_seg = d_small + (T + 1);
+    MP_HIP(hipMemcpyAsync(d_bounds, seg_bounds, sizeof(uint64_t) * (T + 1), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(seg_pos_kernel, dim3(nblk(T + 1)), dim3(256), 0, ctx->stream,
+                       (const uint64_t *)ctx->keys[ctx->cur].p, n, 2 * (ctx->cfg.k - 10), (const uint64_t *)d_bounds, T,
+                       d_seg);
+    MP_HIP(hipGetLastError());
+    const int rc = filter_zbits(ctx, n, d_seg, T);
+    MP_HIP(hipFreeAsync(d_small, ctx->stream));
+    return rc;
+}
+
+int filter_zbits_groups(mp_ctx *ctx, uint64_t n, const uint64_t *seg_pos, int nseg)
+{
+    uint64_t *d_seg = nullptr;
+    MP_HIP(hipMallocAsync((void **)&d_seg, (size_t)(nseg + 1) * sizeof(uint64_t), ctx->stream));
+    MP_HIP(hipMemcpyAsync(d_seg, seg_pos, sizeof(uint64_t) * (nseg + 1), hipMemcpyHostToDevice, ctx->stream));
+    const int rc = filter_zbits(ctx, n, d_seg, nseg);
+    MP_HIP(hipFreeAsync(d_seg, ctx->stream));
+    return rc;
 }
 
 int filter_union_groups(mp_ctx *ctx, uint64_t n, const uint64_t *seg_pos, int nseg, const uint64_t *grp,

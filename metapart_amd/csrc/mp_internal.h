@@ -124,6 +124,9 @@ struct mp_ctx {
 
     // per-read arrays
     mp::DevArray fq, rec_off, seq_off, seq_len, base_off, pos_off, packed, nmask;
+    mp::DevArray rstart;        // read starts, one bit per base (laid out as nmask), for scans by minimizer bins
+    bool rstart_valid = false;
+    bool plain_letters = false; // no empty read, and no letter but 'N' with bit 3 set: the 2-bit code gives a base's neighbour class
     // graph state
     mp::DevArray parent, bad, filtered, sizes;
     mp::DevArray gparent, gsize;  // pair step: components of the candidate-pair graph
@@ -134,6 +137,12 @@ struct mp_ctx {
     mp::DevArray dig, rts; // counted radix passes: next pass's digit per tuple; per-tile counts and offsets
     mp::DevArray gcnt;     // m-mer histogram: digit counts per generating-pass tile (a scan over every k-mer)
     mp::DevArray segtab;   // a batch's per-sample generating-pass tiles: first tile, first window
+    mp::DevArray binctl;   // scan by minimizer bins: its counters
+    // the last scan went by minimizer bins: its sorted tuples are made when a dump asks for them
+    bool dump_lazy = false;
+    int dump_scan = 0;
+    uint64_t dump_lo = 0, dump_hi = 0;
+    std::vector<uint64_t> dump_bounds;
     mp::DevArray sortaux;  // radix sort: digit bases, segment tables, generating-pass tile table
     // captured radix pass chains (mp_cfg.sort_graph), the latest last, with the
     // shape and buffers each was captured for (a batch sorts its tuples, the
@@ -185,7 +194,7 @@ struct mp_ctx {
     // every device buffer the ctx holds
     template <typename F> void for_each_array(F f)
     {
-        mp::DevArray *arrs[] = {&fq, &rec_off, &seq_off, &seq_len, &base_off, &pos_off, &packed, &nmask, &parent, &bad,
+        mp::DevArray *arrs[] = {&fq, &rec_off, &seq_off, &seq_len, &base_off, &pos_off, &packed, &nmask, &rstart, &binctl, &parent, &bad,
                                 &filtered, &sizes, &gparent, &gsize, &pairc, &scanst, &hpart, &khist, &labsnap,
                                 &runbits, &dig, &rts, &gcnt, &segtab, &sortaux, &keys[0], &keys[1], &lab[0], &lab[1], &adj[0], &adj[1], &zbits, &wg_cnt,
                                 &wg_off, &status, &scratch, &hist, &out, &items[0], &items[1], &ilens[0], &ilens[1],
@@ -309,6 +318,29 @@ int bucket_prefix_range(mp_ctx *ctx, uint64_t lo, uint64_t hi, std::vector<uint6
 // Labels of scan s for every read as they stand now; the scan's k-mer
 // kernels use them until use_labsnap is cleared.
 int snapshot_labels(mp_ctx *ctx, int s);
+// A scan by minimizer bins (mp_bins.hip): filter and union of the tuples in
+// buckets [lo, hi) without sorting them.  Plain: T segments at bounds[0..T].
+// A batch: T samples (first: T + 1 first read ids, host), each one segment;
+// *tpos takes their tuple offsets.  *done = false: nothing was joined and the
+// caller takes the radix path.
+struct BinJob {
+    int s = 0;
+    uint64_t lo = 0, hi = 0;
+    const uint64_t *bounds = nullptr;
+    int T = 0;
+    const uint64_t *first = nullptr;
+    uint64_t expected = 0;
+};
+bool bins_apply(const mp_ctx *ctx, int T);
+int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uint64_t> *tpos, uint64_t *n_out, bool *done);
+// filtered reads to BAD ones; *d_nbad (device, zero before) takes their number
+int refilter_reads(mp_ctx *ctx, unsigned long long *d_nbad);
+// joins every run of the n labels (run starts in st_bits), then compresses
+int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, uint64_t n);
+// the zeroed runs of the sorted tuples in the current buffers (zbits), segments at device positions d_seg[0..nseg]
+int filter_zbits(mp_ctx *ctx, uint64_t n, const uint64_t *d_seg, int nseg);
+int filter_zbits_scan(mp_ctx *ctx, uint64_t n, const uint64_t *seg_bounds, int T);
+int filter_zbits_groups(mp_ctx *ctx, uint64_t n, const uint64_t *seg_pos, int nseg);
 int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st);
 int write_partitions(mp_ctx *ctx, const char *out_prefix, int T, const uint64_t *W, const int64_t *il_start,
                      uint64_t *bytes_out);

@@ -151,7 +151,7 @@ __global__ void rec_finalize_kernel(const uint8_t *__restrict__ fq, uint64_t n_r
                                     const uint64_t *__restrict__ seq_off, const uint64_t *__restrict__ seq_end,
                                     const uint64_t *__restrict__ plus_end, const uint64_t *__restrict__ rec_off,
                                     uint32_t *__restrict__ seq_len, uint32_t *__restrict__ npos,
-                                    unsigned long long *__restrict__ first_bad)
+                                    unsigned long long *__restrict__ first_bad, uint32_t *__restrict__ odd)
 {
     const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n_rec) return;
@@ -162,6 +162,7 @@ __global__ void rec_finalize_kernel(const uint8_t *__restrict__ fq, uint64_t n_r
     bool ok = (r != 0 || fq[rs] == '@') && qual == L && L < 65536;
     if (ok && L > (uint64_t)K && L - K >= 300) ok = false;  // enumerateKmers.c:155
     if (!ok) atomicMin(first_bad, (unsigned long long)r);
+    if (L == 0) atomicOr(odd, 1u);
     seq_len[r] = (uint32_t)L;
     npos[r] = L > (uint64_t)K ? (uint32_t)(L - K + 1) : 0u;
 }
@@ -236,13 +237,17 @@ int parse_reads(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *chunk_fi
     MP_TRY(ensure(ctx, ctx->hist, 4096));
     unsigned long long *first_bad = (unsigned long long *)ctx->hist.p;
     MP_TRY(fill_u32(ctx, first_bad, 0xFFFFFFFFu, 2));
+    uint32_t *d_odd = (uint32_t *)(first_bad + 1);  // an empty read, or a letter that PackSink marks
+    MP_TRY(fill_u32(ctx, d_odd, 0, 1));
+    ctx->plain_letters = false;
+    ctx->rstart_valid = false;
     hipLaunchKernelGGL(nl_write_kernel, dim3((unsigned)nblk), dim3(kParseBlock), 0, ctx->stream, fq, nbytes,
                        (const uint64_t *)ctx->wg_off.p, N, (uint64_t *)ctx->seq_off.p, seq_end, plus_end, rec_off,
                        first_bad);
     MP_HIP(hipGetLastError());
     hipLaunchKernelGGL(rec_finalize_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, ctx->stream, fq, N, K,
                        (const uint64_t *)ctx->seq_off.p, seq_end, plus_end, (const uint64_t *)rec_off,
-                       (uint32_t *)ctx->seq_len.p, npos, first_bad);
+                       (uint32_t *)ctx->seq_len.p, npos, first_bad, d_odd);
     MP_HIP(hipGetLastError());
     unsigned long long bad = 0;
     MP_HIP(hipMemcpyAsync(&bad, first_bad, sizeof(bad), hipMemcpyDeviceToHost, ctx->stream));
@@ -296,10 +301,13 @@ int parse_reads(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *chunk_fi
     MP_TRY(tmp_alloc(ctx, (void **)&first, (nb + 1) * sizeof(uint64_t)));
     const int rc = launch_gather(ctx, fq, ctx->fq_bytes, (const uint64_t *)ctx->base_off.p, N, tb, nthreads * 64, first,
                                  SeqSrc{(const uint64_t *)ctx->seq_off.p},
-                                 PackSink{(uint32_t *)ctx->packed.p, (uint16_t *)ctx->nmask.p});
+                                 PackSink{(uint32_t *)ctx->packed.p, (uint16_t *)ctx->nmask.p, d_odd});
     MP_TRY(tmp_free(ctx, first));
     MP_TRY(rc);
+    uint32_t odd = 0;
+    MP_HIP(hipMemcpyAsync(&odd, d_odd, sizeof(odd), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->plain_letters = odd == 0;
     return 0;
 }
 

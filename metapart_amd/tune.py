@@ -65,7 +65,8 @@ def tune_sort_tile(k: int = 31, reads: int = 2_000_000, seed: int = 2, device: i
     buf = synth(2, n_reads=reads, seed=seed)
     times = {}
     for shape in TILE_SHAPES:
-        with Context(k=k, device=device, sort_tile=shape) as ctx:
+        # a digit width is named so that every shape, 0 too, times the radix passes
+        with Context(k=k, device=device, sort_tile=shape, sort_digit_bits=7) as ctx:
             best = None
             for _ in range(2):  # the first run allocates
                 ctx.load(buf, [0, buf.nbytes])

@@ -1,0 +1,146 @@
+"""Scans by minimizer bins (the default for k = 20..31) against the radix path
+on the same reads: labels, plan, per-scan counts, at the sizes where the bins
+can go wrong -- every k they take, reads at and just past k, 'N's at record
+ends, runs past a bin, one k-mer alone (the first-run quirk), many dead reads
+and a few live ones, letters the bins leave to the radix path -- and batches."""
+import numpy as np
+import pytest
+
+import metapart_amd as mp
+
+FIELDS = ("tuples", "bad_labels", "zeroed_runs", "evaluated_runs", "quirk_segments")
+
+
+def _fastq(seqs):
+    return np.frombuffer("".join("@r%d\n%s\n+\n%s\n" % (i, s, "I" * len(s)) for i, s in enumerate(seqs)).encode(),
+                         dtype=np.uint8).copy()
+
+
+def _run(buf, C, K, S, T, **kw):
+    with mp.Context(k=K, **kw) as ctx:
+        ctx.load(buf, mp.index_buffer(buf, C))
+        r = mp.partition(ctx, S=S, T=T, want_parent=True, build_output=False)
+        return r, [[s[f] for f in FIELDS] for s in r.scans], [s["ms_sort_gen"] == 0 for s in r.scans]  # a radix scan times its generating pass
+
+
+def _same(buf, C, K, S, T, bins=True):
+    a, sa, pa = _run(buf, C, K, S, T)
+    b, sb, pb = _run(buf, C, K, S, T, sort_digit_bits=7)  # a digit width asks for the radix sort
+    assert not any(pb)
+    if bins is not None:
+        assert all(p == bins for p in pa), pa
+    assert sa == sb
+    assert np.array_equal(a.parent, b.parent)
+    assert np.array_equal(a.W, b.W)
+    return a
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", list(range(20, 32)))
+def test_every_k_equals_radix(K):
+    print("gpu bins k", K, flush=True)
+    buf = mp.synth(0, n_reads=6000, seed=300 + K, read_len_min=K - 3, read_len_max=K + 90, n_rate=0.004)
+    _same(buf, 4, K, 1, 1 + K % 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(2, 1), (3, 2), (1, 16)])
+def test_scans_and_segments_equal_radix(S, T):
+    print("gpu bins scans, segments", S, T, flush=True)
+    _same(mp.synth(0, n_reads=20000, seed=77, read_len=120), 16, 27, S, T)
+
+
+@pytest.mark.gpu
+def test_records_at_read_and_step_ends():
+    # reads of k - 1 .. k + 2 bases and of every length around a step's 960
+    # positions, 'N' first, last, beside and between windows
+    print("gpu bins record ends", flush=True)
+    rng = np.random.default_rng(5)
+    K = 31
+    base = "".join("ACGT"[i] for i in rng.integers(0, 4, 4000))
+    seqs = []
+    for i in range(3000):
+        L = [K - 1, K, K + 1, K + 2, 60, 64, 96, 240, 300, 20][i % 10]
+        o = int(rng.integers(0, 4000 - 330))
+        s = list(base[o:o + L])
+        for p in {0: [], 1: [0], 2: [L - 1], 3: [L // 2], 4: [0, L - 1]}[i // 10 % 5]:
+            s[p] = "N"
+        if i % 7 == 0:
+            s = [c.lower() if c != "N" else c for c in s]
+        seqs.append("".join(s))
+    _same(_fastq(seqs), 1, K, 1, 1)
+
+
+@pytest.mark.gpu
+def test_homopolymers_and_one_kmer():
+    # one k-mer (the only run is the last, so the first-run quirk shows: the
+    # radix path answers), the k-mer 0 alone beside others, and both ends
+    print("gpu bins homopolymers", flush=True)
+    a = _same(_fastq(["C" * 100] * 20), 1, 31, 1, 1, bins=False)
+    assert a.scans[0]["quirk_segments"] == 1
+    _same(_fastq(["A" * 90, "T" * 200] * 40 + ["ACGTTGCATCAGGATCAGCATTACGAGCATCGGACT"] * 4), 1, 25, 1, 1, bins=None)
+    _same(_fastq(["AC" * 60, "CA" * 45, "AAC" * 40, "ACGT" * 30] * 200), 1, 31, 1, 1, bins=None)
+
+
+@pytest.mark.gpu
+def test_bins_past_the_table_and_a_few_live_reads():
+    # a 500 bp genome at ~12000x (bins of far more windows and, by its errors,
+    # k-mers than a table holds), then two reads of k + 1 bases that nothing filters
+    print("gpu bins deep", flush=True)
+    deep = mp.synth(0, n_reads=40000, n_genomes=1, genome_len_min=500, genome_len_max=500, read_len=150,
+                    err_rate=0.01, seed=21)
+    a = _same(deep, 4, 31, 1, 1)
+    assert a.scans[0]["sort_long_groups"] > 0
+    live = _fastq(["ACGGATTACCAGATTGCAGGCTTAACGGATCG", "TTGACCGATAGGACCAGTTTACCAGAGGATCC"])
+    _same(np.concatenate([np.frombuffer(deep.tobytes(), dtype=np.uint8), live]), 1, 31, 1, 1, bins=None)
+
+
+@pytest.mark.gpu
+def test_other_letters_take_the_radix_path():
+    print("gpu bins letters", flush=True)
+    buf = np.frombuffer(mp.synth(0, n_reads=2000, seed=9, read_len=100).tobytes(), dtype=np.uint8).copy()
+    nl = np.flatnonzero(buf == 10)
+    buf[nl[40] + 50] = ord("Y")  # bit 3 set: its neighbour class is not in the 2-bit code
+    _same(buf, 2, 27, 1, 1, bins=False)
+    seqs = ["ACGGATTACCAGATTGCAGGCTTAACGGATCGAC"] * 10
+    seqs[3] = ""
+    _same(_fastq(seqs), 1, 27, 1, 1, bins=False)
+
+
+@pytest.mark.gpu
+def test_dump_after_bins_equals_radix():
+    print("gpu bins dump", flush=True)
+    buf = mp.synth(0, n_reads=5000, seed=4, read_len=90, n_rate=0.002)
+    got = []
+    for kw in ({}, {"sort_digit_bits": 7}):
+        with mp.Context(k=25, **kw) as ctx:
+            ctx.load(buf, mp.index_buffer(buf, 4))
+            hist, _, _, _ = ctx.count()
+            scan, thread = mp.plan_ranges(hist, 2, 2)
+            out = []
+            for s in range(2):
+                ctx.scan(s, int(scan[s]), int(scan[s + 1]), thread[2 * s:2 * s + 3])
+                out.append(ctx.dump_tuples())
+            W, _ = ctx.finish()
+            got.append((out, W, ctx.parent(), ctx.dump_tuples()))
+    for x, y in zip(got[0][0] + [got[0][3]], got[1][0] + [got[1][3]]):
+        assert np.array_equal(x, y)
+    assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 70, 256])
+def test_batch_equals_radix(n):
+    print("gpu bins batch", n, flush=True)
+    rng = np.random.default_rng(n)
+    bufs = [mp.synth(0, n_reads=2 * int(rng.integers(1, 400)), seed=500 + i % 50, read_len=int(rng.integers(40, 150)))
+            for i in range(n)]
+    got = []
+    for kw in ({}, {"sort_digit_bits": 7}):
+        with mp.Context(k=31, **kw) as ctx:
+            ctx.batch_load(bufs)
+            res, st, _ = ctx.batch_partition()
+            got.append(([[r[f] for f in ("reads", "tuples", "components", "largest")] + list(map(int, r["W"])) for r in res],
+                        [getattr(st, f) for f in FIELDS], np.concatenate([ctx.batch_parent(i) for i in range(n)])))
+    assert got[0][0] == got[1][0] and got[0][1] == got[1][1]
+    assert np.array_equal(got[0][2], got[1][2])
