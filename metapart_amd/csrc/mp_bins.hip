@@ -49,8 +49,8 @@ constexpr int kStepPos = 960;       // base positions a wave takes per step: 60 
 constexpr int kStepRec = 480;       // records of a step (more: the radix path)
 constexpr int kMaxRun = 31;         // windows per record
 constexpr uint32_t kBinCap = 4096;  // windows of a bin that bin_runs takes; its table's slots
-constexpr uint32_t kBinRec = 1024;  // records of such a bin
-constexpr uint32_t kBinAim = 3072;  // windows per bin aimed at
+constexpr uint32_t kBinRec = 640;   // records of such a bin
+constexpr uint32_t kBinAim = kBinCap * 3 / 4;  // windows per bin aimed at, at most (fewer where records hold few)
 constexpr int kRunThreads = 1024;
 constexpr int kBinWit = 8;          // witnesses per bin (bin_runs)
 constexpr int kMaxSeg = 256;        // segments (samples of a batch)
@@ -67,6 +67,8 @@ constexpr uint32_t kPrevN = 1, kNextN = 2;  // flags: no base before the first /
 struct BinDesc {
     uint32_t rec0, nrec, nwin, smp;
 };
+
+constexpr uint32_t kErrRange = 16;  // BinCtl::err: a k-mer outside the scan's range where every one was to be inside
 
 struct BinCtl {  // device counters of a scan, cleared before it
     unsigned long long nvalid[kMaxSeg];  // windows without 'N' per sample (plain: [0])
@@ -119,14 +121,16 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// inclusive prefix sum over the wave's lanes (all active): four shifts inside
+// the 16-lane rows, then the rows' totals, on the vector unit alone
 __device__ __forceinline__ uint32_t wave_incl(uint32_t v)
 {
-    const unsigned lane = __lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint32_t o = __shfl_up(v, d, kWave);
-        if (lane >= (unsigned)d) v += o;
-    }
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);  // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2 and 3
     return v;
 }
 
@@ -499,14 +503,15 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(KParams G, const uint6
 
 // ---------------------------------------------------------------- bins of a coarse bin
 // One workgroup per coarse bin: records and windows per cell in LDS, cells cut
-// into bins where the running window count passes a multiple of kBinAim, the
+// into bins where the running window count passes a multiple of `aim`, the
 // records moved to their bin (a cursor per bin: a bin's records are written in
 // order, so its lines fill in L2).
 template <int NM>
 __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict__ rec, const uint32_t *__restrict__ coarse,
                                                          const uint32_t *__restrict__ smp_of,
                                                          uint4 *__restrict__ out, BinDesc *__restrict__ bins,
-                                                         BinDesc *__restrict__ big, uint32_t big_cap, BinCtl *ctl)
+                                                         BinDesc *__restrict__ big, uint32_t big_cap, uint32_t aim,
+                                                         BinCtl *ctl)
 {
     constexpr int kPer = NM / 1024;
     __shared__ unsigned long long s_h[NM];  // records << 32 | windows per cell; then the cell's bin
@@ -555,8 +560,10 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
         if (w < wave) run += s_w[w];
         total += s_w[w];
     }
-    // a cell starts a bin where its first window falls into another multiple of kBinAim than its
-    // predecessor's (cell - 1's first window is this cell's less that cell's windows)
+    // a cell starts a bin where its first window falls into another multiple of `aim` than its
+    // predecessor's (cell - 1's first window is this cell's less that cell's windows), and a cell of
+    // more than aim / 3 windows (a deep genome's) is a bin by itself: a bin of several cells holds
+    // at most 4/3 aim windows, however deep its cells
     uint32_t lead = 0;
     uint64_t st[kPer];
     uint64_t prev = tid ? s_h[tid * kPer - 1] : 0;
@@ -566,7 +573,8 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
         for (int q = 0; q < kPer; q++) {
             st[q] = p;
             const uint32_t w1 = (uint32_t)p, w0 = (uint32_t)p - (uint32_t)prev;
-            if ((tid == 0 && q == 0) || w1 / kBinAim != w0 / kBinAim) lead |= 1u << q;
+            if ((tid == 0 && q == 0) || w1 / aim != w0 / aim || (uint32_t)v[q] > aim / 3 || (uint32_t)prev > aim / 3)
+                lead |= 1u << q;
             prev = v[q];
             p += v[q];
         }
@@ -691,11 +699,12 @@ __device__ __forceinline__ void bases64(const uint64_t *__restrict__ packed, uin
     }
 }
 
+// multiply-add hash of a key's 24-bit pieces (24-bit products run at the full
+// rate, 32-bit ones at a quarter of it); its top bits are the good ones
 __device__ __forceinline__ uint32_t key_hash(uint64_t k)
 {
-    uint32_t x = ((uint32_t)k * 0x9E3779B1u) ^ ((uint32_t)(k >> 32) * 0x85EBCA77u);
-    x ^= x >> 15;
-    return x * 0x2C1B3C6Du;
+    const uint32_t a = (uint32_t)k, b = (uint32_t)(k >> 24), c = (uint32_t)(k >> 48);
+    return __umul24(a & 0xFFFFFF, 0xD1B54B) + __umul24(b & 0xFFFFFF, 0x9E3779) + __umul24(c, 0xB5297A5 & 0xFFFFFF);
 }
 
 constexpr uint64_t kNoKey = ~0ull;  // k <= 31: no k-mer
@@ -752,7 +761,7 @@ __device__ __forceinline__ void side_verdict(const uint32_t tl[4], uint32_t len,
 }
 
 // meta word of a slot, first the tallies ...
-constexpr uint32_t kCntMask = 0xFFFF;         // tuples; 16-19: in classes seen, 20-23: out classes seen
+constexpr uint32_t kCntMask = 0xFFFF;  // tuples; 16 + c: in class c seen, 24 + c: out class c (7, 'N', is not counted)
 // ... then the run's verdict: place of its labels (13 bits) and
 constexpr uint32_t kRunJoin = 1u << 13, kRunSide = 1u << 14, kRunOut = 1u << 15, kRunWit = 1u << 31, kRunRatio = 1u << 28;
 constexpr uint32_t kRunLast = kRunRatio;  // CHECK: the last run of the last segment
@@ -768,116 +777,194 @@ __device__ __forceinline__ void note_found(uint32_t f, uint32_t *flag)
     if (all && __lane_id() == 0 && (all & ~*flag)) atomicOr(flag, all);
 }
 
-template <bool CHECK>
+// LDS of bin_runs: the staged records are dead once every window is expanded
+// into registers, so the table takes their place; its keys are dead once the
+// runs are evaluated, and make room for the labels and the side tallies.
+struct RunsStage {
+    ulonglong2 fw[kBinRec];   // 64 bases from the one before the first window
+    ulonglong2 rc[kBinRec];   // their reverse complement, from 32 - K bases on
+    uint32_t lab[kBinRec];
+    uint32_t map[kBinCap];    // window: record | its place in the record << 10 | 'N' class before << 15, after << 16
+};
+struct RunsTable {
+    unsigned long long key[kBinCap];
+    uint32_t meta[kBinCap];
+};
+union RunsLds {
+    RunsStage st;
+    RunsTable tb;
+    struct {
+        uint32_t lab[kBinCap];      // labels in run order
+        uint32_t tal[kBinCap];      // 4 x 16-bit tallies of every branching side
+    } out;
+};
+
+// CHECK: only note which live labels there are (the first-run quirk's test).
+// PART: the scan holds part of the buckets.
+template <bool CHECK, bool PART>
 __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
 {
-    constexpr int kPer = kBinCap / kRunThreads;  // windows and slots a lane
+    constexpr int kPer = kBinCap / kRunThreads;  // windows a lane, distinct k-mers a lane at most
     constexpr int kWaves = kRunThreads / kWave;
-    __shared__ __align__(16) unsigned long long s_key[kBinCap];
-    __shared__ uint32_t s_meta[kBinCap];
-    __shared__ __align__(16) ulonglong2 s_seq[kBinRec];
-    __shared__ uint32_t s_lab[kBinRec];
-    __shared__ uint8_t s_fl[kBinRec];
-    __shared__ unsigned long long s_wb[kBinCap / 64 + 2];  // record starts among the windows
-    __shared__ uint16_t s_wp[kBinCap / 64 + 1];            // records that start before a word
-    __shared__ unsigned long long s_ob[kBinCap / 64];      // run starts among the labels
-    __shared__ uint32_t s_sum[kWaves], s_red[3];
+    __shared__ __align__(16) RunsLds U;
+    __shared__ uint16_t s_list[kBinCap];               // slots in use
+    __shared__ unsigned long long s_ob[kBinCap / 64];  // run starts among the labels
+    __shared__ uint32_t s_sum[kWaves], s_nkey, s_red[3];
     __shared__ uint64_t s_out;
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const BinDesc d = P.bins[blockIdx.x];
     const int K = P.K;
-    // the records' windows are laid end to end: a record a lane
-    static_assert(kBinRec == kRunThreads, "a record a lane");
-    const uint4 rc = P.rec[d.rec0 + min(tid, d.nrec - 1)];
-#pragma unroll
-    for (int q = 0; q < kPer; q++) {
-        s_key[q * kRunThreads + tid] = kNoKey;
-        s_meta[q * kRunThreads + tid] = 0;
+    static_assert(kBinRec <= kRunThreads, "a record a lane");
+    const bool have = tid < d.nrec;
+    uint4 rc = make_uint4(0u, 0u, 0u, 0u);
+    uint64_t fh = 0, fl = 0;
+    if (have) {
+        rc = P.rec[d.rec0 + tid];
+        bases64(P.packed, (((uint64_t)rc.y << 32) | rc.x) & ((1ull << 40) - 1), fh, fl);
     }
-    if (tid < kBinCap / 64 + 2) s_wb[tid] = 0;
-    if (tid < kBinCap / 64) s_ob[tid] = 0;
-    if (tid < 3) s_red[tid] = 0;
-    const uint32_t L = tid < d.nrec ? (rc.y >> 8) & 31 : 0u;
+    const uint32_t L = (rc.y >> 8) & 31;  // 0 past the records
     const uint32_t inc = wave_incl(L);
     if (lane == kWave - 1) s_sum[wave] = inc;
-    uint64_t bh, bl;
-    bases64(P.packed, (((uint64_t)rc.y << 32) | rc.x) & ((1ull << 40) - 1), bh, bl);
+    if (tid < kBinCap / 64) s_ob[tid] = 0;
+    if (tid < 3) s_red[tid] = 0;
+    if (tid == 0) s_nkey = 0;
     __syncthreads();
-    {
+    if (have) {  // the records' windows laid end to end
         uint32_t o = inc - L;
         for (uint32_t w = 0; w < wave; w++) o += s_sum[w];
-        if (L) {
-            s_seq[tid] = make_ulonglong2(bh, bl);
-            s_lab[tid] = rc.z;
-            s_fl[tid] = (uint8_t)((rc.y >> 13) & 3);
-            atomicOr(&s_wb[o >> 6], 1ull << (o & 63));
+        U.st.fw[tid] = make_ulonglong2(fh, fl);
+        const uint64_t rh = revcomp(fl, 32), rl = revcomp(fh, 32);
+        const int sh = 2 * (32 - K);  // 2 .. 24
+        U.st.rc[tid] = make_ulonglong2((rh << sh) | (rl >> (64 - sh)), rl << sh);
+        U.st.lab[tid] = rc.z;
+        const uint32_t f = (rc.y >> 13) & 3;
+        uint32_t e = tid | ((f & kPrevN) << 15);
+        for (uint32_t q = 0; q + 1 < L; q++) {
+            U.st.map[o + q] = e;
+            e = (e & 0x7FFF) + 1024;
         }
-        if (tid == 0) atomicOr(&s_wb[d.nwin >> 6], 1ull << (d.nwin & 63));  // the end starts no record, but ends one
+        U.st.map[o + L - 1] = e | ((f & kNextN) << 15);
     }
     __syncthreads();
-    if (wave == 0) {
-        const uint32_t c = (uint32_t)__popcll(s_wb[lane]), i = wave_incl(c);
-        s_wp[lane] = (uint16_t)(i - c);
-    }
-    __syncthreads();
-    // every window: its k-mer into the table, its place in the run, the classes seen
-    uint32_t st[kPer], lab[kPer];
-    uint32_t nin = 0;
+    // every window's k-mer, neighbour classes and label
+    uint64_t key[kPer];
+    uint32_t lab[kPer], st[kPer];  // st: slot | place in its run << 12 | classes << 24; ~0: no tuple
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-        const uint32_t w = i * kWaves + wave;
+        const uint32_t j = i * kRunThreads + tid;
         st[i] = ~0u;
         lab[i] = 0;
-        if (w * kWave >= d.nwin) continue;
-        const uint32_t j = w * kWave + lane;
+        key[i] = 0;
         if (j < d.nwin) {
-            const uint64_t bits = s_wb[w];
-            const uint64_t up = bits & (lane == 63 ? ~0ull : (2ull << lane) - 1);
-            const uint32_t r = s_wp[w] + (uint32_t)__popcll(up) - 1;
-            const uint32_t o = up ? lane - (63 - (uint32_t)__builtin_clzll(up))
-                                  : lane + 1 + (uint32_t)__builtin_clzll(s_wb[w - 1]);
-            const bool last = lane == 63 ? s_wb[w + 1] & 1 : (bits >> (lane + 1)) & 1;
-            const ulonglong2 sq = s_seq[r];
-            const uint32_t fl = s_fl[r];
-            lab[i] = s_lab[r];
-            const Window x = expand(sq.x, sq.y, o, o == 0 && (fl & kPrevN), last && (fl & kNextN), K, P.lo, P.hi);
-            if (x.in) {
-                bool fresh;
-                const uint32_t s = table_slot(s_key, x.key, key_hash(x.key), fresh);
-                const uint32_t ci = x.cls & 7, co = x.cls >> 3;
-                const uint32_t seen = (ci < 4 ? 1u << (16 + ci) : 0u) | (co < 4 ? 1u << (20 + co) : 0u);
-                const uint32_t old = atomicAdd(&s_meta[s], 1u);
-                if (seen & ~old) atomicOr(&s_meta[s], seen);
-                st[i] = s | ((old & 0xFFF) << 12) | (x.cls << 24);
-                nin++;
+            const uint32_t m = U.st.map[j], r = m & 1023, o2 = (m >> 9) & 62;
+            const ulonglong2 f = U.st.fw[r], g = U.st.rc[r];
+            lab[i] = U.st.lab[r];
+            const uint64_t y = (f.x << o2) | ((f.y >> 1) >> (63 - o2));
+            const uint32_t q2 = 60 - o2;
+            const uint64_t z = (g.x << q2) | ((g.y >> 1) >> (63 - q2));
+            // y: base before, K bases ...; z: complement of the base after, reverse complement of the K bases ...
+            const uint64_t F = (y << 2) >> (64 - 2 * K), R = (z << 2) >> (64 - 2 * K);
+            const bool fwd = F < R;
+            key[i] = fwd ? F : R;
+            const uint32_t yh = (uint32_t)(y >> 32), zh = (uint32_t)(z >> 32);
+            const uint32_t u = (fwd ? zh : yh) >> 30, v = (fwd ? yh : zh) >> 30;
+            // class of a base: bits 1-3 of its letter (A 0, C 1, T 2, G 3), code ^ code >> 1; the complement flips bit 1
+            const uint32_t pn = (m >> 15) & 1, nn = (m >> 16) & 1;
+            const uint32_t ci = (u ^ (u >> 1) ^ 2) | ((fwd ? nn : pn) ? 7u : 0u), co = (v ^ (v >> 1)) | ((fwd ? pn : nn) ? 7u : 0u);
+            const uint32_t b = (uint32_t)(key[i] >> (2 * K - 20));
+            if (!PART || (b >= P.lo && b < P.hi)) st[i] = (ci << 24) | (co << 27) | (key_hash(key[i]) >> 20);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+        U.tb.key[q * kRunThreads + tid] = kNoKey;
+        U.tb.meta[q * kRunThreads + tid] = 0;
+    }
+    __syncthreads();
+    // into the table: the first probes of a lane's windows together, then the
+    // ones that met another k-mer (a lane's next unsettled window per step, so
+    // that a wave takes the longest sum over a lane's windows, not the sum of
+    // its longest probes)
+    uint32_t open = 0, fresh = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; i++) {
+        if (st[i] == ~0u) continue;
+        const uint64_t old = atomicCAS(&U.tb.key[st[i] & 0xFFF], kNoKey, (unsigned long long)key[i]);
+        if (old == kNoKey) fresh |= 1u << i;
+        else if (old != key[i]) open |= 1u << i;
+    }
+    while (__any(open != 0)) {
+        if (open) {
+            const uint32_t i = (uint32_t)__builtin_ctz(open);
+            uint64_t k = key[0];
+            uint32_t s = st[0];
+#pragma unroll
+            for (int q = 1; q < kPer; q++) {
+                k = i == (uint32_t)q ? key[q] : k;
+                s = i == (uint32_t)q ? st[q] : s;
             }
+            const uint32_t n = (s + 1) & 0xFFF;
+            const uint64_t old = atomicCAS(&U.tb.key[n], kNoKey, (unsigned long long)k);
+            s = (s & ~0xFFFu) | n;
+#pragma unroll
+            for (int q = 0; q < kPer; q++) st[q] = i == (uint32_t)q ? s : st[q];
+            if (old == kNoKey) fresh |= 1u << i;
+            if (old == kNoKey || old == k) open &= open - 1;
+        }
+    }
+    // counts, places and classes seen; the slots taken first to the list
+    {
+        const uint32_t nf = (uint32_t)__popc(fresh), fi = wave_incl(nf);
+        uint32_t at = 0;
+        if (lane == kWave - 1) at = atomicAdd(&s_nkey, fi);
+        at = __shfl(at, kWave - 1, kWave) + fi - nf;
+        uint32_t old[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; i++)
+            if (st[i] != ~0u) old[i] = atomicAdd(&U.tb.meta[st[i] & 0xFFF], 1u);
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            if (st[i] == ~0u) continue;
+            const uint32_t s = st[i] & 0xFFF;
+            const uint32_t seen = (1u << (16 + ((st[i] >> 24) & 7))) | (1u << (24 + (st[i] >> 27)));
+            if (seen & ~old[i]) atomicOr(&U.tb.meta[s], seen);
+            if ((fresh >> i) & 1) s_list[at++] = (uint16_t)s;
+            st[i] |= (old[i] & 0xFFF) << 12;
         }
     }
     __syncthreads();
     // every run: evaluated unless it is its segment's last
-    uint32_t sm[kPer], run[kPer];  // tallies; verdict
-    uint32_t add = 0, nev = 0, nz = 0;
-    const uint64_t lk = P.T == 1 || P.batch ? P.ctl->kmax1[d.smp] : 0;
+    const uint32_t nkey = s_nkey;
+    uint32_t cnt[kPer], run[kPer], at[kPer];  // tuples; verdict; slot
+    uint32_t add = 0, nz = 0, nlast = 0;
+    const bool one = P.T == 1 || P.batch;
+    const uint64_t lk = one ? P.ctl->kmax1[d.smp] : 0;
 #pragma unroll
-    for (int i = 0; i < kPer; i++) {
-        const uint32_t s = i * kRunThreads + tid;
-        const uint32_t m = s_meta[s], c = m & kCntMask;
-        sm[i] = m;
-        run[i] = 0;
-        if (!c) continue;
-        const uint64_t key = s_key[s];
-        const bool is_last = key + 1 == (P.T == 1 || P.batch ? lk : last_of(P, key, d.smp));
-        const bool bi = __popc((m >> 16) & 15) > 1, bo = __popc((m >> 20) & 15) > 1;
-        nev += !is_last;
+    for (int q = 0; q < kPer; q++) {
+        cnt[q] = run[q] = at[q] = 0;
+        if (q * kRunThreads >= nkey) continue;  // uniform
+        const uint32_t x = q * kRunThreads + tid;
+        if (x >= nkey) continue;
+        const uint32_t s = s_list[x], m = U.tb.meta[s], c = m & kCntMask;
+        const uint64_t k = U.tb.key[s];
+        const uint32_t b = (uint32_t)(k >> (2 * K - 20));
+        at[q] = s;
+        cnt[q] = c;
+        const bool is_last = k + 1 == (one ? lk : last_of(P, k, d.smp));
+        const uint32_t mi = (m >> 16) & 15, mo = (m >> 24) & 15;
+        const bool bi = mi & (mi - 1), bo = mo & (mo - 1);  // more than one class
+        nlast += is_last;
         const bool zero = !is_last && bi && bo;
         nz += zero;
         uint32_t v = 0;
         if (!zero) {
-            if (c >= 2 && key != 0) v |= kRunJoin;
+            if (c >= 2 && k != 0) v |= kRunJoin;
             if (!is_last && (bi || bo)) v |= kRunSide | (bo ? kRunOut : 0u);
-            if (key != 0 && (uint32_t)(key >> (2 * K - 20)) >= P.last_lo) v |= !is_last ? kRunWit : CHECK ? kRunLast : 0u;
+            if (k != 0 && b >= P.last_lo) v |= !is_last ? kRunWit : CHECK ? kRunLast : 0u;
         }
-        run[i] = v;
+        if (!PART && b >= P.hi) atomicOr(&P.ctl->err, kErrRange);
+        run[q] = v;
         add += ((v & kRunJoin) ? c : 0u) | ((v & kRunSide) ? 1u << 16 : 0u);
     }
     const uint32_t ainc = wave_incl(add);
@@ -890,77 +977,79 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         tot += s_sum[w];
     }
     const uint32_t nout = tot & 0xFFFF, nside = tot >> 16, npad = (nout + 63) & ~63u;
-    uint32_t *const s_lout = (uint32_t *)s_key;           // labels in run order
-    uint32_t *const s_tal = (uint32_t *)s_key + kBinCap;  // 4 x 16-bit tallies of the branching side
     if (!CHECK && tid == 0) {
         s_out = npad ? atomicAdd(&P.ctl->out, (unsigned long long)npad) : 0;
         if (s_out + npad > P.out_cap) atomicOr(&P.ctl->err, 8u);
     }
 #pragma unroll
-    for (int i = 0; i < kPer; i++) {
-        if (!(sm[i] & kCntMask)) continue;
-        uint32_t v = run[i];
+    for (int q = 0; q < kPer; q++) {
+        if (!cnt[q]) continue;
+        uint32_t v = run[q];
         if (v & kRunJoin) {
             const uint32_t p = base & 0xFFFF;
             v |= p;
             if (!CHECK) atomicOr(&s_ob[p >> 6], 1ull << (p & 63));
-            base += sm[i] & kCntMask;
+            base += cnt[q];
         }
         if (v & kRunSide) {
             v |= (base >> 16) << 16;
+            if (!CHECK) {  // the list's slots are in registers: the sides' slots and lengths take its place
+                s_list[base >> 16] = (uint16_t)at[q];
+                s_list[kBinCap / 2 + (base >> 16)] = (uint16_t)cnt[q];
+            }
             base += 1u << 16;
         }
-        run[i] = v;
-        s_meta[i * kRunThreads + tid] = v;
+        U.tb.meta[at[q]] = v;
     }
     if (!CHECK)
-        for (uint32_t j = tid; j < 2 * nside; j += kRunThreads) s_tal[j] = 0;
+        for (uint32_t j = tid; j < 2 * nside; j += kRunThreads) U.out.tal[j] = 0;
     __syncthreads();
     if constexpr (CHECK) {
         uint32_t f = 0;
 #pragma unroll
         for (int i = 0; i < kPer; i++) {
             if (st[i] == ~0u) continue;
-            const uint32_t v = s_meta[st[i] & 0xFFF];
+            const uint32_t v = U.tb.meta[st[i] & 0xFFF];
             if ((v & (kRunWit | kRunLast)) && !P.bad[lab[i]]) f |= v & kRunWit ? kFoundOther : kFoundLast;
         }
         note_found(f, &P.ctl->found[P.batch ? d.smp : 0]);
         return;
     }
+    uint32_t ver[kPer], nin = 0;
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
+        ver[i] = 0;
         if (st[i] == ~0u) continue;
-        const uint32_t v = s_meta[st[i] & 0xFFF];
-        if (v & kRunJoin) s_lout[(v & 0x1FFF) + ((st[i] >> 12) & 0xFFF)] = lab[i];
+        nin++;
+        const uint32_t v = U.tb.meta[st[i] & 0xFFF];
+        ver[i] = v;
+        if (v & kRunJoin) U.out.lab[(v & 0x1FFF) + ((st[i] >> 12) & 0xFFF)] = lab[i];
         if (v & kRunSide) {
             const uint32_t c = (st[i] >> ((v & kRunOut) ? 27 : 24)) & 7;
-            if (c < 4) atomicAdd(&s_tal[2 * ((v >> 16) & 0xFFF) + (c >> 1)], 1u << (16 * (c & 1)));
+            if (c < 4) atomicAdd(&U.out.tal[2 * ((v >> 16) & 0xFFF) + (c >> 1)], 1u << (16 * (c & 1)));
         }
-        if (i == 0) {
+        if (i == 0 && wave < kBinWit) {
             const uint64_t wm = __ballot((v & kRunWit) != 0);
-            if (wave < kBinWit && wm && (wm & lanemask_lt()) == 0 && (v & kRunWit)) P.wit[blockIdx.x * kBinWit + wave] = lab[i];
+            if (wm && (wm & lanemask_lt()) == 0 && (v & kRunWit)) P.wit[blockIdx.x * kBinWit + wave] = lab[i];
         }
     }
     if (nside) {
         __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kPer; i++) {
-            if (!(run[i] & kRunSide)) continue;
-            const uint32_t h = 2 * ((run[i] >> 16) & 0xFFF), t0 = s_tal[h], t1 = s_tal[h + 1];
+        for (uint32_t h = tid; h < nside; h += kRunThreads) {
+            const uint32_t sl = s_list[h], t0 = U.out.tal[2 * h], t1 = U.out.tal[2 * h + 1];
             const uint32_t tl[4] = {t0 & 0xFFFF, t0 >> 16, t1 & 0xFFFF, t1 >> 16};
             uint32_t arg;
             bool ratio;
-            side_verdict(tl, sm[i] & kCntMask, arg, ratio);
-            s_meta[i * kRunThreads + tid] = run[i] | (ratio ? kRunRatio : 0u) | (arg << 29);
+            side_verdict(tl, s_list[kBinCap / 2 + h], arg, ratio);
+            U.tb.meta[sl] |= (ratio ? kRunRatio : 0u) | (arg << 29);
         }
     }
     __syncthreads();
     if (nside) {
 #pragma unroll
         for (int i = 0; i < kPer; i++) {
-            if (st[i] == ~0u) continue;
-            const uint32_t v = s_meta[st[i] & 0xFFF];
-            if (!(v & kRunSide)) continue;
+            if (!(ver[i] & kRunSide)) continue;
+            const uint32_t v = U.tb.meta[st[i] & 0xFFF];
             const uint32_t c = (st[i] >> ((v & kRunOut) ? 27 : 24)) & 7;
             if ((v & kRunRatio) || c != ((v >> 29) & 3)) P.filtered[lab[i]] = 1;
         }
@@ -968,24 +1057,27 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     const uint64_t ob = s_out;
     const bool room = ob + npad <= P.out_cap;
     if (room)
-        for (uint32_t j = tid; j < npad; j += kRunThreads) P.lab_out[ob + j] = j < nout ? s_lout[j] : 0u;
+        for (uint32_t j = tid; j < npad; j += kRunThreads) P.lab_out[ob + j] = j < nout ? U.out.lab[j] : 0u;
     if (room && tid * 64 < npad) {
         uint64_t m = s_ob[tid];
         if (tid * 64 + 64 > nout) m |= ~0ull << (nout & 63);  // the padding: runs of one
         P.st_bits[ob / 64 + tid] = m;
     }
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        nev += __shfl_down(nev, o, kWave);
-        nz += __shfl_down(nz, o, kWave);
-        nin += __shfl_down(nin, o, kWave);
+    const uint64_t zm = __ballot(nz != 0);
+    if (zm) {
+        for (int o = kWave / 2; o > 0; o >>= 1) nz += __shfl_down(nz, o, kWave);
+        if (lane == 0) atomicAdd(&s_red[1], nz);
     }
-    if (lane == 0) {
-        atomicAdd(&s_red[0], nev);
-        if (nz) atomicAdd(&s_red[1], nz);
-        atomicAdd(&s_red[2], nin);
+    if (nlast) atomicSub(&s_red[0], nlast);
+    if constexpr (PART) {
+        for (int o = kWave / 2; o > 0; o >>= 1) nin += __shfl_down(nin, o, kWave);
+        if (lane == 0) atomicAdd(&s_red[2], nin);
     }
     __syncthreads();
-    if (tid < 3 && s_red[tid]) atomicAdd(&P.ctl->stat[blockIdx.x % kStripes][tid], (unsigned long long)s_red[tid]);
+    if (tid < 3) {
+        const uint32_t v = s_red[tid] + (tid == 0 ? nkey : tid == 2 && !PART ? d.nwin : 0u);
+        if (v) atomicAdd(&P.ctl->stat[blockIdx.x % kStripes][tid], (unsigned long long)v);
+    }
 }
 
 // A bin past the table: its windows in parts by the top bits of the k-mer's
@@ -1485,7 +1577,9 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     if (!batch)
         for (int i = 0; i < T; i++)
             if (hc->kmax1[i]) last_lo = h_bnd[i];
-    const uint64_t bin_cap = nv / kBinAim + kNC + 64;
+    // bins of at most kBinRec records, with room for the cell that passes the aim
+    const uint32_t aim = (uint32_t)std::max<uint64_t>(512, std::min<uint64_t>(kBinAim, nv * (kBinRec * 3 / 4) / nrec));
+    const uint64_t bin_cap = 7 * nv / aim + kNC + 64;  // a cell of more than aim / 3 windows starts two
     MP_ROOM(ensure(ctx, ctx->keys[1], nrec * sizeof(BinRec)));
     MP_ROOM(ensure(ctx, ctx->lab[1], bin_cap * (2 * sizeof(BinDesc) + kBinWit * sizeof(uint32_t) * 2)));
     BinDesc *const d_bins = (BinDesc *)ctx->lab[1].p, *const d_big = d_bins + bin_cap;
@@ -1498,11 +1592,11 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     if (cell_bits == 13)
         hipLaunchKernelGGL((bin_group_kernel<8192>), dim3(kNC), dim3(1024), 0, ctx->stream, (const uint4 *)rec_a,
                            (const uint32_t *)d_coarse, (const uint32_t *)(batch ? d_smp : nullptr), rec_b, d_bins, d_big,
-                           (uint32_t)bin_cap, d_ctl);
+                           (uint32_t)bin_cap, aim, d_ctl);
     else
         hipLaunchKernelGGL((bin_group_kernel<2048>), dim3(kNC), dim3(1024), 0, ctx->stream, (const uint4 *)rec_a,
                            (const uint32_t *)d_coarse, (const uint32_t *)(batch ? d_smp : nullptr), rec_b, d_bins, d_big,
-                           (uint32_t)bin_cap, d_ctl);
+                           (uint32_t)bin_cap, aim, d_ctl);
     MP_HIP(hipGetLastError());
     MP_HIP(hipMemcpyAsync(hc.get(), d_ctl, sizeof(BinCtl), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
@@ -1534,12 +1628,16 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     R.st_bits = (uint64_t *)ctx->runbits.p;
     R.out_cap = out_cap;
     R.ctl = d_ctl;
+    // every k-mer is in the scan when the histogram sized it so; a k-mer outside it all the same sets kErrRange
+    const bool n_part = !batch && !(lo == 0 && (hi == MP_NBUCKETS || job.expected == nv));
     auto runs = [&](bool check) -> int {
         R.bins = d_bins;
         R.nbin = (uint32_t)nbin;
         R.wit = d_wit;
-        if (nbin && check) hipLaunchKernelGGL(bin_runs_kernel<true>, dim3((unsigned)nbin), dim3(kRunThreads), 0, ctx->stream, R);
-        if (nbin && !check) hipLaunchKernelGGL(bin_runs_kernel<false>, dim3((unsigned)nbin), dim3(kRunThreads), 0, ctx->stream, R);
+        const dim3 gs((unsigned)nbin), ts(kRunThreads);
+        if (nbin && check) hipLaunchKernelGGL((bin_runs_kernel<true, true>), gs, ts, 0, ctx->stream, R);
+        if (nbin && !check && n_part) hipLaunchKernelGGL((bin_runs_kernel<false, true>), gs, ts, 0, ctx->stream, R);
+        if (nbin && !check && !n_part) hipLaunchKernelGGL((bin_runs_kernel<false, false>), gs, ts, 0, ctx->stream, R);
         R.bins = d_big;
         R.nbin = (uint32_t)nbig;
         R.wit = d_wit + nbin * kBinWit;
@@ -1568,7 +1666,12 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
         }
         return 0;
     };
-    if (hc->err) return restore();  // the radix path marks the same reads again
+    if (hc->err & ~kErrRange) return restore();  // the radix path marks the same reads again
+    if (hc->err) {
+        MP_TRY(restore());
+        return ctx->fail(MP_ECOUNT, "scan %d: the histogram's %llu tuples are not all in its buckets", job.s,
+                         (unsigned long long)job.expected);
+    }
     if (job.expected && n != job.expected) {
         MP_TRY(restore());
         return ctx->fail(MP_ECOUNT, "scan %d enumerated %llu tuples, the histogram sized %llu", job.s,
