@@ -523,8 +523,6 @@ __device__ __forceinline__ bool is_bad(const uint64_t *bits, uint32_t x) { retur
 // labels, so the work is the label and BAD-bit reads, not the finds.
 constexpr int kUW = 4;  // bitmap words a wave takes per step, their loads in flight together
 
-// ALL: every run is joined (rs_bits unused; a scan by minimizer bins lists only those)
-template <bool ALL>
 __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *__restrict__ rs_bits,
                                                     const uint64_t *__restrict__ st_bits,
                                                     const uint64_t *__restrict__ badbits)
@@ -543,7 +541,7 @@ __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *_
 #pragma unroll
         for (int u = 0; u < kUW; u++) {
             st[u] = w0 + u < nw ? st_bits[w0 + u] : 0;
-            rs[u] = ALL ? ~0ull : w0 + u < nw ? rs_bits[w0 + u] : 0;
+            rs[u] = w0 + u < nw ? rs_bits[w0 + u] : 0;
             lb[u] = G.lab[min((w0 + u) * 64 + lane, G.n - 1)];
         }
         // the run holding tuple w0 * 64 when it began before: its start and whether it is joined
@@ -555,7 +553,7 @@ __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *_
             if (m) {
                 const int bit = 63 - __builtin_clzll(m);
                 cs = q * 64 + bit;
-                cjoin = ALL || ((rs_bits[q] >> bit) & 1);
+                cjoin = (rs_bits[q] >> bit) & 1;
             }
         }
         uint32_t b[kUW];
@@ -617,6 +615,96 @@ __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *_
                         break;
                     }
                 }
+            }
+        }
+    }
+}
+
+// The same over a list that holds only runs to join (a scan by minimizer
+// bins), in whole bitmap words.  A wave takes kLW consecutive words, the loads
+// of kUW of them in flight together, and carries the last live label of the
+// run that goes on into the next word; only its first word may have to look
+// back in memory.  Most words of a shallow sample hold two or three live
+// labels, and most joins of a deep one are of labels joined before: a join
+// first compares the ancestors that plain (cached) loads reach, which may be
+// old but are always members of the same set, and takes the coherent find and
+// its compare-and-swap only where they differ.  Against union_kernel's way on
+// the same lists: 12 M reads at 5x (96 % BAD) 3.4 -> 2.4 ms, 2.2 M reads at 46x
+// 3.9 -> 1.6, a batch of 24 samples 1.5 -> 0.56.
+constexpr int kLW = 16;
+static_assert(kLW % kUW == 0, "whole steps");
+
+__device__ __forceinline__ void uf_join(uint32_t *parent, uint32_t a, uint32_t b)
+{
+    for (;;) {
+        const uint32_t pa = parent[a], pb = parent[b];
+        if (pa == pb) return;
+        if (pa == a && pb == b) break;
+        a = pa;
+        b = pb;
+    }
+    uf_union(parent, a, b);
+}
+
+__global__ __launch_bounds__(256) void union_list_kernel(const uint32_t *__restrict__ lab,
+                                                         const uint64_t *__restrict__ st_bits, uint64_t nw,
+                                                         const uint32_t *__restrict__ badbits, uint32_t *parent)
+{
+    const uint32_t lane = __lane_id();
+    const uint64_t w0 = (((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave) * kLW;
+    if (w0 >= nw) return;
+    const uint64_t lt = lanemask_lt(), upto = lane == 63 ? ~0ull : (2ull << lane) - 1;
+    uint32_t carry = 0;       // the last live label of the run that goes on, if any
+    bool have = false;
+    if (w0 > 0 && !(st_bits[w0] & 1)) {  // the wave's first run began before: its last live label (uniform)
+        for (uint64_t q = w0; q-- > 0 && !have;) {
+            const uint64_t m = st_bits[q];
+            const uint32_t l = lab[q * 64 + lane];
+            const int s = m ? 63 - __builtin_clzll(m) : 0;  // the run's start in this word, if it began here
+            const uint64_t v = __ballot((int)lane >= s && !((badbits[l >> 5] >> (l & 31)) & 1));
+            if (v) {
+                carry = __shfl(l, 63 - __builtin_clzll(v), kWave);
+                have = true;
+            }
+            if (m) break;
+        }
+    }
+    for (int g = 0; g < kLW && w0 + g < nw; g += kUW) {
+        uint64_t st[kUW];
+        uint32_t lb[kUW], bw[kUW];
+#pragma unroll
+        for (int u = 0; u < kUW; u++) {
+            const uint64_t w = min(w0 + g + u, nw - 1);
+            st[u] = st_bits[w];
+            lb[u] = lab[w * 64 + lane];
+        }
+#pragma unroll
+        for (int u = 0; u < kUW; u++) bw[u] = badbits[lb[u] >> 5];
+#pragma unroll
+        for (int u = 0; u < kUW; u++) {
+            if (w0 + g + u >= nw) break;
+            const bool live = !((bw[u] >> (lb[u] & 31)) & 1);
+            const uint64_t lv = __ballot(live);
+            if (lv) {
+                const uint64_t sm = st[u] & upto;
+                uint64_t cand = lv & lt;
+                if (sm) cand &= ~0ull << (63 - __builtin_clzll(sm));  // lanes of the same run
+                uint32_t a = __shfl(lb[u], cand ? 63 - __builtin_clzll(cand) : 0, kWave);
+                bool join = live && cand != 0;
+                if (live && !cand && !sm && have) {  // the first live label here of a run from before
+                    a = carry;
+                    join = true;
+                }
+                if (join && a != lb[u]) uf_join(parent, a, lb[u]);
+            }
+            // the run that goes on past this word
+            const uint64_t s = st[u];
+            const uint64_t tail = s ? lv & (~0ull << (63 - __builtin_clzll(s))) : lv;
+            if (tail) {
+                carry = __shfl(lb[u], 63 - __builtin_clzll(tail), kWave);
+                have = true;
+            } else if (s) {
+                have = false;
             }
         }
     }
@@ -1071,7 +1159,7 @@ static int filter_union_core(mp_ctx *ctx, uint64_t n, const uint64_t *d_seg, int
         hipLaunchKernelGGL(bad_bits_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint8_t *)G.bad, N,
                            badbits);
         MP_HIP(hipGetLastError());
-        hipLaunchKernelGGL(union_kernel<false>, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0, ctx->stream,
+        hipLaunchKernelGGL(union_kernel, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0, ctx->stream,
                            G, (const uint64_t *)rs_bits, (const uint64_t *)st_bits, (const uint64_t *)badbits);
         MP_HIP(hipGetLastError());
     }
@@ -1279,7 +1367,7 @@ int two_sweep_scan(mp_ctx *ctx, const std::vector<uint64_t> &cuts, const uint64_
                            badbits);
         const uint64_t rwords = (n + 63) / 64 + 1;
         const uint64_t *rs_bits = (const uint64_t *)ctx->runbits.p;
-        hipLaunchKernelGGL(union_kernel<false>, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0,
+        hipLaunchKernelGGL(union_kernel, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0,
                            ctx->stream, G, rs_bits, rs_bits + rwords, (const uint64_t *)badbits);
         MP_HIP(hipGetLastError());
         hipEventRecord(ctx->ev[5], ctx->stream);
@@ -1321,12 +1409,11 @@ int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, 
         uint64_t *badbits = (uint64_t *)ctx->scratch.p;
         hipLaunchKernelGGL(bad_bits_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint8_t *)ctx->bad.p, N,
                            badbits);
-        GParams G{};
-        G.lab = lab;
-        G.n = n;
-        G.parent = (uint32_t *)ctx->parent.p;
-        hipLaunchKernelGGL(union_kernel<true>, dim3(wave_grid(((n + 63) / 64 + kUW - 1) / kUW)), dim3(256), 0,
-                           ctx->stream, G, (const uint64_t *)nullptr, st_bits, (const uint64_t *)badbits);
+        const uint64_t nw = n / 64, blocks = ((nw + kLW - 1) / kLW + 3) / 4;
+        if (!grid_fits(blocks, 256))
+            return ctx->fail(MP_EINVAL, "union over %llu labels exceeds one dispatch: use more scans", (unsigned long long)n);
+        hipLaunchKernelGGL(union_list_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, lab, st_bits, nw,
+                           (const uint32_t *)badbits, (uint32_t *)ctx->parent.p);
         MP_HIP(hipGetLastError());
     }
     return compress_labels(ctx, (uint32_t *)ctx->parent.p, (const uint8_t *)ctx->bad.p, N);
