@@ -407,15 +407,6 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
     if (lane == 0 && rec_total) atomicAdd(&P.ctl->nrec, rec_total);
 }
 
-// read starts as bits, and one at the end of the last read (the array is zero before)
-__global__ void read_start_kernel(const uint64_t *__restrict__ base_off, uint64_t N, uint32_t *__restrict__ bits)
-{
-    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r > N) return;
-    const uint64_t b = base_off[r];
-    atomicOr(&bits[2 * (b >> 6) + 1 - ((b >> 5) & 1)], 0x80000000u >> (b & 31));
-}
-
 // ---------------------------------------------------------------- offsets of (tile, coarse bin)
 constexpr int kColTiles = 32;
 
@@ -1464,16 +1455,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
         MP_TRY(enough((x), &ok));  \
         if (!ok) return 0;         \
     } while (0)
-    // read starts
-    const uint64_t sw = (tb + 63) / 64 + 2;
-    MP_ROOM(ensure(ctx, ctx->rstart, sw * sizeof(uint64_t)));
-    if (!ctx->rstart_valid) {
-        MP_TRY(fill_u32(ctx, ctx->rstart.p, 0, 2 * sw));
-        hipLaunchKernelGGL(read_start_kernel, dim3((unsigned)((N + 256) / 256)), dim3(256), 0, ctx->stream,
-                           (const uint64_t *)ctx->base_off.p, N, (uint32_t *)ctx->rstart.p);
-        MP_HIP(hipGetLastError());
-        ctx->rstart_valid = true;
-    }
+    MP_ROOM(read_starts(ctx));
     // tables: counts per tile, chunk sums, coarse bins, per step counts and ranks, the segments
     const uint64_t o_csum = (uint64_t)tiles * kNC * 4, o_coarse = o_csum + (uint64_t)chunks * kNC * 4,
                    o_nrec = o_coarse + (kNC + 1) * 4, o_rank = o_nrec + nsteps * 4, o_bnd = o_rank + nsteps * 4,

@@ -124,7 +124,7 @@ struct mp_ctx {
 
     // per-read arrays
     mp::DevArray fq, rec_off, seq_off, seq_len, base_off, pos_off, packed, nmask;
-    mp::DevArray rstart;        // read starts, one bit per base (laid out as nmask), for scans by minimizer bins
+    mp::DevArray rstart;        // read starts, one bit per base (laid out as nmask): read_starts()
     bool rstart_valid = false;
     bool plain_letters = false; // no empty read, and no letter but 'N' with bit 3 set: the 2-bit code gives a base's neighbour class
     // graph state
@@ -135,7 +135,7 @@ struct mp_ctx {
     mp::DevArray keys[2], lab[2], adj[2], zbits;
     mp::DevArray runbits;  // filter -> union: starts of runs to join, starts of all runs
     mp::DevArray dig, rts; // counted radix passes: next pass's digit per tuple; per-tile counts and offsets
-    mp::DevArray gcnt;     // m-mer histogram: digit counts per generating-pass tile (a scan over every k-mer)
+    mp::DevArray gcnt;     // a batch's digit counts per generating-pass tile
     mp::DevArray segtab;   // a batch's per-sample generating-pass tiles: first tile, first window
     mp::DevArray binctl;   // scan by minimizer bins: its counters
     // the last scan went by minimizer bins: its sorted tuples are made when a dump asks for them
@@ -151,7 +151,7 @@ struct mp_ctx {
     uint64_t sort_graph_captures = 0, sort_graph_replays = 0;
     int sort_graph_last = 0;  // the last sort's chain: 0 launched pass by pass, 1 captured, 2 replayed
     std::vector<uint64_t> seg_wpos;  // first window of every sample (C + 1)
-    int khist_copies = 32; // copies of the byte counts in khist (one per sample for a batch)
+    int khist_copies = 0;  // samples that khist counts
     bool gcnt_seg = false; // gcnt over every sample's own tiles
     bool gcnt_valid = false;
     uint64_t gcnt_tile = 0, gcnt_tiles = 0;
@@ -161,7 +161,7 @@ struct mp_ctx {
     mp::DevArray hpart;   // m-mer histogram: tile table, partition bounds, work list
     mp::DevArray labsnap;  // a two-sweep scan's labels, taken at its start
     bool use_labsnap = false;
-    mp::DevArray khist;   // m-mer histogram: counts of the k-mer bytes the scans' radix passes read
+    mp::DevArray khist;   // a batch's counts of the k-mer bytes its radix passes read, per sample
     bool khist_valid = false;
     uint32_t khist_mask = 0;  // passes (bit 1 + byte) khist counts
     uint64_t kmer_total = 0;  // k-mers of the loaded reads (last m-mer histogram)
@@ -243,6 +243,8 @@ int fill_u32(mp_ctx *ctx, void *p, uint32_t v, uint64_t n_words);
 
 // stages (each .hip file)
 int parse_reads(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *chunk_first_id, int C);
+// read starts of the loaded reads as bits (ctx->rstart), and one at the end of the last; made once per load
+int read_starts(mp_ctx *ctx);
 int count_chunks_device(mp_ctx *ctx, const uint64_t *chunk_first_id, int C, uint32_t *d_counts);
 // A batch (chunk = sample): the byte counts of every sample and the generating
 // pass's digit counts over tiles of every sample's windows (gen_histograms

@@ -19,9 +19,8 @@
 // The plain tuples themselves are not enumerated into memory: the first radix
 // pass of the sort generates them from the reads in the same order (read
 // order, then position order within a read).  This file gives it the digit
-// counts: the m-mer histogram's counting pass also counts the k-mer bytes the
-// sort reads, and kmer_digit_hist_kernel counts a scan that holds part of the
-// buckets.
+// counts of the scan's k-mers (kmer_digit_hist_kernel; batch_count_kernel for
+// a batch sorted sample by sample).
 //
 // 3-minimizer variant (countMmers_3minimizers.c:83-271,
 // enumerateKmers_3minimizers.c:129-474): a sequential window state machine per
@@ -40,49 +39,251 @@ namespace mp {
 // The per-chunk table has 2^20 bins per chunk, far beyond LDS, and one global
 // atomic per k-mer is bound by the atomic rate of the memory side.  So the
 // histogram is built in three LDS-privatised steps:
-//   1. tiles of up to 1024 reads of one chunk count their k-mers per digit
-//      (top 5 bits of the 20-bit bucket) in LDS,
+//   1. tiles of one chunk's base positions count their k-mers per digit (top 7
+//      bits of the 20-bit bucket) in LDS,
 //   2. a scan over (chunk, digit, tile) places every tile's digit run, and the
-//      tiles write the low 15 bucket bits of each k-mer there (u16); few
-//      digits keep few partially written lines open per tile,
-//   3. each (chunk, digit) partition is counted in a 32K-bin LDS histogram and
+//      tiles group the low 13 bucket bits of their k-mers by digit in LDS and
+//      write each digit's run with neighbouring lanes,
+//   3. each (chunk, digit) partition is counted in an 8K-bin LDS histogram and
 //      written to its slice of the chunk's row.
-// Bucket order inside a run does not matter to a histogram, so step 2 takes
-// slots with LDS atomics instead of a stable ranking.
-constexpr int kHDigitBits = 5;
+// A k-mer's bucket needs no k-mer: the first 20 bits of the canonical code are
+// the smaller of its first 10 bases and the reverse complement of its last 10
+// (at k = 32 the reference's forward code is 0 past a read's first position).
+// So a lane takes 16 consecutive base positions of the 2-bit stream, with the
+// windows' validity from bit masks of the 'N's and the read starts.
+// Measured at 1.44e9 k-mers (k = 31, 16 chunks), steps 1, 2, 3: k-mers rolled
+// per lane, 5-bit digits, single 2-byte stores 3.0, 3.1, 1.0 ms; this form
+// 0.8, 2.2, 0.7 (and 0.15 for the read starts).
+constexpr int kHDigitBits = 7;
 constexpr int kHDigits = 1 << kHDigitBits;
 constexpr int kHLowBits = 20 - kHDigitBits;
 constexpr int kHLow = 1 << kHLowBits;
-constexpr uint32_t kHReads = 1024;       // reads per tile (steps 1, 2)
-constexpr uint64_t kHSlab = 4u << 20;    // items per workgroup (step 3)
+constexpr uint64_t kHSlab = 1u << 20;    // items per workgroup (step 3)
+constexpr int kHLanes = 512;
+constexpr int kHPos = 16 * kHLanes;      // base positions of a step (a tile is some steps)
+constexpr int kHCopies = 4;              // copies of a step's digit counters: lanes l, l + 1, .. take different ones
+constexpr int kHCopy = kHDigits + 16;    // words from one copy to the next (their banks differ)
 constexpr int kHWords = 1024;            // staged stream words of a group of kRG reads (150 bp: ~450)
 
-constexpr int kBhRep = 32;  // copies of the byte histograms (tile t adds to copy t % kBhRep)
-
-struct HParams {
-    unsigned long long *bh;     // kBhRep x 8 x 256 counts of the k-mer digits in bmask
-    uint32_t bmask;             // bit 1 + b: count digit b (the radix passes of the scans)
-    KeyLayout kl;               // the scans' key digits
-    const uint64_t *chunk_ids;  // C+1 first read ids
-    const uint32_t *tile0;      // C+1 first tile of each chunk
-    int C;
+struct HistParams {
+    const uint64_t *packed, *nmask, *rstart;  // 2-bit, 'N' and read-start streams
+    uint64_t nw32, nw64;        // words of the 2-bit stream and of the other two
+    const uint64_t *base_off;
+    uint64_t total;             // bases
+    int K, C;
+    const uint64_t *chunk_ids;  // C + 1 first read ids
+    uint64_t tile;              // base positions per tile, a multiple of kHPos
+    const uint32_t *tile0;      // C + 1 first tile of each chunk
     uint32_t *tcnt;             // [c][d][tile of c] digit counts
     const uint64_t *toff;       // exclusive scan of tcnt
     uint16_t *items;            // low bucket bits, grouped by (chunk, digit)
+};
+
+// a chunk's tiles cover its bases from the 16-aligned position at or before its first
+__global__ __launch_bounds__(256) void hist_tiles_kernel(HistParams P, uint32_t *__restrict__ tile0)
+{
+    __shared__ uint32_t s_n[256];
+    uint32_t run = 0;
+    for (int c0 = 0; c0 < P.C; c0 += 256) {
+        const int c = c0 + (int)threadIdx.x;
+        uint32_t n = 0;
+        if (c < P.C) {
+            const uint64_t a = P.base_off[P.chunk_ids[c]], e = P.base_off[P.chunk_ids[c + 1]];
+            n = e > a ? (uint32_t)((e - (a & ~15ull) + P.tile - 1) / P.tile) : 0u;
+        }
+        s_n[threadIdx.x] = n;
+        __syncthreads();
+        uint32_t before = run, all = 0;
+        for (int j = 0; j < 256; j++) {
+            before += j < (int)threadIdx.x ? s_n[j] : 0u;
+            all += s_n[j];
+        }
+        if (c < P.C) tile0[c] = before;
+        run += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) tile0[P.C] = run;
+}
+
+// What a lane needs of its 16 positions p .. p + 15 (p a multiple of 16): the
+// 48 bases, 'N' bits and read-start bits from p on, as the words that hold
+// them (loaded apart from their use, one step ahead).
+struct HistWords {
+    uint64_t b0, b1, n0, n1, e0, e1;
+};
+
+__device__ __forceinline__ HistWords hist_load(const HistParams &P, uint64_t p)
+{
+    HistWords w;
+    const uint64_t i = min(p >> 5, P.nw32 - 2), j = min(p >> 6, P.nw64 - 2);  // past the end: not used
+    w.b0 = P.packed[i];
+    w.b1 = P.packed[i + 1];
+    w.n0 = P.nmask[j];
+    w.n1 = P.nmask[j + 1];
+    w.e0 = P.rstart[j];
+    w.e1 = P.rstart[j + 1];
+    return w;
+}
+
+// Buckets of the windows at p .. p + 15 (fn(j, bucket) for each valid one), a
+// window at base i of the lane being valid when it has no 'N' in [i, i + K),
+// no read start in (i, i + K), is not a read of K bases, and i is in [lo, hi).
+template <typename Fn>
+__device__ __forceinline__ void hist_windows(const HistWords &w, int K, uint64_t p, uint64_t lo, uint64_t hi, Fn fn)
+{
+    const uint32_t o = (uint32_t)p & 48;
+    const uint64_t n = (w.n0 << o) | ((w.n1 >> 1) >> (63 - o)), e = (w.e0 << o) | ((w.e1 >> 1) >> (63 - o));
+    uint64_t x = n | (e << 1);
+    x |= x << 1;
+    x |= x << 2;
+    x |= x << 4;
+    if (K > 17) {
+        x |= x << 8;
+        x |= x << (K - 17);
+    } else {
+        x |= x << (K - 9);
+    }
+    x |= n << (K - 1);
+    x |= e & (e << K);
+    uint32_t V = (uint32_t)(~x >> 48);
+    const uint32_t in = p + 16 <= hi ? 16u : p < hi ? (uint32_t)(hi - p) : 0u;
+    V &= 0xFFFF0000u >> in;
+    V &= p >= lo ? 0xFFFFu : lo - p >= 16 ? 0u : 0xFFFFu >> (lo - p);
+    const uint32_t h0 = (uint32_t)(w.b0 >> 32), h1 = (uint32_t)w.b0, h2 = (uint32_t)(w.b1 >> 32), h3 = (uint32_t)w.b1;
+    const bool odd = p & 16;
+    const uint32_t X[3] = {odd ? h1 : h0, odd ? h2 : h1, odd ? h3 : h2};
+    // reverse complement of the 48 bases, from its base 33 - K on: the window at j takes 10 bases from 15 - j
+    uint32_t y[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const uint32_t v = __builtin_bitreverse32(~X[2 - q]);
+        y[q] = ((v >> 1) & 0x55555555u) | ((v & 0x55555555u) << 1);
+    }
+    const int off = 2 * (33 - K);  // 2 .. 44
+    const uint64_t w01 = ((uint64_t)y[0] << 32) | y[1], w12 = ((uint64_t)y[1] << 32) | y[2];
+    const uint64_t z = off < 32 ? (w01 << off) | ((uint64_t)y[2] >> (32 - off)) : w12 << (off - 32);
+    const uint64_t f = ((uint64_t)X[0] << 32) | X[1];
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        uint32_t b = min((uint32_t)((f << (2 * j)) >> 32), (uint32_t)((z << (2 * (15 - j))) >> 32)) >> 12;
+        if (K == 32 && !((e >> (63 - j)) & 1)) b = 0;
+        fn(j, b, (V >> (15 - j)) & 1);
+    }
+}
+
+// PHASE 0: digit counts per tile, 1: the low bits grouped by digit and written
+template <int PHASE>
+__global__ __launch_bounds__(kHLanes) void hist_pos_kernel(HistParams P)
+{
+    __shared__ uint32_t s_cnt[kHCopies * kHCopy];  // counts; PHASE 1: then the first place of every (digit, copy)
+    __shared__ uint32_t s_beg[PHASE == 1 ? kHDigits + 1 : 1];
+    __shared__ uint64_t s_out[PHASE == 1 ? kHDigits : 1];
+    __shared__ uint32_t s_buf[PHASE == 1 ? kHPos : 1];  // a step's buckets by digit
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    const uint32_t t = blockIdx.x;
+    if (t >= P.tile0[P.C]) return;
+    int c = 0, hi = P.C - 1;  // chunk: last c with tile0[c] <= t
+    while (c < hi) {
+        const int mid = (c + hi + 1) >> 1;
+        if (P.tile0[mid] <= t) c = mid; else hi = mid - 1;
+    }
+    const uint32_t tl = t - P.tile0[c], Tc = P.tile0[c + 1] - P.tile0[c];
+    const uint64_t cb = P.base_off[P.chunk_ids[c]], ce = P.base_off[P.chunk_ids[c + 1]];
+    const uint64_t p_beg = (cb & ~15ull) + (uint64_t)tl * P.tile, p_end = min(p_beg + P.tile, ce);
+    const uint64_t mbase = (uint64_t)kHDigits * P.tile0[c] + tl;
+    const int K = P.K;
+    for (uint32_t j = tid; j < kHCopies * kHCopy; j += kHLanes) s_cnt[j] = 0;
+    if (PHASE == 1 && tid < kHDigits) s_out[tid] = P.toff[mbase + (uint64_t)tid * Tc];
+    uint32_t *const cnt = s_cnt + (lane % kHCopies) * kHCopy;
+    HistWords nx = hist_load(P, p_beg + 16 * tid);
+    __syncthreads();
+    for (uint64_t p0 = p_beg; p0 < p_end; p0 += kHPos) {
+        const HistWords w = nx;
+        if (p0 + kHPos < p_end) nx = hist_load(P, p0 + kHPos + 16 * tid);
+        uint32_t bk[PHASE == 1 ? 16 : 1], rk[PHASE == 1 ? 8 : 1] = {};  // bucket (~0: none); place among the step's of its digit
+        hist_windows(w, K, p0 + 16 * tid, cb, p_end, [&](int j, uint32_t b, bool valid) {
+            if (PHASE == 0) {
+                if (valid) atomicAdd(&cnt[b >> kHLowBits], 1u);
+            } else {
+                bk[j] = valid ? b : ~0u;
+                if (valid) rk[j / 2] |= atomicAdd(&cnt[b >> kHLowBits], 1u) << (16 * (j & 1));
+            }
+        });
+        if (PHASE == 1) {
+            __syncthreads();
+            if (wave == 0) {  // the first places of the digits and of their copies
+                uint32_t run = 0;
+#pragma unroll
+                for (int q = 0; q < kHDigits / kWave; q++) {
+                    const uint32_t dg = q * kWave + lane;
+                    uint32_t c4[kHCopies], v = 0;
+#pragma unroll
+                    for (int y = 0; y < kHCopies; y++) v += c4[y] = s_cnt[y * kHCopy + dg];
+                    uint32_t inc = v;
+                    for (int o = 1; o < kWave; o <<= 1) {
+                        const uint32_t u = __shfl_up(inc, o, kWave);
+                        if (lane >= (uint32_t)o) inc += u;
+                    }
+                    uint32_t at = run + inc - v;
+                    s_beg[dg] = at;
+                    s_out[dg] -= at;  // the digit's next place, less its first place in the step
+#pragma unroll
+                    for (int y = 0; y < kHCopies; y++) {
+                        s_cnt[y * kHCopy + dg] = at;
+                        at += c4[y];
+                    }
+                    run += __shfl(inc, kWave - 1, kWave);
+                }
+                if (lane == 0) s_beg[kHDigits] = run;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+                if (bk[j] != ~0u) s_buf[cnt[bk[j] >> kHLowBits] + ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFF)] = bk[j];
+            __syncthreads();
+            const uint32_t m = s_beg[kHDigits];
+#pragma unroll 4
+            for (uint32_t i = tid; i < m; i += kHLanes) {
+                const uint32_t b = s_buf[i];
+                P.items[s_out[b >> kHLowBits] + i] = (uint16_t)(b & (kHLow - 1));
+            }
+            for (uint32_t j = tid; j < kHCopies * kHCopy; j += kHLanes) s_cnt[j] = 0;
+            __syncthreads();
+            if (tid < kHDigits) s_out[tid] += s_beg[tid + 1];
+        }
+    }
+    if (PHASE == 0) {
+        __syncthreads();
+        if (tid < kHDigits) {
+            uint32_t v = 0;
+            for (int y = 0; y < kHCopies; y++) v += s_cnt[y * kHCopy + tid];
+            P.tcnt[mbase + (uint64_t)tid * Tc] = v;
+        }
+    }
+}
+
+// A batch sorted by radix passes, each sample on its own: counts of the k-mer
+// digits its passes read per sample, and of the generating pass's digit per
+// tile of every sample's windows, over tiles of up to kBReads reads.
+constexpr uint32_t kBReads = 1024;
+
+struct HParams {
+    unsigned long long *bh;     // C x 8 x 256 counts of the k-mer digits in bmask
+    uint32_t bmask;             // bit 1 + b: count digit b (the radix passes of the scans)
+    KeyLayout kl;               // the scans' key digits
+    const uint64_t *chunk_ids;  // C+1 first read ids
+    const uint32_t *tile0;      // C+1 first tile of each sample
+    int C;
     // digit counts per tile of the generating radix pass (tiles of gtile
-    // consecutive windows), for a scan over every k-mer: gcnt[tile][digit] of
-    // the k-mer byte at gshift
+    // consecutive windows): gcnt[tile][digit] of the k-mer byte at gshift;
+    // sample c's tiles start at gft[c], its windows at gw[c] (C + 1 entries each)
     uint32_t *gcnt;
     uint64_t gtile;
     int gshift;
-    // a batch: byte counts per chunk (bh holds C copies), and generating-pass
-    // tiles over every chunk's own windows: chunk c's tiles start at gft[c],
-    // its windows at gw[c] (C + 1 entries each)
-    int per_chunk;
     const uint64_t *gft, *gw;
 };
 
-constexpr int kGenCntTiles = 24;  // generating-pass tiles a histogram tile counts in LDS (more: global atomics)
+constexpr int kGenCntTiles = 24;  // generating-pass tiles a tile counts in LDS (more: global atomics)
 
 struct HPiece {
     uint64_t b, e;   // item range
@@ -90,48 +291,33 @@ struct HPiece {
     uint32_t split;  // partition spread over several pieces: add atomically
 };
 
-// PHASE 0: digit counts per tile (GC: and the generating pass's digit counts
-// per tile, H.gcnt, whose LDS copy would otherwise cost the plain form two
-// thirds of its workgroups per CU), 1: scatter of the low bits
-template <int PHASE, bool GC = false>
-__global__ __launch_bounds__(kKBlock) void hist_tile_kernel(KParams P, HParams H)
+__global__ __launch_bounds__(kKBlock) void batch_count_kernel(KParams P, HParams H)
 {
     __shared__ uint32_t s_pref[kRG + 1];
     __shared__ uint64_t s_base[kRG];
-    __shared__ uint32_t s_dig[kHDigits];
-    __shared__ uint64_t s_out[kHDigits];
-    __shared__ uint32_t s_bh[PHASE == 0 ? 8 : 1][kSortRadix];
+    __shared__ uint32_t s_bh[8][kSortRadix];
     __shared__ uint64_t s_words[kHWords];  // the group's 2-bit words, then its 'N' words
     // digit d of a generating-pass tile in the 16-bit half d & 1 of word d / 2 (a
     // tile holds at most 2^16 - 1 windows): half the LDS, more workgroups per CU
-    __shared__ uint32_t s_gc[GC ? kGenCntTiles : 1][kSortRadix / 2];
+    __shared__ uint32_t s_gc[kGenCntTiles][kSortRadix / 2];
     static_assert(kSortRadix % 2 == 0, "two digits per word");
     const int tid = threadIdx.x;
-    if (PHASE == 0) {
-        for (int j = tid; j < 8 * kSortRadix; j += kKBlock) (&s_bh[0][0])[j] = 0;
-        if (GC)
-            for (int j = tid; j < kGenCntTiles * kSortRadix / 2; j += kKBlock) (&s_gc[0][0])[j] = 0;
-    }
+    for (int j = tid; j < 8 * kSortRadix; j += kKBlock) (&s_bh[0][0])[j] = 0;
+    for (int j = tid; j < kGenCntTiles * kSortRadix / 2; j += kKBlock) (&s_gc[0][0])[j] = 0;
     const uint32_t t = blockIdx.x;
     int c = 0, hi = H.C - 1;  // chunk: last c with tile0[c] <= t
     while (c < hi) {
         const int mid = (c + hi + 1) >> 1;
         if (H.tile0[mid] <= t) c = mid; else hi = mid - 1;
     }
-    const uint32_t tl = t - H.tile0[c], Tc = H.tile0[c + 1] - H.tile0[c];
-    const uint64_t rb = H.chunk_ids[c] + (uint64_t)tl * kHReads;
-    const uint64_t re = min(rb + kHReads, H.chunk_ids[c + 1]);
-    const uint64_t mbase = (uint64_t)kHDigits * H.tile0[c] + tl;
+    const uint32_t tl = t - H.tile0[c];
+    const uint64_t rb = H.chunk_ids[c] + (uint64_t)tl * kBReads;
+    const uint64_t re = min(rb + kBReads, H.chunk_ids[c + 1]);
     // the generating-pass tiles this tile's windows fall in: [g_lo, g_hi];
     // tiles count from `origin` (window) as tile `tbase`, up to window `cend`
     const uint64_t w_lo = P.pos_off[rb], w_hi = P.pos_off[re];
-    const uint64_t origin = H.per_chunk ? H.gw[c] : 0, tbase = H.per_chunk ? H.gft[c] : 0;
-    const uint64_t cend = H.per_chunk ? H.gw[c + 1] : ~0ull;
-    const uint64_t g_lo = H.gcnt ? tbase + (w_lo - origin) / H.gtile : 0;
-    if (tid < kHDigits) {
-        s_dig[tid] = 0;
-        if (PHASE == 1) s_out[tid] = H.toff[mbase + (uint64_t)tid * Tc];
-    }
+    const uint64_t origin = H.gw[c], tbase = H.gft[c], cend = H.gw[c + 1];
+    const uint64_t g_lo = tbase + (w_lo - origin) / H.gtile;
     for (uint64_t r0 = rb; r0 < re; r0 += kRG) {
         const int nr = (int)min((uint64_t)kRG, re - r0);
         __syncthreads();  // previous group done with s_pref / s_base
@@ -165,30 +351,22 @@ __global__ __launch_bounds__(kKBlock) void hist_tile_kernel(KParams P, HParams H
         // a lane's windows are consecutive: its generating-pass tile advances at most once per gtile windows
         uint64_t gt = ~0ull, gnext = 0;
         auto body = [&](uint64_t canon, uint32_t q) {
-            if (GC) {
-                const uint64_t wi = p0 + q;
-                if (gt == ~0ull) {
-                    const uint64_t lt = (wi - origin) / H.gtile;
-                    gt = tbase + lt;
-                    gnext = origin + (lt + 1) * H.gtile;
-                }
-                while (wi >= gnext) {
-                    gt++;
-                    gnext += H.gtile;
-                }
-                const uint32_t d = (uint32_t)(canon >> H.gshift) & 0xFF;
-                if (gt - g_lo < (uint64_t)kGenCntTiles) atomicAdd(&s_gc[gt - g_lo][d >> 1], 1u << (16 * (d & 1)));
-                else atomicAdd(&H.gcnt[gt * kSortRadix + d], 1u);
+            const uint64_t wi = p0 + q;
+            if (gt == ~0ull) {
+                const uint64_t lt = (wi - origin) / H.gtile;
+                gt = tbase + lt;
+                gnext = origin + (lt + 1) * H.gtile;
             }
-            const uint32_t b = (uint32_t)(canon >> P.bshift);
-            const uint32_t d = b >> kHLowBits;
-            const uint32_t slot = atomicAdd(&s_dig[d], 1u);
-            if (PHASE == 1) H.items[s_out[d] + slot] = (uint16_t)(b & (kHLow - 1));
-            if (PHASE == 0) {  // digit counts of a later sort over every k-mer
+            while (wi >= gnext) {
+                gt++;
+                gnext += H.gtile;
+            }
+            const uint32_t d = (uint32_t)(canon >> H.gshift) & 0xFF;
+            if (gt - g_lo < (uint64_t)kGenCntTiles) atomicAdd(&s_gc[gt - g_lo][d >> 1], 1u << (16 * (d & 1)));
+            else atomicAdd(&H.gcnt[gt * kSortRadix + d], 1u);
 #pragma unroll
-                for (int y = 0; y < 8; y++)
-                    if ((H.bmask >> (y + 1)) & 1) atomicAdd(&s_bh[y][H.kl.digit(canon, y)], 1u);
-            }
+            for (int y = 0; y < 8; y++)
+                if ((H.bmask >> (y + 1)) & 1) atomicAdd(&s_bh[y][H.kl.digit(canon, y)], 1u);
         };
         // the words from LDS or from memory in two copies of the loop: one
         // accessor choosing at run time reads both through flat loads, whose
@@ -203,34 +381,31 @@ __global__ __launch_bounds__(kKBlock) void hist_tile_kernel(KParams P, HParams H
                 [&](uint64_t w) -> uint64_t { return P.packed[w]; }, body);
         }
     }
-    if (PHASE == 0) {
-        __syncthreads();
-        if (tid < kHDigits) H.tcnt[mbase + (uint64_t)tid * Tc] = s_dig[tid];
-        unsigned long long *bh = H.bh + (uint64_t)(H.per_chunk ? c : t % kBhRep) * 8 * kSortRadix;
-        for (int j = tid; j < 8 * kSortRadix; j += kKBlock) {
-            const uint32_t v = (&s_bh[0][0])[j];
-            if (v) atomicAdd(&bh[j], (unsigned long long)v);
-        }
-        if (GC && w_hi > w_lo) {
-            // a tile whose windows all lie in this tile's is written; one shared
-            // with a neighbour (the first and last) is added to
-            const uint64_t g_hi = tbase + (w_hi - 1 - origin) / H.gtile;
-            const uint64_t ng = min(g_hi - g_lo + 1, (uint64_t)kGenCntTiles);
-            for (uint64_t j = tid; j < ng * kSortRadix; j += kKBlock) {
-                const uint64_t g = g_lo + j / kSortRadix;
-                const uint32_t dd = (uint32_t)(j % kSortRadix);
-                const uint32_t v = (s_gc[j / kSortRadix][dd >> 1] >> (16 * (dd & 1))) & 0xFFFFu;
-                const uint64_t gw0 = origin + (g - tbase) * H.gtile, gw1 = min(gw0 + H.gtile, cend);
-                const bool owned = gw0 >= w_lo && gw1 <= w_hi;
-                if (owned) H.gcnt[g * kSortRadix + (j % kSortRadix)] = v;
-                else if (v) atomicAdd(&H.gcnt[g * kSortRadix + (j % kSortRadix)], v);
-            }
+    __syncthreads();
+    unsigned long long *bh = H.bh + (uint64_t)c * 8 * kSortRadix;
+    for (int j = tid; j < 8 * kSortRadix; j += kKBlock) {
+        const uint32_t v = (&s_bh[0][0])[j];
+        if (v) atomicAdd(&bh[j], (unsigned long long)v);
+    }
+    if (w_hi > w_lo) {
+        // a tile whose windows all lie in this tile's is written; one shared
+        // with a neighbour (the first and last) is added to
+        const uint64_t g_hi = tbase + (w_hi - 1 - origin) / H.gtile;
+        const uint64_t ng = min(g_hi - g_lo + 1, (uint64_t)kGenCntTiles);
+        for (uint64_t j = tid; j < ng * kSortRadix; j += kKBlock) {
+            const uint64_t g = g_lo + j / kSortRadix;
+            const uint32_t dd = (uint32_t)(j % kSortRadix);
+            const uint32_t v = (s_gc[j / kSortRadix][dd >> 1] >> (16 * (dd & 1))) & 0xFFFFu;
+            const uint64_t gw0 = origin + (g - tbase) * H.gtile, gw1 = min(gw0 + H.gtile, cend);
+            const bool owned = gw0 >= w_lo && gw1 <= w_hi;
+            if (owned) H.gcnt[g * kSortRadix + (j % kSortRadix)] = v;
+            else if (v) atomicAdd(&H.gcnt[g * kSortRadix + (j % kSortRadix)], v);
         }
     }
 }
 
 // start of every (chunk, digit) partition, and the end of the last
-__global__ void hist_bounds_kernel(HParams H, uint64_t *__restrict__ bounds)
+__global__ void hist_bounds_kernel(HistParams H, uint64_t *__restrict__ bounds)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i > H.C * kHDigits) return;
@@ -240,7 +415,7 @@ __global__ void hist_bounds_kernel(HParams H, uint64_t *__restrict__ bounds)
     bounds[i] = H.toff[(uint64_t)kHDigits * H.tile0[c] + (uint64_t)d * Tc];
 }
 
-__global__ __launch_bounds__(1024) void hist_count_kernel(const uint16_t *__restrict__ items,
+__global__ __launch_bounds__(512) void hist_count_kernel(const uint16_t *__restrict__ items,
                                                           const HPiece *__restrict__ pieces,
                                                           uint32_t *__restrict__ counts)
 {
@@ -273,9 +448,6 @@ __global__ __launch_bounds__(1024) void hist_count_kernel(const uint16_t *__rest
     }
 }
 
-// seg: a batch (chunk = sample): only the first phase runs, for the byte
-// counts per sample (khist, C copies) and the generating pass's digit counts
-// over tiles of every sample's own windows (d_counts unused)
 __global__ void gather_u64_kernel(const uint64_t *__restrict__ src, const uint64_t *__restrict__ idx, uint64_t n,
                                   uint64_t *__restrict__ out)
 {
@@ -283,93 +455,43 @@ __global__ void gather_u64_kernel(const uint64_t *__restrict__ src, const uint64
     if (i < n) out[i] = src[idx[i]];
 }
 
-static int count_plain_partitioned(mp_ctx *ctx, KParams P, const uint64_t *chunk_first_id, int C, uint32_t *d_counts,
-                                   bool seg = false)
+static int count_plain_partitioned(mp_ctx *ctx, const KParams &K, const uint64_t *d_ids, int C, uint32_t *d_counts)
 {
-    std::vector<uint32_t> tile0(C + 1);
-    tile0[0] = 0;
-    for (int c = 0; c < C; c++) {
-        const uint64_t nr = chunk_first_id[c + 1] - chunk_first_id[c];
-        tile0[c + 1] = tile0[c] + (uint32_t)((nr + kHReads - 1) / kHReads);
-    }
-    const uint64_t NT = tile0[C];
-    if (NT == 0) return 0;
+    HistParams H{};
+    MP_TRY(read_starts(ctx));
+    H.packed = K.packed;
+    H.nmask = K.nmask;
+    H.rstart = (const uint64_t *)ctx->rstart.p;
+    H.nw64 = (ctx->total_bases + 63) / 64 + 2;
+    H.nw32 = 2 * H.nw64;
+    H.base_off = K.base_off;
+    H.total = ctx->total_bases;
+    H.K = K.K;
+    H.C = C;
+    H.chunk_ids = d_ids;
+    // about 8192 tiles at the most; the fixed scratch of the allocation-free
+    // entry point takes larger ones, for smaller tables
+    const uint64_t want = ctx->arena ? 128 : 8192;
+    H.tile = kHPos * std::max<uint64_t>(1, (H.total + kHPos * want - 1) / (kHPos * want));
+    const uint64_t NT = H.total / H.tile + 2 * (uint64_t)C + 1;  // at the most: the tile table is made on the device
     const uint64_t M = (uint64_t)kHDigits * NT;
     const uint64_t nparts = (uint64_t)C * kHDigits;
-    // hpart: chunk ids (C+1 u64) | tile0 (C+1 u32, padded) | bounds (nparts+1 u64) | tile counts (M u32)
-    const uint64_t o_ids = 0, o_t0 = o_ids + 8 * (C + 1), o_bd = o_t0 + 8 * ((C + 2) / 2),
-                   o_tc = o_bd + 8 * (nparts + 1), bytes = o_tc + 4 * M + 64;
+    // hpart: tile0 (C+1 u32, padded) | bounds (nparts+1 u64) | tile counts (M u32)
+    const uint64_t o_bd = 8 * (((uint64_t)C + 2) / 2), o_tc = o_bd + 8 * (nparts + 1), bytes = o_tc + 4 * M + 64;
     MP_TRY(ensure(ctx, ctx->hpart, bytes));
     MP_TRY(ensure(ctx, ctx->wg_off, (M + 1) * sizeof(uint64_t)));
     uint8_t *hb = (uint8_t *)ctx->hpart.p;
-    HParams H{};
-    const uint64_t ncopies = seg ? (uint64_t)C : (uint64_t)kBhRep;
-    MP_TRY(ensure(ctx, ctx->khist, sizeof(uint64_t) * ncopies * 8 * kSortRadix));
-    MP_TRY(fill_u32(ctx, ctx->khist.p, 0, 2 * ncopies * 8 * kSortRadix));
-    H.bh = (unsigned long long *)ctx->khist.p;
-    H.bmask = scan_pass_mask(ctx->cfg.k) & 0x1FEu;
-    H.kl = scan_layout(ctx);
-    H.per_chunk = seg ? 1 : 0;
-    ctx->khist_copies = (int)ncopies;
-    // digit counts per generating-pass tile of the lowest sorted byte, for a
-    // batch sorted sample by sample (its generating pass then takes counted
-    // offsets).  A plain run does not count them: at 2.4e9 windows the
-    // counted generating pass measured equal to the look-back one (27.9 ms),
-    // and counting them cost the histogram about 4 ms (LDS for 24 tiles).
-    ctx->gcnt_valid = false;
-    ctx->gcnt_seg = seg;
-    if (H.bmask && !ctx->arena && seg) {
-        const uint64_t gtile = sort_tile_items(ctx);
-        if (gtile >= (1u << 16)) return ctx->fail(MP_EINVAL, "radix tile of %llu windows: counts need 16 bits",
-                                                 (unsigned long long)gtile);
-        uint64_t npos = 0;
-        MP_HIP(hipMemcpyAsync(&npos, (const uint64_t *)ctx->pos_off.p + ctx->N, sizeof(uint64_t),
-                              hipMemcpyDeviceToHost, ctx->stream));
-        MP_HIP(hipStreamSynchronize(ctx->stream));
-        uint64_t gtiles = (npos + gtile - 1) / gtile;
-        if (seg) {  // every sample's windows in tiles of their own
-            ctx->seg_wpos.assign(C + 1, 0);
-            MP_TRY(ensure(ctx, ctx->segtab, 3 * (uint64_t)(C + 1) * sizeof(uint64_t)));
-            uint64_t *d_w = (uint64_t *)ctx->segtab.p, *d_ids = d_w + 2 * (C + 1);
-            MP_HIP(hipMemcpyAsync(d_ids, chunk_first_id, (C + 1) * sizeof(uint64_t), hipMemcpyHostToDevice,
-                                  ctx->stream));
-            hipLaunchKernelGGL(gather_u64_kernel, dim3((C + 256) / 256), dim3(256), 0, ctx->stream,
-                               (const uint64_t *)ctx->pos_off.p, (const uint64_t *)d_ids, (uint64_t)(C + 1),
-                               d_w + (C + 1));
-            MP_HIP(hipGetLastError());
-            MP_HIP(hipMemcpyAsync(ctx->seg_wpos.data(), d_w + (C + 1), (C + 1) * sizeof(uint64_t),
-                                  hipMemcpyDeviceToHost, ctx->stream));
-            MP_HIP(hipStreamSynchronize(ctx->stream));
-            std::vector<uint64_t> gft(C + 1, 0);
-            for (int c = 0; c < C; c++)
-                gft[c + 1] = gft[c] + (ctx->seg_wpos[c + 1] - ctx->seg_wpos[c] + gtile - 1) / gtile;
-            gtiles = gft[C];
-            MP_HIP(hipMemcpyAsync(d_w, gft.data(), (C + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
-            H.gft = d_w;
-            H.gw = d_w + (C + 1);
-            MP_HIP(hipStreamSynchronize(ctx->stream));  // gft is read by the copy above
-        }
-        if (gtiles) {
-            MP_TRY(ensure(ctx, ctx->gcnt, gtiles * kSortRadix * sizeof(uint32_t)));
-            MP_TRY(fill_u32(ctx, ctx->gcnt.p, 0, gtiles * kSortRadix));
-            H.gcnt = (uint32_t *)ctx->gcnt.p;
-            H.gtile = gtile;
-            H.gshift = H.kl.shift[__builtin_ctz(H.bmask) - 1];  // the generating pass's digit: a whole byte
-            ctx->gcnt_tile = gtile;
-            ctx->gcnt_tiles = gtiles;
-            ctx->gcnt_byte = __builtin_ctz(H.bmask) - 1;
-        }
-    }
-    H.chunk_ids = (const uint64_t *)(hb + o_ids);
-    H.tile0 = (const uint32_t *)(hb + o_t0);
-    H.C = C;
+    uint32_t *d_tile0 = (uint32_t *)hb;
+    uint64_t *d_bounds = (uint64_t *)(hb + o_bd);
+    H.tile0 = d_tile0;
     H.tcnt = (uint32_t *)(hb + o_tc);
     H.toff = (const uint64_t *)ctx->wg_off.p;
-    uint64_t *d_bounds = (uint64_t *)(hb + o_bd);
-    MP_HIP(hipMemcpyAsync(hb + o_ids, chunk_first_id, 8 * (C + 1), hipMemcpyHostToDevice, ctx->stream));
-    MP_HIP(hipMemcpyAsync(hb + o_t0, tile0.data(), 4 * (C + 1), hipMemcpyHostToDevice, ctx->stream));
-    if (H.gcnt) hipLaunchKernelGGL((hist_tile_kernel<0, true>), dim3((unsigned)NT), dim3(kKBlock), 0, ctx->stream, P, H);
-    else hipLaunchKernelGGL((hist_tile_kernel<0, false>), dim3((unsigned)NT), dim3(kKBlock), 0, ctx->stream, P, H);
+    ctx->khist_valid = false;  // a radix sort of these reads counts its own digits
+    ctx->gcnt_valid = false;
+    ctx->kmer_total = 0;
+    if (H.total == 0) return 0;
+    hipLaunchKernelGGL(hist_tiles_kernel, dim3(1), dim3(256), 0, ctx->stream, H, d_tile0);
+    hipLaunchKernelGGL(hist_pos_kernel<0>, dim3((unsigned)NT), dim3(kHLanes), 0, ctx->stream, H);
     MP_HIP(hipGetLastError());
     MP_TRY(scan_u32(ctx, H.tcnt, (uint64_t *)ctx->wg_off.p, M));
     hipLaunchKernelGGL(hist_bounds_kernel, dim3((unsigned)((nparts + 256) / 256)), dim3(256), 0, ctx->stream, H,
@@ -379,16 +501,12 @@ static int count_plain_partitioned(mp_ctx *ctx, KParams P, const uint64_t *chunk
     MP_HIP(hipMemcpyAsync(bounds.data(), d_bounds, 8 * (nparts + 1), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
     const uint64_t total = bounds[nparts];
-    ctx->khist_mask = H.bmask;
-    ctx->khist_valid = true;
-    ctx->gcnt_valid = H.gcnt != nullptr;
-    if (seg) return 0;  // a batch's counts: nothing more
     ctx->kmer_total = total;
     if (total == 0) return 0;
     // the low bits stage in the second tuple buffer, unused until the first scan's sort
     MP_TRY(ensure(ctx, ctx->keys[1], total * sizeof(uint16_t) + 64));
     H.items = (uint16_t *)ctx->keys[1].p;
-    hipLaunchKernelGGL(hist_tile_kernel<1>, dim3((unsigned)NT), dim3(kKBlock), 0, ctx->stream, P, H);
+    hipLaunchKernelGGL(hist_pos_kernel<1>, dim3((unsigned)NT), dim3(kHLanes), 0, ctx->stream, H);
     MP_HIP(hipGetLastError());
     std::vector<HPiece> pieces;
     for (uint64_t p = 0; p < nparts; p++) {
@@ -402,12 +520,82 @@ static int count_plain_partitioned(mp_ctx *ctx, KParams P, const uint64_t *chunk
     MP_TRY(tmp_alloc(ctx, (void **)&d_pieces, pieces.size() * sizeof(HPiece)));
     MP_HIP(hipMemcpyAsync(d_pieces, pieces.data(), pieces.size() * sizeof(HPiece), hipMemcpyHostToDevice,
                           ctx->stream));
-    hipLaunchKernelGGL(hist_count_kernel, dim3((unsigned)pieces.size()), dim3(1024), 0, ctx->stream,
+    hipLaunchKernelGGL(hist_count_kernel, dim3((unsigned)pieces.size()), dim3(512), 0, ctx->stream,
                        (const uint16_t *)H.items, (const HPiece *)d_pieces, d_counts);
     MP_HIP(hipGetLastError());
     MP_TRY(tmp_free(ctx, d_pieces));
     // the host vectors above must outlive the copies
     MP_HIP(hipStreamSynchronize(ctx->stream));
+    return 0;
+}
+
+// The batch's digit counts for a segmented radix sort (batch_count_kernel):
+// khist per sample, gcnt per tile of every sample's windows.
+static int count_batch_digits(mp_ctx *ctx, KParams P, const uint64_t *chunk_first_id, int C)
+{
+    std::vector<uint32_t> tile0(C + 1);
+    tile0[0] = 0;
+    for (int c = 0; c < C; c++) {
+        const uint64_t nr = chunk_first_id[c + 1] - chunk_first_id[c];
+        tile0[c + 1] = tile0[c] + (uint32_t)((nr + kBReads - 1) / kBReads);
+    }
+    const uint64_t NT = tile0[C];
+    if (NT == 0) return 0;
+    // hpart: chunk ids (C+1 u64) | tile0 (C+1 u32, padded)
+    const uint64_t o_t0 = 8 * ((uint64_t)C + 1);
+    MP_TRY(ensure(ctx, ctx->hpart, o_t0 + 8 * (((uint64_t)C + 2) / 2) + 64));
+    uint8_t *hb = (uint8_t *)ctx->hpart.p;
+    HParams H{};
+    MP_TRY(ensure(ctx, ctx->khist, sizeof(uint64_t) * C * 8 * kSortRadix));
+    MP_TRY(fill_u32(ctx, ctx->khist.p, 0, 2 * (uint64_t)C * 8 * kSortRadix));
+    H.bh = (unsigned long long *)ctx->khist.p;
+    H.bmask = scan_pass_mask(ctx->cfg.k) & 0x1FEu;
+    H.kl = scan_layout(ctx);
+    ctx->khist_copies = C;
+    ctx->gcnt_seg = true;
+    ctx->gcnt_valid = false;
+    const uint64_t gtile = sort_tile_items(ctx);
+    if (gtile >= (1u << 16)) return ctx->fail(MP_EINVAL, "radix tile of %llu windows: counts need 16 bits",
+                                             (unsigned long long)gtile);
+    // every sample's windows in tiles of their own
+    ctx->seg_wpos.assign(C + 1, 0);
+    MP_TRY(ensure(ctx, ctx->segtab, 3 * (uint64_t)(C + 1) * sizeof(uint64_t)));
+    uint64_t *d_w = (uint64_t *)ctx->segtab.p, *d_ids = d_w + 2 * (C + 1);
+    MP_HIP(hipMemcpyAsync(d_ids, chunk_first_id, (C + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(gather_u64_kernel, dim3((C + 256) / 256), dim3(256), 0, ctx->stream,
+                       (const uint64_t *)ctx->pos_off.p, (const uint64_t *)d_ids, (uint64_t)(C + 1), d_w + (C + 1));
+    MP_HIP(hipGetLastError());
+    MP_HIP(hipMemcpyAsync(ctx->seg_wpos.data(), d_w + (C + 1), (C + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost,
+                          ctx->stream));
+    MP_HIP(hipStreamSynchronize(ctx->stream));
+    std::vector<uint64_t> gft(C + 1, 0);
+    for (int c = 0; c < C; c++)
+        gft[c + 1] = gft[c] + (ctx->seg_wpos[c + 1] - ctx->seg_wpos[c] + gtile - 1) / gtile;
+    const uint64_t gtiles = gft[C];
+    MP_HIP(hipMemcpyAsync(d_w, gft.data(), (C + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
+    H.gft = d_w;
+    H.gw = d_w + (C + 1);
+    ctx->khist_mask = H.bmask;
+    if (gtiles) {
+        MP_TRY(ensure(ctx, ctx->gcnt, gtiles * kSortRadix * sizeof(uint32_t)));
+        MP_TRY(fill_u32(ctx, ctx->gcnt.p, 0, gtiles * kSortRadix));
+        H.gcnt = (uint32_t *)ctx->gcnt.p;
+        H.gtile = gtile;
+        H.gshift = H.kl.shift[__builtin_ctz(H.bmask) - 1];  // the generating pass's digit: a whole byte
+        ctx->gcnt_tile = gtile;
+        ctx->gcnt_tiles = gtiles;
+        ctx->gcnt_byte = __builtin_ctz(H.bmask) - 1;
+        H.chunk_ids = (const uint64_t *)hb;
+        H.tile0 = (const uint32_t *)(hb + o_t0);
+        H.C = C;
+        MP_HIP(hipMemcpyAsync(hb, chunk_first_id, 8 * (C + 1), hipMemcpyHostToDevice, ctx->stream));
+        MP_HIP(hipMemcpyAsync(hb + o_t0, tile0.data(), 4 * (C + 1), hipMemcpyHostToDevice, ctx->stream));
+        hipLaunchKernelGGL(batch_count_kernel, dim3((unsigned)NT), dim3(kKBlock), 0, ctx->stream, P, H);
+        MP_HIP(hipGetLastError());
+    }
+    MP_HIP(hipStreamSynchronize(ctx->stream));  // gft and tile0 are read by the copies above
+    ctx->khist_valid = true;
+    ctx->gcnt_valid = H.gcnt != nullptr;
     return 0;
 }
 
@@ -633,7 +821,7 @@ int batch_counts(mp_ctx *ctx)
 {
     KParams P = base_params(ctx);
     P.C = ctx->C;
-    return count_plain_partitioned(ctx, P, ctx->chunk_ids.data(), ctx->C, nullptr, true);
+    return count_batch_digits(ctx, P, ctx->chunk_ids.data(), ctx->C);
 }
 
 int count_chunks_device(mp_ctx *ctx, const uint64_t *chunk_first_id, int C, uint32_t *d_counts)
@@ -651,7 +839,7 @@ int count_chunks_device(mp_ctx *ctx, const uint64_t *chunk_first_id, int C, uint
                            dim3(kKBlock), 0, ctx->stream, P);
         MP_HIP(hipGetLastError());
     } else {
-        MP_TRY(count_plain_partitioned(ctx, P, chunk_first_id, C, d_counts));
+        MP_TRY(count_plain_partitioned(ctx, P, d_ids, C, d_counts));
     }
     MP_TRY(tmp_free(ctx, d_ids));
     return 0;

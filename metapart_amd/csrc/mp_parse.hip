@@ -193,6 +193,32 @@ __global__ void chunk_ids_kernel(const uint64_t *__restrict__ rec_off, uint64_t 
     if (rec_off[lo] != target) atomicMin(first_bad, (unsigned long long)(1ull << 62) + (unsigned long long)c);
 }
 
+// read starts as bits, and one at the end of the last read (the array is zero before)
+__global__ void read_start_kernel(const uint64_t *__restrict__ base_off, uint64_t N, uint32_t *__restrict__ bits)
+{
+    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r > N) return;
+    const uint64_t b = base_off[r];
+    atomicOr(&bits[2 * (b >> 6) + 1 - ((b >> 5) & 1)], 0x80000000u >> (b & 31));
+}
+
+int read_starts(mp_ctx *ctx)
+{
+    if (ctx->rstart_valid) return 0;
+    const uint64_t N = ctx->N, words = (ctx->total_bases + 63) / 64 + 2, bytes = words * sizeof(uint64_t);
+    if (ctx->arena && ctx->keys[0].bytes >= bytes) {
+        ctx->rstart = ctx->keys[0];  // idle once the reads are parsed, and no scan follows: the fixed scratch holds no more than without
+    } else {
+        MP_TRY(ensure(ctx, ctx->rstart, bytes));
+    }
+    MP_TRY(fill_u32(ctx, ctx->rstart.p, 0, 2 * words));
+    hipLaunchKernelGGL(read_start_kernel, dim3((unsigned)((N + 256) / 256)), dim3(256), 0, ctx->stream,
+                       (const uint64_t *)ctx->base_off.p, N, (uint32_t *)ctx->rstart.p);
+    MP_HIP(hipGetLastError());
+    ctx->rstart_valid = true;
+    return 0;
+}
+
 int parse_reads(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *chunk_first_id, int C)
 {
     const uint64_t nbytes = ctx->fq_bytes;
