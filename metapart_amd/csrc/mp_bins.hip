@@ -52,6 +52,7 @@ constexpr uint32_t kBinCap = 4096;  // windows of a bin that bin_runs takes; its
 constexpr uint32_t kBinRec = 640;   // records of such a bin
 constexpr uint32_t kBinAim = kBinCap * 3 / 4;  // windows per bin aimed at, at most (fewer where records hold few)
 constexpr int kRunThreads = 1024;
+constexpr uint64_t kRunGrid = 1ull << 21;  // bins of a dispatch of bin_runs: fewer than 2^32 threads
 constexpr int kBinWit = 8;          // witnesses per bin (bin_runs)
 constexpr int kMaxSeg = 256;        // segments (samples of a batch)
 constexpr int kStripes = 64;        // copies of the global counters, a cache line each
@@ -61,6 +62,7 @@ struct BinRec {  // a super-k-mer: consecutive windows of one read with one mini
     uint32_t label;
     uint32_t pad;
 };
+static_assert(kRunGrid * kRunThreads < (1ull << 32), "one dispatch");
 static_assert(sizeof(BinRec) == 16, "one 16-byte access");
 constexpr uint32_t kPrevN = 1, kNextN = 2;  // flags: no base before the first / after the last window ('N' class)
 
@@ -1617,13 +1619,17 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     // every k-mer is in the scan when the histogram sized it so; a k-mer outside it all the same sets kErrRange
     const bool n_part = !batch && !(lo == 0 && (hi == MP_NBUCKETS || job.expected == nv));
     auto runs = [&](bool check) -> int {
-        R.bins = d_bins;
-        R.nbin = (uint32_t)nbin;
-        R.wit = d_wit;
-        const dim3 gs((unsigned)nbin), ts(kRunThreads);
-        if (nbin && check) hipLaunchKernelGGL((bin_runs_kernel<true, true>), gs, ts, 0, ctx->stream, R);
-        if (nbin && !check && n_part) hipLaunchKernelGGL((bin_runs_kernel<false, true>), gs, ts, 0, ctx->stream, R);
-        if (nbin && !check && !n_part) hipLaunchKernelGGL((bin_runs_kernel<false, false>), gs, ts, 0, ctx->stream, R);
+        // a dispatch holds fewer than 2^32 threads, so past 4 M bins (some 6e9 windows) there are several
+        for (uint64_t b0 = 0; b0 < nbin; b0 += kRunGrid) {
+            R.bins = d_bins + b0;
+            R.nbin = (uint32_t)std::min(kRunGrid, nbin - b0);
+            R.wit = d_wit + b0 * kBinWit;
+            const dim3 gs(R.nbin), ts(kRunThreads);
+            if (check) hipLaunchKernelGGL((bin_runs_kernel<true, true>), gs, ts, 0, ctx->stream, R);
+            else if (n_part) hipLaunchKernelGGL((bin_runs_kernel<false, true>), gs, ts, 0, ctx->stream, R);
+            else hipLaunchKernelGGL((bin_runs_kernel<false, false>), gs, ts, 0, ctx->stream, R);
+            MP_HIP(hipGetLastError());
+        }
         R.bins = d_big;
         R.nbin = (uint32_t)nbig;
         R.wit = d_wit + nbin * kBinWit;
