@@ -114,46 +114,6 @@ static int load_common(mp_ctx *ctx, const uint64_t *chunk_ofs, const uint64_t *c
     return 0;
 }
 
-// Host to device copy of FASTQ bytes.  Large inputs go through two pinned
-// staging buffers: host threads fill one while the DMA engine drains the
-// other, so pageable memory is read once at memory speed and PCIe runs at the
-// pinned rate.
-constexpr int kStageThreads = 8;
-
-static void parallel_copy(char *dst, const char *src, uint64_t n)
-{
-    std::vector<std::thread> th;
-    const uint64_t part = (n + kStageThreads - 1) / kStageThreads;
-    for (int t = 0; t < kStageThreads; t++) {
-        const uint64_t a = t * part, b = std::min(n, a + part);
-        if (a >= b) break;
-        th.emplace_back([=] { memcpy(dst + a, src + a, b - a); });
-    }
-    for (auto &x : th) x.join();
-}
-
-static int copy_to_device(mp_ctx *ctx, uint8_t *dst, const char *src, uint64_t nbytes)
-{
-    if (nbytes < 2 * kStageBytes) {
-        MP_HIP(hipMemcpyAsync(dst, src, nbytes, hipMemcpyHostToDevice, ctx->stream));
-        return 0;
-    }
-    for (int b = 0; b < 2; b++) {
-        if (!ctx->stage[b]) MP_HIP(hipHostMalloc(&ctx->stage[b], kStageBytes, hipHostMallocDefault));
-        if (!ctx->stage_ev[b]) MP_HIP(hipEventCreateWithFlags(&ctx->stage_ev[b], hipEventDisableTiming));
-    }
-    for (uint64_t off = 0, c = 0; off < nbytes; off += kStageBytes, c++) {
-        const int b = (int)(c & 1);
-        const uint64_t len = std::min(kStageBytes, nbytes - off);
-        if (ctx->stage_used[b]) MP_HIP(hipEventSynchronize(ctx->stage_ev[b]));  // its previous copy has left
-        parallel_copy((char *)ctx->stage[b], src + off, len);
-        MP_HIP(hipMemcpyAsync(dst + off, ctx->stage[b], len, hipMemcpyHostToDevice, ctx->stream));
-        MP_HIP(hipEventRecord(ctx->stage_ev[b], ctx->stream));
-        ctx->stage_used[b] = true;
-    }
-    return 0;
-}
-
 static int upload_fq(mp_ctx *ctx, const char *fq, uint64_t nbytes)
 {
     MP_TRY(ensure(ctx, ctx->fq, nbytes + 64));
@@ -176,8 +136,7 @@ int mp_count_chunks(mp_ctx *ctx, const char *fq, uint64_t nbytes, const uint64_t
     MP_TRY(ensure(ctx, ctx->scratch, words * sizeof(uint32_t) + 4096));
     uint32_t *d_counts = (uint32_t *)ctx->scratch.p;
     MP_TRY(count_chunks_device(ctx, ctx->chunk_ids.data(), C, d_counts));
-    MP_HIP(hipMemcpyAsync(counts, d_counts, words * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    MP_HIP(hipStreamSynchronize(ctx->stream));
+    MP_TRY(copy_to_host(ctx, counts, d_counts, words * sizeof(uint32_t)));
     uint64_t tot = 0;
     for (uint64_t i = 0; i < words; i++) tot += counts[i];
     if (total_kmers) *total_kmers = tot;
@@ -199,12 +158,10 @@ int mp_count_loaded(mp_ctx *ctx, uint32_t *counts, uint64_t *hist, uint64_t *rea
     MP_TRY(count_chunks_device(ctx, ctx->chunk_ids.data(), C, d_counts));
     uint64_t *d_tot = (uint64_t *)ctx->hist.p, *d_pre = d_tot + MP_NBUCKETS;
     MP_TRY(bucket_totals(ctx, d_counts, C, d_tot));
-    if (counts) MP_HIP(hipMemcpyAsync(counts, d_counts, words * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     MP_TRY(scan_u64(ctx, d_tot, d_pre, MP_NBUCKETS));
-    // straight into the caller's buffers
+    if (counts) MP_TRY(copy_to_host(ctx, counts, d_counts, words * sizeof(uint32_t)));
     uint64_t total = 0;
-    if (hist)
-        MP_HIP(hipMemcpyAsync(hist, d_pre, sizeof(uint64_t) * (MP_NBUCKETS + 1), hipMemcpyDeviceToHost, ctx->stream));
+    if (hist) MP_TRY(copy_to_host(ctx, hist, d_pre, sizeof(uint64_t) * (MP_NBUCKETS + 1)));
     MP_HIP(hipMemcpyAsync(&total, d_pre + MP_NBUCKETS, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
     if (total_kmers) *total_kmers = total;
@@ -465,11 +422,7 @@ int mp_get_parent(mp_ctx *ctx, uint64_t *parent)
     if (!ctx || !parent) return MP_EINVAL;
     if (ctx->N == 0) return ctx->fail(MP_ESTATE, "no reads loaded");
     MP_HIP(hipSetDevice(ctx->device));
-    std::vector<uint32_t> p(ctx->N);
-    MP_HIP(hipMemcpyAsync(p.data(), ctx->parent.p, ctx->N * 4, hipMemcpyDeviceToHost, ctx->stream));
-    MP_HIP(hipStreamSynchronize(ctx->stream));
-    for (uint64_t i = 0; i < ctx->N; i++) parent[i] = p[i];
-    return 0;
+    return labels_to_host(ctx, parent, (const uint32_t *)ctx->parent.p, ctx->N);
 }
 
 int mp_get_bad(mp_ctx *ctx, uint8_t *bad)

@@ -180,32 +180,37 @@ extern "C" int mp_index_buffer(const char *buf, uint64_t nbytes, int num_chunks,
 
 // metapart.c:3720-3791 with one MPI rank: the process ranges equal the scan
 // ranges (same thresholds), so only the scan and thread walks remain.  Each
-// walk moves at most one boundary per bucket, and the thread walk copies the
-// scan boundary at every multiple of T.
+// moves at most one boundary per bucket, so both go in one pass over the 8 MB
+// table (it is what the walks cost: 0.4 ms each).  The thread walk takes the
+// scan boundary at every multiple of T, filled in once the scan's are known.
 extern "C" int mp_plan_ranges(const uint64_t *H, int S, int T, uint64_t *scan, uint64_t *thread)
 {
     if (!H || !scan || !thread || S <= 0 || T <= 0) return MP_EINVAL;
     const uint64_t tot = H[MP_NBUCKETS];
-    uint64_t avgS = tot / (uint64_t)S + (tot % (uint64_t)S ? 1 : 0);
-    memset(scan, 0, sizeof(uint64_t) * (size_t)(S + 1));
-    int r = 1;
-    uint32_t i;
-    for (i = 0; i < MP_NBUCKETS; i++)
-        if (H[i] >= avgS * (uint64_t)r) {
-            if (r > S) return MP_EPLAN;
-            scan[r++] = i;
-        }
-    if (r == S) scan[r] = i;
+    const uint64_t avgS = tot / (uint64_t)S + (tot % (uint64_t)S ? 1 : 0);
     const uint64_t avgT = avgS / (uint64_t)T;
+    memset(scan, 0, sizeof(uint64_t) * (size_t)(S + 1));
     memset(thread, 0, sizeof(uint64_t) * (size_t)(S * T + 1));
-    r = 1;
-    for (i = 0; i < MP_NBUCKETS; i++)
-        if (H[i] >= (uint64_t)r * avgT) {
-            if (r > S * T) return MP_EPLAN;
-            thread[r] = (r % T == 0) ? scan[r / T] : i;
-            r++;
+    int rs = 1, rt = 1;
+    uint64_t ths = avgS, tht = avgT;
+    for (uint32_t i = 0; i < MP_NBUCKETS; i++) {
+        const uint64_t lo = std::min(ths, tht);
+        while (i < MP_NBUCKETS && H[i] < lo) i++;
+        if (i == MP_NBUCKETS) break;
+        if (H[i] >= ths) {
+            if (rs > S) return MP_EPLAN;
+            scan[rs++] = i;
+            ths = avgS * (uint64_t)rs;
         }
-    if (r == S * T) thread[r] = i;
+        if (H[i] >= tht) {
+            if (rt > S * T) return MP_EPLAN;
+            thread[rt++] = i;
+            tht = avgT * (uint64_t)rt;
+        }
+    }
+    if (rs == S) scan[rs] = MP_NBUCKETS;
+    for (int r = T; r < rt; r += T) thread[r] = scan[r / T];
+    if (rt == S * T) thread[rt] = MP_NBUCKETS;
     for (int q = 0; q < S * T; q++)
         if (!(thread[q] < thread[q + 1])) return MP_EPLAN;
     return 0;

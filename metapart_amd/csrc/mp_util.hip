@@ -1,5 +1,10 @@
 // Device memory accounting, fills and a single-pass (decoupled look-back)
 // exclusive scan used for record, k-mer and output offsets.
+#include <algorithm>
+#include <cstring>
+#include <thread>
+#include <vector>
+
 #include "mp_internal.h"
 
 namespace mp {
@@ -203,5 +208,125 @@ static int scan_impl(mp_ctx *ctx, const T *in, uint64_t *out, uint64_t n)
 
 int scan_u32(mp_ctx *ctx, const uint32_t *in, uint64_t *out, uint64_t n) { return scan_impl(ctx, in, out, n); }
 int scan_u64(mp_ctx *ctx, const uint64_t *in, uint64_t *out, uint64_t n) { return scan_impl(ctx, in, out, n); }
+
+// ---------------------------------------------------------------- host copies
+// The runtime moves pageable memory at 27 GB/s up, and a first touch of fresh
+// pages inside its copy down costs far more than the copy.  Through two pinned
+// 8 MB buffers of the ctx (0.6 ms to pin, once) the link runs at its rate
+// while host threads move the other buffer's bytes, page faults among them:
+// 167 MB up 6.3 -> 3.6 ms, 12 M labels widened into fresh memory 12-18 -> 4.5,
+// 67 MB of counts down 17 -> 7.  Each line below lies where the gain on a
+// ctx's first call pays for the pinning (16 MB up 0.60 -> 0.52 and 8 MB down
+// do not).
+constexpr uint64_t kStagedUp = 32ull << 20, kStagedDown = 16ull << 20, kStagedLabels = 1ull << 20;
+
+static int stage_buffers(mp_ctx *ctx)
+{
+    for (int b = 0; b < 2; b++) {
+        if (!ctx->stage[b]) MP_HIP(hipHostMalloc(&ctx->stage[b], kStageBytes, hipHostMallocDefault));
+        if (!ctx->stage_ev[b]) MP_HIP(hipEventCreateWithFlags(&ctx->stage_ev[b], hipEventDisableTiming));
+    }
+    return 0;
+}
+
+// f(a, b) over [0, n) on up to `threads` host threads, the caller among them;
+// parts whose thread cannot be started run here
+template <typename F> static void host_parallel(unsigned threads, uint64_t n, F f)
+{
+    const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
+    const uint64_t T = std::max<uint64_t>(1, std::min<uint64_t>({threads, hw, n >> 16}));  // 64 K items a thread at the least
+    const uint64_t part = (n + T - 1) / T;
+    std::vector<std::thread> th;
+    uint64_t next = part;
+    try {
+        th.reserve(T);
+        for (; next < n; next += part) th.emplace_back(f, next, std::min(n, next + part));
+    } catch (const std::exception &) {
+    }
+    f(0, std::min(n, part));
+    for (; next < n; next += part) f(next, std::min(n, next + part));
+    for (auto &x : th) x.join();
+}
+
+int copy_to_device(mp_ctx *ctx, uint8_t *dst, const char *src, uint64_t nbytes)
+{
+    if (nbytes < kStagedUp) {
+        MP_HIP(hipMemcpyAsync(dst, src, nbytes, hipMemcpyHostToDevice, ctx->stream));
+        return 0;
+    }
+    MP_TRY(stage_buffers(ctx));
+    for (uint64_t off = 0, c = 0; off < nbytes; off += kStageBytes, c++) {
+        const int b = (int)(c & 1);
+        const uint64_t len = std::min(kStageBytes, nbytes - off);
+        if (ctx->stage_used[b]) MP_HIP(hipEventSynchronize(ctx->stage_ev[b]));  // its previous copy has left
+        char *const to = (char *)ctx->stage[b];
+        host_parallel(4, len, [=](uint64_t x, uint64_t y) { memcpy(to + x, src + off + x, y - x); });
+        MP_HIP(hipMemcpyAsync(dst + off, to, len, hipMemcpyHostToDevice, ctx->stream));
+        MP_HIP(hipEventRecord(ctx->stage_ev[b], ctx->stream));
+        ctx->stage_used[b] = true;
+    }
+    return 0;
+}
+
+int stream_to_host(mp_ctx *ctx, const void *src, uint64_t nbytes, const std::function<int(const char *, uint64_t)> &sink)
+{
+    MP_TRY(stage_buffers(ctx));
+    for (int b = 0; b < 2; b++)  // an upload that is still reading them
+        if (ctx->stage_used[b]) MP_HIP(hipEventSynchronize(ctx->stage_ev[b]));
+    // four pieces at the least, so that a small copy overlaps its host side too
+    const uint64_t piece = std::min(kStageBytes, std::max<uint64_t>(1u << 20, (nbytes / 4 + 4095) & ~4095ull));
+    auto issue = [&](uint64_t c) -> int {
+        const uint64_t off = c * piece;
+        MP_HIP(hipMemcpyAsync(ctx->stage[c & 1], (const char *)src + off, std::min(piece, nbytes - off), hipMemcpyDeviceToHost,
+                              ctx->stream));
+        MP_HIP(hipEventRecord(ctx->stage_ev[c & 1], ctx->stream));
+        return 0;
+    };
+    const uint64_t n = (nbytes + piece - 1) / piece;
+    int rc = n ? issue(0) : 0;
+    for (uint64_t c = 0; c < n && !rc; c++) {
+        if (c + 1 < n) rc = issue(c + 1);
+        if (rc) break;
+        MP_HIP(hipEventSynchronize(ctx->stage_ev[c & 1]));
+        rc = sink((const char *)ctx->stage[c & 1], std::min(piece, nbytes - c * piece));
+    }
+    MP_HIP(hipStreamSynchronize(ctx->stream));  // nothing is left in flight into the buffers
+    return rc;
+}
+
+int copy_to_host(mp_ctx *ctx, void *dst, const void *src, uint64_t nbytes)
+{
+    if (ctx->arena || nbytes < kStagedDown) {  // the allocation-free entry point pins nothing
+        MP_HIP(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, ctx->stream));
+        MP_HIP(hipStreamSynchronize(ctx->stream));
+        return 0;
+    }
+    char *to = (char *)dst;
+    return stream_to_host(ctx, src, nbytes, [&](const char *p, uint64_t len) {
+        host_parallel(8, len, [=](uint64_t x, uint64_t y) { memcpy(to + x, p + x, y - x); });
+        to += len;
+        return 0;
+    });
+}
+
+int labels_to_host(mp_ctx *ctx, uint64_t *dst, const uint32_t *src, uint64_t n)
+{
+    if (n < kStagedLabels) {
+        std::vector<uint32_t> p(n);
+        MP_HIP(hipMemcpyAsync(p.data(), src, n * 4, hipMemcpyDeviceToHost, ctx->stream));
+        MP_HIP(hipStreamSynchronize(ctx->stream));
+        for (uint64_t i = 0; i < n; i++) dst[i] = p[i];
+        return 0;
+    }
+    return stream_to_host(ctx, src, n * 4, [&](const char *p, uint64_t len) {
+        const uint32_t *const q = (const uint32_t *)p;
+        uint64_t *const o = dst;
+        host_parallel(8, len / 4, [=](uint64_t x, uint64_t y) {
+            for (uint64_t i = x; i < y; i++) o[i] = q[i];
+        });
+        dst += len / 4;
+        return 0;
+    });
+}
 
 }  // namespace mp
