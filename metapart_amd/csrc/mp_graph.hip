@@ -877,15 +877,197 @@ __global__ void pair_graph_kernel(const uint32_t *__restrict__ parent, const uin
     if (j < P && pair_candidate(parent, sizes, j, a, b)) uf_union(gparent, a, b);
 }
 
-// 1 for a candidate pair inside a candidate-graph component of > 1000 reads
-__global__ void pair_classify_kernel(const uint32_t *__restrict__ parent, const uint32_t *__restrict__ sizes,
-                                     const uint32_t *__restrict__ gparent, const uint32_t *__restrict__ gsize,
-                                     uint32_t *__restrict__ ordered, uint64_t P)
+// 1 for a candidate pair inside a candidate-graph component of > 1000 reads;
+// st: those pairs, and the reads of the largest of those components
+__global__ __launch_bounds__(256) void pair_classify_kernel(const uint32_t *__restrict__ parent,
+                                                            const uint32_t *__restrict__ sizes,
+                                                            const uint32_t *__restrict__ gparent,
+                                                            const uint32_t *__restrict__ gsize,
+                                                            uint32_t *__restrict__ ordered, uint64_t P,
+                                                            unsigned long long *__restrict__ st)
+{
+    uint32_t cnt = 0, most = 0;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < P; j += stride) {
+        uint32_t a, b, o = 0;
+        if (pair_candidate(parent, sizes, j, a, b)) {
+            const uint32_t g = gsize[gparent[a]];
+            o = g > MP_PAIR_GATE;
+            most = max(most, o ? g : 0u);
+        }
+        ordered[j] = o;
+        cnt += o;
+    }
+    block_add(cnt, &st[0]);
+    for (int d = kWave / 2; d > 0; d >>= 1) most = max(most, (uint32_t)__shfl_down(most, d, kWave));
+    if (__lane_id() == 0 && most > st[1]) atomicMax(&st[1], (unsigned long long)most);
+}
+
+// The ordered pairs in parallel rounds with the sequential loop's outcome.
+// Let q be the number of a pair; a pair still in play is dropped once its two
+// components are one, or both hold more than 1000 reads (neither ever changes
+// again).  The others join their components in one of two cases:
+//   one holds more than 1000: when q is the lowest number in play on the small
+//     one.  No earlier pair changes the small one any more, so the loop joins
+//     them at q; and taking it early is unseen by the earlier pairs on the
+//     large one, which is large to them with it or without it.
+//   both are small: when q is the lowest number in play on both.
+// The lowest number in play always qualifies, so every round settles a pair;
+// with numbers in no order along the graph the rounds are about its logarithm.
+// A component's label is its largest read id, whatever the order of its joins.
+//
+// Most pairs wait, for many rounds, on the few components that grow through
+// their first thousand reads, so what a waiting pair costs is what a round
+// costs: a root's parts lie in one 16-byte node; its lowest pair stands until a
+// join changes the root (only a join takes a root's lowest pair out of play:
+// pairs are dropped between roots that a join made one, or large); a pair that
+// is not the lowest is left out of the round's second kernel; and the list is
+// closed up every kPairStep rounds only.  450,000 waiting pairs of 4 M reads
+// take 41 + 32 -> 30 + 14 us a round, the first of them the two nodes a pair
+// from 64 MB.  (Pairs that wait for the bit of the lowest pair to be set, and
+// read no node meanwhile: 30 + 10, since most wait on a root that changes in
+// every round.)
+struct __align__(16) PairTree {
+    uint32_t up;    // forest over the roots: any root stays one, a large component's always does
+    uint32_t size;  // reads, exact up to 1000
+    uint32_t res;   // lowest pair in play (small components); ~0: to be found
+    uint32_t lab;   // largest read id
+};
+struct PairRounds {
+    PairTree *t;
+    uint4 *list[2];  // pairs in play: two roots, pair number, state
+    uint32_t *n;     // pairs in play after every closing up
+    unsigned long long *unions;
+};
+constexpr uint32_t kPairMaxRounds = 256, kPairStep = 4;
+constexpr uint64_t kPairsForRounds = 100000;
+constexpr uint32_t kPairSmall = 0, kPairLarge = 1, kPairWait = 2, kPairDead = 3;  // both small; y is large; not yet; settled
+
+__global__ void pair_forest_kernel(const uint32_t *__restrict__ sizes, PairTree *__restrict__ t, uint64_t N)
+{
+    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < N) *(uint4 *)&t[x] = make_uint4((uint32_t)x, sizes[x], ~0u, (uint32_t)x);
+}
+
+// place in a list for every lane with `in`, one atomic per block (all lanes of the block call)
+__device__ __forceinline__ uint32_t block_place(bool in, uint32_t *n)
+{
+    __shared__ uint32_t s_n, s_at;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const uint64_t m = __ballot(in);
+    uint32_t w = 0;
+    if (__lane_id() == 0 && m) w = atomicAdd(&s_n, (uint32_t)__popcll(m));
+    w = __shfl(w, 0, kWave);
+    __syncthreads();
+    if (threadIdx.x == 0) s_at = s_n ? atomicAdd(n, s_n) : 0u;
+    __syncthreads();
+    return s_at + w + (uint32_t)__popcll(m & lanemask_lt());
+}
+
+__global__ __launch_bounds__(1024) void pair_start_kernel(const uint32_t *__restrict__ ordered,
+                                                          const uint32_t *__restrict__ parent, uint64_t P, PairRounds R)
 {
     const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= P) return;
-    uint32_t a, b;
-    ordered[j] = pair_candidate(parent, sizes, j, a, b) && gsize[gparent[a]] > MP_PAIR_GATE;
+    const bool in = j < P && ordered[j];
+    const uint32_t at = block_place(in, &R.n[0]);
+    if (!in) return;
+    R.list[0][at] = make_uint4(parent[2 * j], parent[2 * j + 1], (uint32_t)j, kPairWait);
+}
+
+__device__ __forceinline__ uint4 pair_root(const PairTree *t, uint32_t &x)
+{
+    uint4 v = *(const uint4 *)&t[x];
+    while (v.x != x) {
+        x = v.x;
+        v = *(const uint4 *)&t[x];
+    }
+    return v;
+}
+
+// first half of a round: roots as they are now, the lowest pair on every small one
+__global__ __launch_bounds__(256) void pair_mark_kernel(PairRounds R, uint32_t step)
+{
+    const uint32_t n = R.n[step], stride = gridDim.x * blockDim.x;
+    uint4 *const list = R.list[step & 1];
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const uint4 o = list[i];
+        if (o.w == kPairDead) continue;
+        uint4 e = o;
+        uint4 x = pair_root(R.t, e.x), y = pair_root(R.t, e.y);
+        const bool lx = x.y > MP_PAIR_GATE, ly = y.y > MP_PAIR_GATE;
+        if (e.x == e.y || (lx && ly)) {
+            list[i].w = kPairDead;
+            continue;
+        }
+        if (lx) {
+            const uint32_t r = e.x;
+            e.x = e.y;
+            e.y = r;
+            x = y;
+        }
+        // (a res read while others lower it is not below the true one)
+        e.w = x.z < e.z ? kPairWait : lx || ly ? kPairLarge : y.z < e.z ? kPairWait : kPairSmall;
+        if (x.z > e.z) atomicMin(&R.t[e.x].res, e.z);
+        if (!lx && !ly && y.z > e.z) atomicMin(&R.t[e.y].res, e.z);
+        if (e.x != o.x || e.y != o.y || e.w != o.w) list[i] = e;
+    }
+}
+
+// second half: the joins.  x is in no other join of the round, nor is a small y
+__global__ __launch_bounds__(256) void pair_join_kernel(PairRounds R, uint32_t step)
+{
+    const uint32_t n = R.n[step], stride = gridDim.x * blockDim.x;
+    uint4 *const list = R.list[step & 1];
+    uint32_t cnt = 0;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const uint4 e = list[i];
+        if (e.w > kPairLarge || R.t[e.x].res != e.z || (e.w == kPairSmall && R.t[e.y].res != e.z)) continue;
+        cnt++;
+        list[i].w = kPairDead;
+        PairTree &x = R.t[e.x], &y = R.t[e.y];
+        x.up = e.y;
+        if (e.w == kPairSmall) {
+            y.size += x.size;
+            y.res = ~0u;
+        }
+        const uint32_t l = x.lab;
+        if (y.lab < l) atomicMax(&y.lab, l);
+    }
+    block_add(cnt, R.unions);
+}
+
+__global__ __launch_bounds__(1024) void pair_close_kernel(PairRounds R, uint32_t step)
+{
+    const uint32_t n = R.n[step], stride = gridDim.x * blockDim.x;
+    for (uint32_t i0 = blockIdx.x * blockDim.x; i0 < n; i0 += stride) {
+        const uint32_t i = i0 + threadIdx.x;
+        uint4 e = make_uint4(0, 0, 0, kPairDead);
+        if (i < n) e = R.list[step & 1][i];
+        const bool keep = e.w != kPairDead;
+        const uint32_t at = block_place(keep, &R.n[step + 1]);
+        if (keep) R.list[(step + 1) & 1][at] = e;
+    }
+}
+
+// initial roots of the larger candidate-graph components take their trees'
+// labels, and a label its component's size as the loop's remaining pairs need it
+__global__ void pair_label_kernel(uint32_t *__restrict__ parent, const uint32_t *__restrict__ gparent,
+                                  const uint32_t *__restrict__ gsize, uint32_t *__restrict__ sizes,
+                                  const PairTree *__restrict__ t, uint64_t N)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N || gsize[gparent[i]] <= MP_PAIR_GATE || parent[i] != (uint32_t)i) return;
+    uint32_t x = (uint32_t)i;
+    const uint4 v = pair_root(t, x);
+    parent[i] = v.w;
+    if (x == (uint32_t)i) sizes[v.w] = v.y;
+}
+
+__global__ void pair_left_kernel(PairRounds R, uint32_t step, uint32_t *__restrict__ ordered)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < R.n[step]) ordered[R.list[step & 1][i].z] = 1;
 }
 
 // The ordered pass works on compact ids: the roots of the candidate-graph
@@ -1508,6 +1690,59 @@ static uint32_t hfind(PairNode *nd, uint32_t x)
     return x;
 }
 
+// The pairs flagged in `ordered` in rounds on the device, until none is left
+// or the rounds end: then *left pairs remain, flagged in `ordered` again, on
+// the labels so far (in the roots of parent, with their sizes).  A round takes
+// 15 us and 35 us per million pairs, the host 0.6 ms and 9 ms per million, so
+// the rounds end where they have taken as long as the host would for what is
+// left: numbers that ascend along a chain of components settle one link a
+// round (in no order, half the pairs go in the first eight).
+static int pair_rounds(mp_ctx *ctx, uint32_t *ordered, uint64_t P, unsigned long long *d_unions, uint64_t *left)
+{
+    const uint64_t N = ctx->N, n0 = *left;
+    constexpr uint32_t kSteps = kPairMaxRounds / kPairStep;
+    static_assert(kSteps % 2 == 0, "two steps per look at what is left");
+    const uint64_t o_list = N * sizeof(PairTree), o_n = o_list + 2 * n0 * sizeof(uint4);
+    MP_TRY(ensure(ctx, ctx->pairc, o_n + (kSteps + 4) * sizeof(uint32_t)));
+    uint8_t *const pc = (uint8_t *)ctx->pairc.p;
+    PairRounds R{};
+    R.t = (PairTree *)pc;
+    R.list[0] = (uint4 *)(pc + o_list);
+    R.list[1] = R.list[0] + n0;
+    R.n = (uint32_t *)(pc + o_n);
+    R.unions = d_unions;
+    MP_TRY(fill_u32(ctx, R.n, 0, kSteps + 4));
+    hipLaunchKernelGGL(pair_forest_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)ctx->sizes.p, R.t, N);
+    hipLaunchKernelGGL(pair_start_kernel, dim3((unsigned)((P + 1023) / 1024)), dim3(1024), 0, ctx->stream,
+                       (const uint32_t *)ordered, (const uint32_t *)ctx->parent.p, P, R);
+    MP_HIP(hipGetLastError());
+    uint32_t step = 0, n = (uint32_t)n0;
+    while (n && step < kSteps && step * kPairStep < 48 + n / 2500) {
+        const unsigned grid = stride_grid(n);
+        for (const uint32_t end = step + 2; step < end; step++) {
+            for (uint32_t i = 0; i < kPairStep; i++) {
+                hipLaunchKernelGGL(pair_mark_kernel, dim3(grid), dim3(256), 0, ctx->stream, R, step);
+                hipLaunchKernelGGL(pair_join_kernel, dim3(grid), dim3(256), 0, ctx->stream, R, step);
+            }
+            hipLaunchKernelGGL(pair_close_kernel, dim3((grid + 3) / 4), dim3(1024), 0, ctx->stream, R, step);
+        }
+        MP_HIP(hipGetLastError());
+        MP_HIP(hipMemcpyAsync(&n, R.n + step, sizeof(n), hipMemcpyDeviceToHost, ctx->stream));
+        MP_HIP(hipStreamSynchronize(ctx->stream));
+        if (step == 2 && n > n0 / 8 * 7) break;
+    }
+    hipLaunchKernelGGL(pair_label_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (uint32_t *)ctx->parent.p,
+                       (const uint32_t *)ctx->gparent.p, (const uint32_t *)ctx->gsize.p, (uint32_t *)ctx->sizes.p,
+                       (const PairTree *)R.t, N);
+    if (n) {
+        MP_TRY(fill_u32(ctx, ordered, 0, P));
+        hipLaunchKernelGGL(pair_left_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream, R, step, ordered);
+    }
+    MP_HIP(hipGetLastError());
+    *left = n;
+    return 0;
+}
+
 int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
 {
     const uint64_t N = ctx->N;
@@ -1526,9 +1761,9 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
     // A component of G holding <= 1000 reads in total can never contain a
     // component > 1000, so every candidate inside it joins whatever the order:
     // it ends as one component rooted at its largest id.  Only candidates
-    // inside larger components of G depend on the order; those run the exact
-    // sequential loop on the host, on their own (they share no reads with the
-    // rest).
+    // inside larger components of G depend on the order (they share no reads
+    // with the rest): pair_rounds() settles those, and leaves what it could
+    // not settle in its rounds to the sequential loop on the host.
     const uint64_t P = N / 2;
     uint64_t *d_small = nullptr;
     MP_HIP(hipMallocAsync((void **)&d_small, 64 * sizeof(uint64_t), ctx->stream));
@@ -1541,6 +1776,7 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
     uint32_t *gparent = (uint32_t *)ctx->gparent.p, *gsize = (uint32_t *)ctx->gsize.p;
     uint32_t *ordered = (uint32_t *)ctx->wg_cnt.p;
     uint64_t n_ordered = 0;
+    uint64_t n_host = 0;  // those that the rounds on the device leave over
     // host side, in the ctx's pinned buffer: the ordered pairs, the compact
     // roots' sizes, the components' ranges of pairs (first [0, Kg), ends
     // [Kg, 2 Kg)) and the compact roots' final roots
@@ -1558,30 +1794,41 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
         MP_TRY(fill_u32(ctx, gsize, 0, N));
         hipLaunchKernelGGL(sizes_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)gparent, gsize,
                            N);
-        hipLaunchKernelGGL(pair_classify_kernel, dim3(nblk(P)), dim3(256), 0, ctx->stream, (const uint32_t *)parent,
-                           (const uint32_t *)sizes, (const uint32_t *)gparent, (const uint32_t *)gsize, ordered, P);
+        hipLaunchKernelGGL(pair_classify_kernel, dim3(stride_grid(P)), dim3(256), 0, ctx->stream,
+                           (const uint32_t *)parent, (const uint32_t *)sizes, (const uint32_t *)gparent,
+                           (const uint32_t *)gsize, ordered, P, (unsigned long long *)(d_small + 41));
         MP_HIP(hipGetLastError());
-        MP_TRY(scan_u32(ctx, ordered, (uint64_t *)ctx->wg_off.p, P));
-        MP_HIP(hipMemcpyAsync(&n_ordered, (uint64_t *)ctx->wg_off.p + P, sizeof(uint64_t), hipMemcpyDeviceToHost,
-                              ctx->stream));
+        uint64_t cl[2];
+        MP_HIP(hipMemcpyAsync(cl, d_small + 41, sizeof(cl), hipMemcpyDeviceToHost, ctx->stream));
         MP_HIP(hipStreamSynchronize(ctx->stream));
-        if (n_ordered) {  // the ordered pairs on compact root ids, and those roots' sizes
-            MP_TRY(ensure(ctx, ctx->pairc, N * 4 + 2 * (N + 1) * 8 + n_ordered * 8 + 3 * N * 4 + 256));
+        n_ordered = n_host = cl[0];
+        // the host takes 0.6 ms and 9 ms per million pairs, as one thread does
+        // on the largest component or 16 on all; the rounds about 1.2 ms and
+        // 1.1 per million (134 k pairs of 24 samples: 1.0 against 1.9 with 0.7
+        // of them on the host; 446 k of one component: 4.7 against 2.3)
+        if (std::max(n_ordered / 16, std::min(n_ordered, cl[1] / 2)) >= kPairsForRounds)
+            MP_TRY(pair_rounds(ctx, ordered, P, d_unions, &n_host));
+        if (n_host) {  // the pairs left over, on the labels that the rounds left
+            if (n_host < n_ordered) MP_TRY(compress_labels(ctx, parent, nullptr, N));
+            MP_TRY(scan_u32(ctx, ordered, (uint64_t *)ctx->wg_off.p, P));
+        }
+        if (n_host) {  // the ordered pairs on compact root ids, and those roots' sizes
+            MP_TRY(ensure(ctx, ctx->pairc, N * 4 + 2 * (N + 1) * 8 + n_host * 8 + 3 * N * 4 + 256));
             uint8_t *pc = (uint8_t *)ctx->pairc.p;
             d_flag = (uint32_t *)pc;
             d_cid = (uint64_t *)(pc + ((N * 4 + 7) & ~7ull));
             uint64_t *d_gid = d_cid + (N + 1);
             d_pairs = d_gid + (N + 1);
-            d_csize = (uint32_t *)(d_pairs + n_ordered);
+            d_csize = (uint32_t *)(d_pairs + n_host);
             d_corig = d_csize + N;
             d_cfinal = d_corig + N;
             // pairs of different candidate-graph components share no roots: they
             // are grouped by component (a stable sort), and the components run
             // on several host threads
             for (int b = 0; b < 2; b++) {
-                MP_TRY(ensure(ctx, ctx->items[b], n_ordered * sizeof(uint64_t)));
-                MP_TRY(ensure(ctx, ctx->ilens[b], n_ordered * sizeof(uint32_t)));
-                MP_TRY(ensure(ctx, ctx->iaux[b], n_ordered + 16));
+                MP_TRY(ensure(ctx, ctx->items[b], n_host * sizeof(uint64_t)));
+                MP_TRY(ensure(ctx, ctx->ilens[b], n_host * sizeof(uint32_t)));
+                MP_TRY(ensure(ctx, ctx->iaux[b], n_host + 16));
             }
             hipLaunchKernelGGL(big_groot_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)gparent,
                                (const uint32_t *)gsize, d_flag, N);
@@ -1604,20 +1851,20 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
             MP_HIP(hipStreamSynchronize(ctx->stream));
             const uint32_t gmask = Kg <= 256 ? 0x2u : Kg <= 65536 ? 0x6u : Kg <= (1u << 24) ? 0xEu : 0x1Eu;
             int cur = 0, gpasses = 0;
-            MP_TRY(radix_sort_generic(ctx, ctx->items, ctx->ilens, ctx->iaux, &cur, n_ordered, gmask, &gpasses,
+            MP_TRY(radix_sort_generic(ctx, ctx->items, ctx->ilens, ctx->iaux, &cur, n_host, gmask, &gpasses,
                                       nullptr, 0, nullptr));
             MP_HIP(hipMallocAsync((void **)&d_cfl, 2 * Kg * sizeof(uint32_t), ctx->stream));
             MP_TRY(fill_u32(ctx, d_cfl, 0, 2 * Kg));
             uint64_t *d_sorted = (uint64_t *)ctx->items[1 - cur].p;
-            hipLaunchKernelGGL(pair_group_kernel, dim3(nblk(n_ordered)), dim3(256), 0, ctx->stream,
+            hipLaunchKernelGGL(pair_group_kernel, dim3(nblk(n_host)), dim3(256), 0, ctx->stream,
                                (const uint64_t *)ctx->items[cur].p, (const uint32_t *)ctx->ilens[cur].p,
-                               (const uint64_t *)d_pairs, n_ordered, d_sorted, d_cfl, d_cfl + Kg);
+                               (const uint64_t *)d_pairs, n_host, d_sorted, d_cfl, d_cfl + Kg);
             MP_HIP(hipGetLastError());
             // pinned: the ctx's own buffer when it is large enough, else the FASTQ
             // upload's two staging buffers when present (idle once the upload
             // has left) and each part fits one, else a new buffer of the ctx
             // (pinning costs about 0.25 ms per MB, once)
-            const uint64_t need_a = (n_ordered * 8 + 63) & ~63ull, need_b = (2 * M + 2 * Kg) * 4 + 64;
+            const uint64_t need_a = (n_host * 8 + 63) & ~63ull, need_b = (2 * M + 2 * Kg) * 4 + 64;
             uint8_t *pa = nullptr, *pb = nullptr;
             if (ctx->pair_host_bytes >= need_a + need_b) {
                 pa = (uint8_t *)ctx->pair_host;
@@ -1642,7 +1889,7 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
             cs = (uint32_t *)pb;
             cfl = cs + M;
             cp = cfl + 2 * Kg;
-            MP_HIP(hipMemcpyAsync(hpairs, d_sorted, n_ordered * 8, hipMemcpyDeviceToHost, ctx->stream));
+            MP_HIP(hipMemcpyAsync(hpairs, d_sorted, n_host * 8, hipMemcpyDeviceToHost, ctx->stream));
             MP_HIP(hipMemcpyAsync(cs, d_csize, M * 4, hipMemcpyDeviceToHost, ctx->stream));
             MP_HIP(hipMemcpyAsync(cfl, d_cfl, 2 * Kg * 4, hipMemcpyDeviceToHost, ctx->stream));
             MP_HIP(hipFreeAsync(d_cfl, ctx->stream));
@@ -1653,7 +1900,7 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
     }
     uint64_t unions = 0;
     double host_ms = 0;
-    if (n_ordered) {
+    if (n_host) {
         MP_HIP(hipStreamSynchronize(ctx->stream));
         const auto t0 = std::chrono::steady_clock::now();
         // parent and size side by side: a find ends on the line it reads the size from
