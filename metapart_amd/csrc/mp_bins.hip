@@ -49,7 +49,7 @@ constexpr int kStepPos = 960;       // base positions a wave takes per step: 60 
 constexpr int kStepRec = 480;       // records of a step (more: the radix path)
 constexpr int kMaxRun = 31;         // windows per record
 constexpr uint32_t kBinCap = 4096;  // windows of a bin that bin_runs takes; its table's slots
-constexpr uint32_t kBinRec = 640;   // records of such a bin
+constexpr uint32_t kBinRec = 1024;  // records of such a bin
 constexpr uint32_t kBinAim = kBinCap * 3 / 4;  // windows per bin aimed at, at most (fewer where records hold few)
 constexpr int kRunThreads = 1024;
 constexpr uint64_t kRunGrid = 1ull << 21;  // bins of a dispatch of bin_runs: fewer than 2^32 threads
@@ -60,7 +60,7 @@ constexpr int kStripes = 64;        // copies of the global counters, a cache li
 struct BinRec {  // a super-k-mer: consecutive windows of one read with one minimizer
     uint64_t a;      // first window's base (40 bits) | windows << 40 (5) | flags << 45 (2) | cell << 47 (13)
     uint32_t label;
-    uint32_t pad;
+    uint32_t in;     // its windows in the bucket range, the last at bit 0 (scans of part of the buckets)
 };
 static_assert(kRunGrid * kRunThreads < (1ull << 32), "one dispatch");
 static_assert(sizeof(BinRec) == 16, "one 16-byte access");
@@ -70,10 +70,8 @@ struct BinDesc {
     uint32_t rec0, nrec, nwin, smp;
 };
 
-constexpr uint32_t kErrRange = 16;  // BinCtl::err: a k-mer outside the scan's range where every one was to be inside
-
 struct BinCtl {  // device counters of a scan, cleared before it
-    unsigned long long nvalid[kMaxSeg];  // windows without 'N' per sample (plain: [0])
+    unsigned long long nvalid[kMaxSeg];  // windows without 'N' per sample (plain: [0], in the bucket range: [1])
     unsigned long long kmax1[kMaxSeg];   // 1 + the largest k-mer of every segment (0: none)
     unsigned long long nrec;
     unsigned long long out;              // labels written (64-aligned per bin)
@@ -81,7 +79,7 @@ struct BinCtl {  // device counters of a scan, cleared before it
     uint32_t nbin, nbig, err;
     uint32_t pad;
     uint32_t found[kMaxSeg];             // live labels seen in the last segment (of the sample): kFoundOther, kFoundLast
-    unsigned long long stat[kStripes][16];  // [0] runs, [1] zeroed, [2] windows in range
+    unsigned long long stat[kStripes][16];  // [0] runs, [1] zeroed
 };
 
 struct BinScan {
@@ -93,6 +91,7 @@ struct BinScan {
     int K, steps;             // wave steps per wave of a tile
     uint64_t nsteps;          // wave steps of the input
     uint32_t lo, hi;          // bucket range
+    uint16_t *inr;            // windows in it, one bit per base, as nmask; nullptr: all are
     int T;                    // segments (plain) or samples (batch)
     const uint32_t *bounds;   // T + 1 bucket boundaries (plain)
     const uint64_t *first;    // T + 1 first read ids (batch), else nullptr
@@ -170,7 +169,7 @@ __device__ __forceinline__ void bin_of(uint32_t h, uint32_t nc, int cell_bits, u
 // first position of a lane whose 16 windows are all valid without a start
 // (about 2 % more records; it bounds a record to 16 + 15 windows).
 template <int M, int W>
-__global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
+__global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
 {
     __shared__ uint64_t s_rec[4][kStepRec];
     __shared__ uint32_t s_cnt[kNC];
@@ -186,6 +185,7 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
         s_max[j] = P.ctl->kmax1[j];
         s_nv[j] = 0;
     }
+    if (tid == 0) s_nv[1] = 0;
     for (uint32_t j = tid; j <= (uint32_t)P.T; j += 256) {
         if (batch) {
             s_first[j] = P.first[j];
@@ -213,7 +213,8 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
         rank = lo + 1;
     }
     const uint64_t nh = (P.total + 127) / 16;  // halves that the streams hold at the least
-    uint32_t over = 0, nv = 0;
+    uint32_t over = 0, nv = 0, nin = 0;
+    const uint32_t lo12 = P.lo << 12, span = P.inr ? (P.hi << 12) - lo12 : ~0u;  // of the top 16 bases
     unsigned long long rec_total = 0;
     for (uint64_t ws = ws0; ws < ws1; ws++) {
         const uint64_t p0 = ws * kStepPos, h = p0 / 16 + lane;
@@ -326,8 +327,6 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
                     c0 = s_cb[s];
                     nc = s_cb[s + 1] - c0;
                     atomicAdd(&s_nv[s], (misc >> 10) & 31);
-                } else {
-                    nv += (misc >> 10) & 31;
                 }
                 uint32_t coarse, cell;
                 bin_of((uint32_t)(v >> 32), nc, P.cell_bits, coarse, cell);
@@ -344,14 +343,37 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
             const int zs = 2 * (33 - K);
             const uint32_t Z0 = fun32(Y0, Y1, zs), Z1 = fun32(Y1, Y2, zs);
             uint32_t cand = 0;
+            if (!batch) {
+                nv += (uint32_t)__popc(Vo);
+                uint32_t I = 0xFFFF;
+                if (P.inr) {
+                    I = 0;
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        const uint32_t c = min(fun32(X0, X1, 2 * j), fun32(Z0, Z1, 2 * (15 - j)));
+                        I = I + I + (c - lo12 < span ? 1u : 0u);
+                    }
+                    I &= Vo;
+                    nin += (uint32_t)__popc(I);
+                    if (lane < 60) P.inr[h ^ 3] = (uint16_t)I;
+                }
+                cand = I;
+            }
             if (P.T == 1 && !batch) {
                 const unsigned long long m1 = s_max[0];
-                const uint32_t thr = m1 ? (uint32_t)((m1 - 1) >> sh) : 0u;
+                const uint32_t thr = m1 ? (uint32_t)((m1 - 1) >> sh) : 0u, top = P.inr ? lo12 + span - thr : 0u - thr;
+                // [thr, end of the range); thr = 0 (nothing seen yet) or the end at 2^32: all from thr on
+                bool any = false;
 #pragma unroll
                 for (int j = 0; j < 16; j++) {
                     const uint32_t c = min(fun32(X0, X1, 2 * j), fun32(Z0, Z1, 2 * (15 - j)));
-                    const uint32_t b = c >> 12;
-                    if (c >= thr && b >= P.lo && b < P.hi) cand |= 1u << (15 - j);
+                    any |= c - thr <= top - 1;
+                }
+                if (!any) cand = 0;
+                else {
+#pragma unroll
+                    for (int j = 0; j < 16; j++)
+                        if (min(fun32(X0, X1, 2 * j), fun32(Z0, Z1, 2 * (15 - j))) < thr) cand &= ~(0x8000u >> j);
                 }
             } else if (batch) {
                 // the sample of the lane's windows, when they all lie in one read's sample
@@ -371,10 +393,10 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
                     const uint32_t f = (uint32_t)((((((uint64_t)X0 << 32) | X1) << (2 * j)) >> 32));
                     const uint32_t r = (uint32_t)((((((uint64_t)Z0 << 32) | Z1) << (2 * (15 - j))) >> 32));
                     const uint32_t c = min(f, r), b = c >> 12;
-                    if (b < P.lo || b >= P.hi || !((Vo >> (15 - j)) & 1)) continue;
+                    if (!((cand >> (15 - j)) & 1)) continue;
                     const int t = last_le(s_bnd, P.T, b);
                     const unsigned long long m1 = s_max[t];
-                    if (!m1 || c >= (uint32_t)((m1 - 1) >> sh)) cand |= 1u << (15 - j);
+                    if (m1 && c < (uint32_t)((m1 - 1) >> sh)) cand &= ~(0x8000u >> j);
                 }
             }
             cand &= Vo;
@@ -396,8 +418,14 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
     }
     if (over) atomicOr(&P.ctl->err, 1u);
     if (!batch) {
-        for (int o = kWave / 2; o > 0; o >>= 1) nv += __shfl_down(nv, o, kWave);
-        if (lane == 0) atomicAdd(&s_nv[0], nv);
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            nv += __shfl_down(nv, o, kWave);
+            nin += __shfl_down(nin, o, kWave);
+        }
+        if (lane == 0) {
+            atomicAdd(&s_nv[0], nv);
+            if (nin) atomicAdd(&s_nv[1], nin);
+        }
     }
     __syncthreads();
     for (uint32_t j = tid; j < kNC; j += 256) P.cnt[(uint64_t)blockIdx.x * kNC + j] = s_cnt[j];
@@ -405,7 +433,7 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(BinScan P)
         if (s_max[j] > P.ctl->kmax1[j]) atomicMax(&P.ctl->kmax1[j], s_max[j]);
         if (batch && s_nv[j]) atomicAdd(&P.ctl->nvalid[j], (unsigned long long)s_nv[j]);
     }
-    if (!batch && tid == 0 && s_nv[0]) atomicAdd(&P.ctl->nvalid[0], (unsigned long long)s_nv[0]);
+    if (!batch && tid < 2 && s_nv[tid]) atomicAdd(&P.ctl->nvalid[tid], (unsigned long long)s_nv[tid]);
     if (lane == 0 && rec_total) atomicAdd(&P.ctl->nrec, rec_total);
 }
 
@@ -467,7 +495,7 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(KParams G, const uint6
                                                           const uint32_t *__restrict__ nrec,
                                                           const uint32_t *__restrict__ erank,
                                                           const uint32_t *__restrict__ offs, int steps, uint64_t nsteps,
-                                                          uint4 *__restrict__ rec)
+                                                          const uint64_t *__restrict__ inr, uint4 *__restrict__ rec)
 {
     __shared__ uint32_t s_cur[kNC];
     // tiles of one XCD in one range: the partial lines of two neighbouring tiles meet in one L2
@@ -488,8 +516,14 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(KParams G, const uint6
             const uint64_t a = pos | ((uint64_t)((misc >> 10) & 31) << 40) | ((uint64_t)((misc >> 15) & 3) << 45) |
                                ((uint64_t)cell << 47);
             const uint32_t label = label_of(G, r);
+            uint32_t in = 0;
+            if (inr) {
+                const uint32_t o = (uint32_t)pos & 63;
+                const uint64_t w = (inr[pos >> 6] << o) | ((inr[(pos >> 6) + 1] >> 1) >> (63 - o));
+                in = (uint32_t)(w >> (64 - ((misc >> 10) & 31)));
+            }
             const uint32_t q = atomicAdd(&s_cur[coarse], 1u);
-            rec[q] = make_uint4((uint32_t)a, (uint32_t)(a >> 32), label, 0u);
+            rec[q] = make_uint4((uint32_t)a, (uint32_t)(a >> 32), label, in);
         }
     }
 }
@@ -499,7 +533,8 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(KParams G, const uint6
 // into bins where the running window count passes a multiple of `aim`, the
 // records moved to their bin (a cursor per bin: a bin's records are written in
 // order, so its lines fill in L2).
-template <int NM>
+// PART: a record's windows are those in the bucket range.
+template <int NM, bool PART>
 __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict__ rec, const uint32_t *__restrict__ coarse,
                                                          const uint32_t *__restrict__ smp_of,
                                                          uint4 *__restrict__ out, BinDesc *__restrict__ bins,
@@ -524,13 +559,17 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
     const uint32_t cmask = NM - 1;
     constexpr int kU = 4;
     for (uint32_t i0 = tid; i0 < n; i0 += kU * 1024) {
-        uint32_t h[kU];
+        uint32_t h[kU], in[kU];
 #pragma unroll
-        for (int u = 0; u < kU; u++) h[u] = r2[2 * (uint64_t)min(i0 + u * 1024, n - 1)].y;
+        for (int u = 0; u < kU; u++) {
+            const uint64_t at = 2 * (uint64_t)min(i0 + u * 1024, n - 1);
+            h[u] = r2[at].y;
+            in[u] = PART ? r2[at + 1].y : 0u;
+        }
 #pragma unroll
         for (int u = 0; u < kU; u++)
             if (i0 + u * 1024 < n)
-                atomicAdd(&s_h[(h[u] >> 15) & cmask], (1ull << 32) | ((h[u] >> 8) & 31));
+                atomicAdd(&s_h[(h[u] >> 15) & cmask], (1ull << 32) | (PART ? (uint32_t)__popc(in[u]) : (h[u] >> 8) & 31));
     }
     __syncthreads();
     // prefix of (records, windows) over the cells, kPer consecutive cells a lane
@@ -753,6 +792,17 @@ __device__ __forceinline__ void side_verdict(const uint32_t tl[4], uint32_t len,
                              : (double)__fdiv_rn((float)(int)second, (float)(int)len) > 0.2;
 }
 
+// a side's tallies by 2-bit code, as bin_runs keeps them (the in side's codes are the complement's), in the
+// order of the classes and back: class of a base is code ^ code >> 1, and the complement flips its bit 1
+__device__ __forceinline__ void code_verdict(uint32_t t0, uint32_t t1, bool out, uint32_t len, uint32_t &arg, bool &ratio)
+{
+    const uint32_t a = t0 & 0xFFFF, b = t0 >> 16, c = t1 & 0xFFFF, d = t1 >> 16;
+    const uint32_t tl[4] = {out ? a : d, out ? b : c, out ? d : a, out ? c : b};
+    uint32_t cls;
+    side_verdict(tl, len, cls, ratio);
+    arg = out ? cls ^ (cls >> 1) : (0x4Bu >> (2 * cls)) & 3;  // 3, 2, 0, 1
+}
+
 // meta word of a slot, first the tallies ...
 constexpr uint32_t kCntMask = 0xFFFF;  // tuples; 16 + c: in class c seen, 24 + c: out class c (7, 'N', is not counted)
 // ... then the run's verdict: place of its labels (13 bits) and
@@ -773,12 +823,22 @@ __device__ __forceinline__ void note_found(uint32_t f, uint32_t *flag)
 // LDS of bin_runs: the staged records are dead once every window is expanded
 // into registers, so the table takes their place; its keys are dead once the
 // runs are evaluated, and make room for the labels and the side tallies.
-struct RunsStage {
-    ulonglong2 fw[kBinRec];   // 64 bases from the one before the first window
-    ulonglong2 rc[kBinRec];   // their reverse complement, from 32 - K bases on
-    uint32_t lab[kBinRec];
-    uint32_t map[kBinCap];    // window: record | its place in the record << 10 | 'N' class before << 15, after << 16
+// A staged record: 64 bases from two before its first window, their reverse
+// complement from 31 - K bases on, its label.  Window o's base before it and
+// its K bases are then two 32-bit funnel shifts by 30 - 2 o of three words from
+// word o / 16 on; its reverse strand's the same of the second sequence by
+// 2 o + 2 from word (30 - o) / 16 on.
+struct RunsRow {
+    uint32_t fw[4], rc[4], lab;
 };
+struct RunsStage {
+    RunsRow row[kBinRec];
+    uint32_t map[kBinCap];  // window: its row's byte offset | 2 x its place in the record << 16 | 'N' flags
+};
+static_assert(sizeof(RunsRow) * kBinRec <= 0x10000, "16-bit offsets");
+// a window's flags: no base before it or after it.  Bits 24 and 27 (in side, out side) where its strand is the
+// canonical one, 28 and 31 where the other is: the sides change places
+constexpr uint32_t kMapPrevN = (1u << 27) | (1u << 28), kMapNextN = (1u << 24) | (1u << 31);
 struct RunsTable {
     unsigned long long key[kBinCap];
     uint32_t meta[kBinCap];
@@ -792,12 +852,11 @@ union RunsLds {
     } out;
 };
 
-// Bound by vector instructions: about 300 per 64 windows, against 380 with the
-// windows' places found by bit scans and a probe loop per window (1.44e9
-// windows, k = 31: 16.9 -> 13.0 ms; 512 lanes of 8 windows: 18.6).  4096
-// windows, a lane for 4, is what two workgroups per CU and 64 registers hold.
+// Bound by vector instructions: FIGURES
+// 4096 windows, a lane for 4, is what two workgroups per CU and 64 registers hold.
 // CHECK: only note which live labels there are (the first-run quirk's test).
-// PART: the scan holds part of the buckets.
+// PART: the scan holds part of the buckets; only the records' windows in them
+// are laid out (4 scans of 2 M reads: FIGPART).
 template <bool CHECK, bool PART>
 __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
 {
@@ -806,7 +865,7 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     __shared__ __align__(16) RunsLds U;
     __shared__ uint16_t s_list[kBinCap];               // slots in use
     __shared__ unsigned long long s_ob[kBinCap / 64];  // run starts among the labels
-    __shared__ uint32_t s_sum[kWaves], s_nkey, s_red[3];
+    __shared__ uint32_t s_sum[kWaves], s_nkey, s_red[2];
     __shared__ uint64_t s_out;
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const BinDesc d = P.bins[blockIdx.x];
@@ -820,32 +879,52 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         bases64(P.packed, (((uint64_t)rc.y << 32) | rc.x) & ((1ull << 40) - 1), fh, fl);
     }
     const uint32_t L = (rc.y >> 8) & 31;  // 0 past the records
-    const uint32_t inc = wave_incl(L);
+    const uint32_t nl = PART ? (uint32_t)__popc(rc.w) : L;
+    const uint32_t inc = wave_incl(nl);
     if (lane == kWave - 1) s_sum[wave] = inc;
     if (tid < kBinCap / 64) s_ob[tid] = 0;
-    if (tid < 3) s_red[tid] = 0;
+    if (tid < 2) s_red[tid] = 0;
     if (tid == 0) s_nkey = 0;
     __syncthreads();
     if (have) {  // the records' windows laid end to end
-        uint32_t o = inc - L;
+        uint32_t o = inc - nl;
         for (uint32_t w = 0; w < wave; w++) o += s_sum[w];
-        U.st.fw[tid] = make_ulonglong2(fh, fl);
+        RunsRow &row = U.st.row[tid];
         const uint64_t rh = revcomp(fl, 32), rl = revcomp(fh, 32);
-        const int sh = 2 * (32 - K);  // 2 .. 24
-        U.st.rc[tid] = make_ulonglong2((rh << sh) | (rl >> (64 - sh)), rl << sh);
-        U.st.lab[tid] = rc.z;
-        const uint32_t f = (rc.y >> 13) & 3;
-        uint32_t e = tid | ((f & kPrevN) << 15);
-        for (uint32_t q = 0; q + 1 < L; q++) {
-            U.st.map[o + q] = e;
-            e = (e & 0x7FFF) + 1024;
+        const int sh = 2 * (31 - K);  // 0 .. 22
+        const uint64_t a = fh >> 2, b = (fh << 62) | (fl >> 2), c = (rh << sh) | ((rl >> 1) >> (63 - sh)), e = rl << sh;
+        row.fw[0] = (uint32_t)(a >> 32);
+        row.fw[1] = (uint32_t)a;
+        row.fw[2] = (uint32_t)(b >> 32);
+        row.fw[3] = (uint32_t)b;
+        row.rc[0] = (uint32_t)(c >> 32);
+        row.rc[1] = (uint32_t)c;
+        row.rc[2] = (uint32_t)(e >> 32);
+        row.rc[3] = (uint32_t)e;
+        row.lab = rc.z;
+        const uint32_t f = (rc.y >> 13) & 3, at = tid * (uint32_t)sizeof(RunsRow);
+        const uint32_t pn = (f & kPrevN) ? kMapPrevN : 0u, nn = (f & kNextN) ? kMapNextN : 0u;
+        if constexpr (PART) {
+            for (uint32_t m = rc.w << ((32 - L) & 31); m;) {
+                const uint32_t q = (uint32_t)__builtin_clz(m);
+                m &= ~(0x80000000u >> q);
+                U.st.map[o++] = at | (q << 17) | (q == 0 ? pn : 0u) | (q + 1 == L ? nn : 0u);
+            }
+        } else {
+            uint32_t e = at | pn;
+            for (uint32_t q = 0; q + 1 < L; q++) {
+                U.st.map[o + q] = e;
+                e = (e & 0x3FFFFF) + (2u << 16);
+            }
+            U.st.map[o + L - 1] = e | nn;
         }
-        U.st.map[o + L - 1] = e | ((f & kNextN) << 15);
     }
     __syncthreads();
-    // every window's k-mer, neighbour classes and label
+    // every window's k-mer (from bit 61 down), neighbour codes and label
     uint64_t key[kPer];
-    uint32_t lab[kPer], st[kPer];  // st: slot | place in its run << 12 | classes << 24; ~0: no tuple
+    uint32_t lab[kPer], st[kPer];  // st: slot | place in its run << 12 | codes << 24; ~0: no tuple
+    const int kz = 62 - 2 * K;     // zero bits below a key
+    const uint64_t kmask = (~0ull >> 2) >> kz << kz;
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
         const uint32_t j = i * kRunThreads + tid;
@@ -853,23 +932,20 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         lab[i] = 0;
         key[i] = 0;
         if (j < d.nwin) {
-            const uint32_t m = U.st.map[j], r = m & 1023, o2 = (m >> 9) & 62;
-            const ulonglong2 f = U.st.fw[r], g = U.st.rc[r];
-            lab[i] = U.st.lab[r];
-            const uint64_t y = (f.x << o2) | ((f.y >> 1) >> (63 - o2));
-            const uint32_t q2 = 60 - o2;
-            const uint64_t z = (g.x << q2) | ((g.y >> 1) >> (63 - q2));
+            const uint32_t m = U.st.map[j], w = (m >> 16) & 63;
+            const char *const row = (const char *)&U.st + (m & 0xFFFF);
+            const uint32_t *const yw = (const uint32_t *)(row + ((w >> 3) & 4));
+            const uint32_t *const zw = (const uint32_t *)(row + 16 + (((60 - w) >> 3) & 4));
+            lab[i] = *(const uint32_t *)(row + 32);
+            const uint32_t y1 = yw[1], z1 = zw[1], zs = w + 2, ys = 0u - zs;
+            const uint32_t yh = __builtin_amdgcn_alignbit(yw[0], y1, ys), yl = __builtin_amdgcn_alignbit(y1, yw[2], ys);
+            const uint32_t zh = __builtin_amdgcn_alignbit(zw[0], z1, zs), zl = __builtin_amdgcn_alignbit(z1, zw[2], zs);
             // y: base before, K bases ...; z: complement of the base after, reverse complement of the K bases ...
-            const uint64_t F = (y << 2) >> (64 - 2 * K), R = (z << 2) >> (64 - 2 * K);
+            const uint64_t F = (((uint64_t)yh << 32) | yl) & kmask, R = (((uint64_t)zh << 32) | zl) & kmask;
             const bool fwd = F < R;
             key[i] = fwd ? F : R;
-            const uint32_t yh = (uint32_t)(y >> 32), zh = (uint32_t)(z >> 32);
-            const uint32_t u = (fwd ? zh : yh) >> 30, v = (fwd ? yh : zh) >> 30;
-            // class of a base: bits 1-3 of its letter (A 0, C 1, T 2, G 3), code ^ code >> 1; the complement flips bit 1
-            const uint32_t pn = (m >> 15) & 1, nn = (m >> 16) & 1;
-            const uint32_t ci = (u ^ (u >> 1) ^ 2) | ((fwd ? nn : pn) ? 7u : 0u), co = (v ^ (v >> 1)) | ((fwd ? pn : nn) ? 7u : 0u);
-            const uint32_t b = (uint32_t)(key[i] >> (2 * K - 20));
-            if (!PART || (b >= P.lo && b < P.hi)) st[i] = (ci << 24) | (co << 27) | (key_hash(key[i]) >> 20);
+            const uint32_t u = (fwd ? zh : yh) >> 30, v = ((fwd ? yh : zh) >> 27) & 0x18;
+            st[i] = ((u | v | ((m >> (fwd ? 22 : 26)) & 0x24)) << 24) | (key_hash(key[i]) >> 20);
         }
     }
     __syncthreads();
@@ -936,7 +1012,7 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     uint32_t cnt[kPer], run[kPer], at[kPer];  // tuples; verdict; slot
     uint32_t add = 0, nz = 0, nlast = 0;
     const bool one = P.T == 1 || P.batch;
-    const uint64_t lk = one ? P.ctl->kmax1[d.smp] : 0;
+    const uint64_t lk = one ? P.ctl->kmax1[d.smp] : 0, last = lk ? (lk - 1) << kz : kNoKey;
 #pragma unroll
     for (int q = 0; q < kPer; q++) {
         cnt[q] = run[q] = at[q] = 0;
@@ -945,10 +1021,10 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         if (x >= nkey) continue;
         const uint32_t s = s_list[x], m = U.tb.meta[s], c = m & kCntMask;
         const uint64_t k = U.tb.key[s];
-        const uint32_t b = (uint32_t)(k >> (2 * K - 20));
+        const uint32_t b = (uint32_t)(k >> 42);
         at[q] = s;
         cnt[q] = c;
-        const bool is_last = k + 1 == (one ? lk : last_of(P, k, d.smp));
+        const bool is_last = one ? k == last : (k >> kz) + 1 == last_of(P, k >> kz, d.smp);
         const uint32_t mi = (m >> 16) & 15, mo = (m >> 24) & 15;
         const bool bi = mi & (mi - 1), bo = mo & (mo - 1);  // more than one class
         nlast += is_last;
@@ -960,7 +1036,6 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
             if (!is_last && (bi || bo)) v |= kRunSide | (bo ? kRunOut : 0u);
             if (k != 0 && b >= P.last_lo) v |= !is_last ? kRunWit : CHECK ? kRunLast : 0u;
         }
-        if (!PART && b >= P.hi) atomicOr(&P.ctl->err, kErrRange);
         run[q] = v;
         add += ((v & kRunJoin) ? c : 0u) | ((v & kRunSide) ? 1u << 16 : 0u);
     }
@@ -1012,12 +1087,11 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         note_found(f, &P.ctl->found[P.batch ? d.smp : 0]);
         return;
     }
-    uint32_t ver[kPer], nin = 0;
+    uint32_t ver[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
         ver[i] = 0;
         if (st[i] == ~0u) continue;
-        nin++;
         const uint32_t v = U.tb.meta[st[i] & 0xFFF];
         ver[i] = v;
         if (v & kRunJoin) U.out.lab[(v & 0x1FFF) + ((st[i] >> 12) & 0xFFF)] = lab[i];
@@ -1034,11 +1108,11 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         __syncthreads();
         for (uint32_t h = tid; h < nside; h += kRunThreads) {
             const uint32_t sl = s_list[h], t0 = U.out.tal[2 * h], t1 = U.out.tal[2 * h + 1];
-            const uint32_t tl[4] = {t0 & 0xFFFF, t0 >> 16, t1 & 0xFFFF, t1 >> 16};
+            const uint32_t v = U.tb.meta[sl];
             uint32_t arg;
             bool ratio;
-            side_verdict(tl, s_list[kBinCap / 2 + h], arg, ratio);
-            U.tb.meta[sl] |= (ratio ? kRunRatio : 0u) | (arg << 29);
+            code_verdict(t0, t1, (v & kRunOut) != 0, s_list[kBinCap / 2 + h], arg, ratio);
+            U.tb.meta[sl] = v | (ratio ? kRunRatio : 0u) | (arg << 29);
         }
     }
     __syncthreads();
@@ -1066,13 +1140,9 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         if (lane == 0) atomicAdd(&s_red[1], nz);
     }
     if (nlast) atomicSub(&s_red[0], nlast);
-    if constexpr (PART) {
-        for (int o = kWave / 2; o > 0; o >>= 1) nin += __shfl_down(nin, o, kWave);
-        if (lane == 0) atomicAdd(&s_red[2], nin);
-    }
     __syncthreads();
-    if (tid < 3) {
-        const uint32_t v = s_red[tid] + (tid == 0 ? nkey : tid == 2 && !PART ? d.nwin : 0u);
+    if (tid < 2) {
+        const uint32_t v = s_red[tid] + (tid == 0 ? nkey : 0u);
         if (v) atomicAdd(&P.ctl->stat[blockIdx.x % kStripes][tid], (unsigned long long)v);
     }
 }
@@ -1097,13 +1167,13 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
     __shared__ ulonglong2 s_seq[kBigRec];
     __shared__ uint32_t s_lab[kBigRec], s_fl[kBigRec], s_off[kBigRec + 1];
     __shared__ uint8_t s_map[kBigRec * kMaxRun + 1];
-    __shared__ uint32_t s_nkey, s_sumc[kWaves], s_sums[kWaves], s_red[3];
+    __shared__ uint32_t s_nkey, s_sumc[kWaves], s_sums[kWaves], s_red[2];
     __shared__ uint64_t s_out;
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int K = P.K;
     for (uint32_t bin = blockIdx.x; bin < P.nbin; bin += gridDim.x) {
         const BinDesc d = P.bins[bin];
-        if (tid < 3) s_red[tid] = 0;
+        if (tid < 2) s_red[tid] = 0;
         // the windows of records [g, g + kBigRec) of the part, fn(window, label, slot valid) per lane
         auto group = [&](uint32_t g, auto fn) {
             __syncthreads();
@@ -1150,7 +1220,6 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
             }
             if (tid == 0) s_nkey = 0;
             bool over = false;
-            uint32_t nin = 0;
             for (uint32_t g = 0; g < d.nrec; g += kBigRec) {
                 group(g, [&](const Window &x, uint32_t, uint32_t h) {
                     if (!mine(h)) return;
@@ -1162,7 +1231,6 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
                     atomicAdd(&s_cnt[s], 1u);
                     if (seen & ~__hip_atomic_load(&s_meta[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
                         atomicOr(&s_meta[s], seen);
-                    nin++;
                 });
                 __syncthreads();
                 if (s_nkey > kBigKeys) {  // uniform: read after the barrier, next written after another
@@ -1299,15 +1367,13 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
                 for (int o = kWave / 2; o > 0; o >>= 1) {
                     nev += __shfl_down(nev, o, kWave);
                     nz += __shfl_down(nz, o, kWave);
-                    nin += __shfl_down(nin, o, kWave);
                 }
                 if (lane == 0) {
                     atomicAdd(&s_red[0], nev);
                     atomicAdd(&s_red[1], nz);
-                    atomicAdd(&s_red[2], nin);
                 }
                 __syncthreads();
-                if (tid < 3) {
+                if (tid < 2) {
                     if (s_red[tid])
                         atomicAdd(&P.ctl->stat[bin % kStripes][tid], (unsigned long long)s_red[tid]);
                     s_red[tid] = 0;
@@ -1466,6 +1532,9 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     MP_ROOM(ensure(ctx, ctx->rts, o_end + 64));
     MP_ROOM(ensure(ctx, ctx->binctl, sizeof(BinCtl) + 64 * sizeof(uint64_t) + (kMaxSeg + 1) * sizeof(uint64_t)));
     MP_ROOM(ensure(ctx, ctx->keys[0], desc_bytes));
+    const uint32_t lo = (uint32_t)std::min<uint64_t>(job.lo, MP_NBUCKETS), hi = (uint32_t)std::min<uint64_t>(job.hi, MP_NBUCKETS);
+    const bool ranged = !batch && !(lo == 0 && hi == MP_NBUCKETS);
+    if (ranged) MP_ROOM(ensure(ctx, ctx->adj[1], nsteps * (kStepPos / 8) + 64));
     // a small scan holds the radix path's tuple buffers too, so that falling back to it, or a dump, allocates nothing
     if (npos <= (1ull << 24))
         for (int b = 0; b < 2; b++) {
@@ -1502,7 +1571,6 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
         for (int i = 0; i <= T; i++) h_bnd[i] = (uint32_t)std::min<uint64_t>(job.bounds[i], MP_NBUCKETS);
     }
     MP_HIP(hipMemcpyAsync(d_bnd, seg.data(), seg.size() * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
-    const uint32_t lo = (uint32_t)std::min<uint64_t>(job.lo, MP_NBUCKETS), hi = (uint32_t)std::min<uint64_t>(job.hi, MP_NBUCKETS);
     // labels as they stand before any union of the scan, kept for a later dump
     KParams G{};
     G.N = N;
@@ -1528,6 +1596,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     S.nsteps = nsteps;
     S.lo = lo;
     S.hi = hi;
+    S.inr = ranged ? (uint16_t *)ctx->adj[1].p : nullptr;
     S.T = T;
     S.bounds = d_bnd;
     S.first = batch ? d_first : nullptr;
@@ -1547,8 +1616,10 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     std::unique_ptr<BinCtl> hc(new BinCtl);
     MP_HIP(hipMemcpyAsync(hc.get(), d_ctl, sizeof(BinCtl), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));  // also: seg is read by the copy above
-    uint64_t nv = 0;
-    for (int i = 0; i < (batch ? T : 1); i++) nv += hc->nvalid[i];
+    uint64_t nv = 0;  // the scan's tuples
+    for (int i = 0; i < (batch ? T : 1); i++) nv += hc->nvalid[ranged ? 1 : i];
+    // a range that holds every window (one scan up to the last bucket that is not empty) needs no choice of windows
+    const bool part = ranged && nv < hc->nvalid[0];
     const uint64_t nrec = hc->nrec;
     if (hc->err || nv == 0 || nrec >= (1ull << 32) || nrec * sizeof(BinRec) > ctx->keys[0].bytes ||
         (nrec * sizeof(BinRec) > key_room(npos) && nrec * sizeof(BinRec) > (64ull << 20)))
@@ -1560,6 +1631,9 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
             (*tpos)[i + 1] = (*tpos)[i] + hc->nvalid[i];
         }
     }
+    if (job.expected && nv != job.expected)  // before any read is marked
+        return ctx->fail(MP_ECOUNT, "scan %d enumerated %llu tuples, the histogram sized %llu", job.s, (unsigned long long)nv,
+                         (unsigned long long)job.expected);
     // the last segment that holds tuples: the first-run quirk can only show there
     uint32_t last_lo = 0;
     if (!batch)
@@ -1574,17 +1648,14 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     uint32_t *const d_wit = (uint32_t *)(d_big + bin_cap);
     uint4 *const rec_a = (uint4 *)ctx->keys[1].p, *const rec_b = (uint4 *)ctx->keys[0].p;
     hipLaunchKernelGGL(bin_scatter_kernel, dim3(tiles), dim3(256), 0, ctx->stream, G, (const uint64_t *)S.desc,
-                       (const uint32_t *)d_nrec, (const uint32_t *)d_rank, (const uint32_t *)d_cnt, steps, nsteps, rec_a);
+                       (const uint32_t *)d_nrec, (const uint32_t *)d_rank, (const uint32_t *)d_cnt, steps, nsteps,
+                       (const uint64_t *)(part ? S.inr : nullptr), rec_a);
     MP_HIP(hipGetLastError());
     hipEventRecord(ctx->pev[1], ctx->stream);
-    if (cell_bits == 13)
-        hipLaunchKernelGGL((bin_group_kernel<8192>), dim3(kNC), dim3(1024), 0, ctx->stream, (const uint4 *)rec_a,
-                           (const uint32_t *)d_coarse, (const uint32_t *)(batch ? d_smp : nullptr), rec_b, d_bins, d_big,
-                           (uint32_t)bin_cap, aim, d_ctl);
-    else
-        hipLaunchKernelGGL((bin_group_kernel<2048>), dim3(kNC), dim3(1024), 0, ctx->stream, (const uint4 *)rec_a,
-                           (const uint32_t *)d_coarse, (const uint32_t *)(batch ? d_smp : nullptr), rec_b, d_bins, d_big,
-                           (uint32_t)bin_cap, aim, d_ctl);
+    auto *const group = cell_bits == 13 ? (part ? bin_group_kernel<8192, true> : bin_group_kernel<8192, false>)
+                                        : (part ? bin_group_kernel<2048, true> : bin_group_kernel<2048, false>);
+    hipLaunchKernelGGL(group, dim3(kNC), dim3(1024), 0, ctx->stream, (const uint4 *)rec_a, (const uint32_t *)d_coarse,
+                       (const uint32_t *)(batch ? d_smp : nullptr), rec_b, d_bins, d_big, (uint32_t)bin_cap, aim, d_ctl);
     MP_HIP(hipGetLastError());
     MP_HIP(hipMemcpyAsync(hc.get(), d_ctl, sizeof(BinCtl), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
@@ -1616,8 +1687,6 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     R.st_bits = (uint64_t *)ctx->runbits.p;
     R.out_cap = out_cap;
     R.ctl = d_ctl;
-    // every k-mer is in the scan when the histogram sized it so; a k-mer outside it all the same sets kErrRange
-    const bool n_part = !batch && !(lo == 0 && (hi == MP_NBUCKETS || job.expected == nv));
     auto runs = [&](bool check) -> int {
         // a dispatch holds fewer than 2^32 threads, so past 4 M bins (some 6e9 windows) there are several
         for (uint64_t b0 = 0; b0 < nbin; b0 += kRunGrid) {
@@ -1625,9 +1694,9 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
             R.nbin = (uint32_t)std::min(kRunGrid, nbin - b0);
             R.wit = d_wit + b0 * kBinWit;
             const dim3 gs(R.nbin), ts(kRunThreads);
-            if (check) hipLaunchKernelGGL((bin_runs_kernel<true, true>), gs, ts, 0, ctx->stream, R);
-            else if (n_part) hipLaunchKernelGGL((bin_runs_kernel<false, true>), gs, ts, 0, ctx->stream, R);
-            else hipLaunchKernelGGL((bin_runs_kernel<false, false>), gs, ts, 0, ctx->stream, R);
+            auto *const kernel = check ? (part ? bin_runs_kernel<true, true> : bin_runs_kernel<true, false>)
+                                       : (part ? bin_runs_kernel<false, true> : bin_runs_kernel<false, false>);
+            hipLaunchKernelGGL(kernel, gs, ts, 0, ctx->stream, R);
             MP_HIP(hipGetLastError());
         }
         R.bins = d_big;
@@ -1645,11 +1714,10 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     // in-range tuples and errors before any read is marked BAD
     MP_HIP(hipMemcpyAsync(hc.get(), d_ctl, sizeof(BinCtl), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
-    uint64_t runs_n = 0, zeroed = 0, n = 0;
+    uint64_t runs_n = 0, zeroed = 0;
     for (int i = 0; i < kStripes; i++) {
         runs_n += hc->stat[i][0];
         zeroed += hc->stat[i][1];
-        n += hc->stat[i][2];
     }
     auto restore = [&]() -> int {
         if (job.s > 0) {
@@ -1658,17 +1726,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
         }
         return 0;
     };
-    if (hc->err & ~kErrRange) return restore();  // the radix path marks the same reads again
-    if (hc->err) {
-        MP_TRY(restore());
-        return ctx->fail(MP_ECOUNT, "scan %d: the histogram's %llu tuples are not all in its buckets", job.s,
-                         (unsigned long long)job.expected);
-    }
-    if (job.expected && n != job.expected) {
-        MP_TRY(restore());
-        return ctx->fail(MP_ECOUNT, "scan %d enumerated %llu tuples, the histogram sized %llu", job.s,
-                         (unsigned long long)n, (unsigned long long)job.expected);
-    }
+    if (hc->err) return restore();  // the radix path marks the same reads again
     hipEventRecord(ctx->ev[2], ctx->stream);
     MP_TRY(refilter_reads(ctx, d_nbad));
     // First-run quirk (metapart.c:2539-2616): it shows only where the last run
@@ -1729,7 +1787,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     st->zeroed_runs = zeroed;
     st->bad_labels = nbad;
     st->quirk_segments = 0;
-    *n_out = n;
+    *n_out = nv;
     *done = true;
     return 0;
 #undef MP_ROOM
