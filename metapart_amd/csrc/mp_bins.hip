@@ -26,8 +26,8 @@
 //   bin_runs_big the same for bins past the table's size, in hashed parts
 //
 // Measured, whole scan (mp_scan) of 12 M reads of 150 bases at k = 31, 1.44e9
-// tuples: 33 ms against 67.7 by radix passes; 2.2 M reads of 60-125 bases at
-// k = 21: 11 against 16.5; 2,500 reads of 100 bases: 0.30 against 0.54.
+// tuples: 23.5 ms against 67.7 by radix passes; 2.2 M reads of 60-125 bases at
+// k = 21: 6.3 against 16.5; 2,500 reads of 100 bases: 0.28 against 0.54.
 //
 // What this path leaves to the radix sort (mp_sort.hip), see bins_apply():
 // k below 20 or 32 (the reference's forward code quirk), 3-minimizer scans,
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(kNC) void bin_col_scan_kernel(uint32_t *__restrict_
     __shared__ uint32_t s_w[kNC / kWave];
     const uint32_t d = threadIdx.x, wave = d / kWave;
     uint32_t run = 0;
-    constexpr int kU = 8;
+    constexpr int kU = 8;  // loads in flight a lane (4: 5 % slower)
     for (uint32_t c0 = 0; c0 < nchunk; c0 += kU) {
         uint32_t v[kU];
 #pragma unroll
@@ -491,40 +491,118 @@ __global__ __launch_bounds__(kNC) void bin_col_apply_kernel(uint32_t *__restrict
 }
 
 // ---------------------------------------------------------------- records to their coarse bin
-__global__ __launch_bounds__(256) void bin_scatter_kernel(KParams G, const uint64_t *__restrict__ desc,
-                                                          const uint32_t *__restrict__ nrec,
-                                                          const uint32_t *__restrict__ erank,
-                                                          const uint32_t *__restrict__ offs, int steps, uint64_t nsteps,
-                                                          const uint64_t *__restrict__ inr, uint4 *__restrict__ rec)
+// A tile's records in batches, ordered by coarse bin in LDS, so that what a
+// batch holds of a bin is written together and the next batch goes on in the
+// same line.  (16 bytes at a time from 32 waves of a CU, a line was written
+// back in parts: twice the bytes.)  Batches of 6144 records fill a CU's LDS and
+// write 96 bytes of a bin at once: 140 M records of 12 M reads 3.18 -> 1.85 ms,
+// 2.10 with 3072.  A tile of few steps holds little more than one such batch,
+// and there two workgroups of 3072 on a CU overlap better: 4 scans of 2 M reads
+// (40 steps, some 4000 records a tile) 2.28 -> 1.10 ms, 1.35 with 6144.
+constexpr int kScThreads = 1024;
+constexpr int kTileSteps = 512;  // wave steps of a tile at most
+constexpr int kScLongTile = 32;  // wave steps per wave of a tile from which the batch is 6144
+
+template <int kScItems>
+__global__ __launch_bounds__(kScThreads) void bin_scatter_kernel(KParams G, const uint64_t *__restrict__ desc,
+                                                                 const uint32_t *__restrict__ nrec,
+                                                                 const uint32_t *__restrict__ erank,
+                                                                 const uint32_t *__restrict__ offs, int steps,
+                                                                 uint64_t nsteps, const uint64_t *__restrict__ inr,
+                                                                 uint4 *__restrict__ rec)
 {
-    __shared__ uint32_t s_cur[kNC];
+    constexpr int kScBatch = kScItems * kScThreads;
+    static_assert(kNC == kScThreads && kTileSteps <= kScThreads, "a bin and a step a lane");
+    __shared__ uint4 s_rec[kScBatch];
+    __shared__ uint16_t s_bin[kScBatch];
+    __shared__ uint32_t s_n[kNC], s_at[kNC], s_to[kNC];  // of a batch: records, first place; then first place in rec less that
+    __shared__ uint32_t s_first[kTileSteps + 1], s_rank[kTileSteps], s_w[kScThreads / kWave];
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     // tiles of one XCD in one range: the partial lines of two neighbouring tiles meet in one L2
     const uint64_t g = gridDim.x, b = blockIdx.x, x = b & 7, per = g >> 3, rem = g & 7;
     const uint64_t tile = x * per + (x < rem ? x : rem) + (b >> 3);
-    for (uint32_t j = threadIdx.x; j < kNC; j += 256) s_cur[j] = offs[tile * kNC + j];
+    const uint64_t ws0 = tile * 4 * steps;
+    const uint32_t ns = (uint32_t)min((uint64_t)(4 * steps), nsteps - ws0);
+    auto prefix = [&](uint32_t v, uint32_t &total) {  // sum over the lanes before this one
+        const uint32_t inc = wave_incl(v);
+        __syncthreads();  // s_w is read until here
+        if (lane == kWave - 1) s_w[wave] = inc;
+        __syncthreads();
+        const uint32_t t = wave_incl(s_w[lane % (kScThreads / kWave)]);
+        total = (uint32_t)__builtin_amdgcn_readlane((int)t, kScThreads / kWave - 1);
+        const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+        return inc - v + (w ? (uint32_t)__builtin_amdgcn_readlane((int)t, (int)w - 1) : 0u);
+    };
+    uint32_t all = 0;
+    {
+        const uint32_t v = tid < ns ? nrec[ws0 + tid] : 0u, at = prefix(v, all);
+        if (tid < ns) {
+            s_first[tid] = at;
+            s_rank[tid] = erank[ws0 + tid];
+        }
+        if (tid == 0) s_first[ns] = all;
+    }
+    uint32_t cur = offs[tile * kNC + tid];
+    s_n[tid] = 0;
     __syncthreads();
-    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const uint64_t ws0 = (tile * 4 + wave) * steps, ws1 = min(ws0 + steps, nsteps);
-    for (uint64_t ws = ws0; ws < ws1; ws++) {
-        const uint32_t n = nrec[ws];
-        const uint64_t r0 = erank[ws];
-        for (uint32_t i = lane; i < n; i += kWave) {
-            const uint64_t v = desc[ws * kStepRec + i];
-            const uint32_t misc = (uint32_t)v, coarse = (uint32_t)(v >> 32) & (kNC - 1), cell = (uint32_t)(v >> 42);
-            const uint64_t r = r0 + (misc >> 17) - 1;
-            const uint64_t pos = ws * kStepPos + (misc & 1023);
+    for (uint32_t r0 = 0; r0 < all; r0 += kScBatch) {
+        uint64_t v[kScItems];
+        uint32_t st[kScItems];
+#pragma unroll
+        for (int i = 0; i < kScItems; i++) {
+            const uint32_t r = r0 + i * kScThreads + tid;
+            st[i] = ~0u;
+            v[i] = 0;
+            if (r >= all) continue;
+            uint32_t lo = 0, hi = ns - 1;  // its step: the last with s_first <= r (steps without records share theirs)
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi + 1) >> 1;
+                if (s_first[mid] <= r) lo = mid; else hi = mid - 1;
+            }
+            st[i] = lo;
+            v[i] = desc[(ws0 + lo) * kStepRec + (r - s_first[lo])];
+        }
+        uint32_t at[kScItems];  // bin | place in it << 10 (no record: ~0)
+        uint4 x[kScItems];
+#pragma unroll
+        for (int i = 0; i < kScItems; i++) {
+            at[i] = ~0u;
+            if (st[i] == ~0u) continue;
+            const uint32_t misc = (uint32_t)v[i], c = (uint32_t)(v[i] >> 32) & (kNC - 1);
+            const uint64_t pos = (ws0 + st[i]) * kStepPos + (misc & 1023);
             const uint64_t a = pos | ((uint64_t)((misc >> 10) & 31) << 40) | ((uint64_t)((misc >> 15) & 3) << 45) |
-                               ((uint64_t)cell << 47);
-            const uint32_t label = label_of(G, r);
+                               (v[i] >> 42 << 47);
             uint32_t in = 0;
             if (inr) {
                 const uint32_t o = (uint32_t)pos & 63;
                 const uint64_t w = (inr[pos >> 6] << o) | ((inr[(pos >> 6) + 1] >> 1) >> (63 - o));
                 in = (uint32_t)(w >> (64 - ((misc >> 10) & 31)));
             }
-            const uint32_t q = atomicAdd(&s_cur[coarse], 1u);
-            rec[q] = make_uint4((uint32_t)a, (uint32_t)(a >> 32), label, in);
+            x[i] = make_uint4((uint32_t)a, (uint32_t)(a >> 32), label_of(G, (uint64_t)s_rank[st[i]] + (misc >> 17) - 1), in);
+            at[i] = c | (atomicAdd(&s_n[c], 1u) << 10);
         }
+        __syncthreads();
+        uint32_t n;
+        const uint32_t mine = s_n[tid], first = prefix(mine, n);
+        s_at[tid] = first;
+        s_to[tid] = cur - first;
+        cur += mine;
+        s_n[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kScItems; i++) {
+            if (at[i] == ~0u) continue;
+            const uint32_t c = at[i] & (kNC - 1), p = s_at[c] + (at[i] >> 10);
+            s_rec[p] = x[i];
+            s_bin[p] = (uint16_t)c;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kScItems; i++) {
+            const uint32_t p = i * kScThreads + tid;
+            if (p < n) rec[s_to[s_bin[p]] + p] = s_rec[p];
+        }
+        // (the next batch writes s_rec and s_to only behind two more barriers)
     }
 }
 
@@ -557,7 +635,7 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
     __syncthreads();
     const uint2 *const r2 = (const uint2 *)(rec + r0);
     const uint32_t cmask = NM - 1;
-    constexpr int kU = 4;
+    constexpr int kU = 8;  // loads in flight a lane (4: 5 % slower)
     for (uint32_t i0 = tid; i0 < n; i0 += kU * 1024) {
         uint32_t h[kU], in[kU];
 #pragma unroll
@@ -823,17 +901,17 @@ __device__ __forceinline__ void note_found(uint32_t f, uint32_t *flag)
 // LDS of bin_runs: the staged records are dead once every window is expanded
 // into registers, so the table takes their place; its keys are dead once the
 // runs are evaluated, and make room for the labels and the side tallies.
-// A staged record: 64 bases from two before its first window, their reverse
-// complement from 31 - K bases on, its label.  Window o's base before it and
-// its K bases are then two 32-bit funnel shifts by 30 - 2 o of three words from
-// word o / 16 on; its reverse strand's the same of the second sequence by
-// 2 o + 2 from word (30 - o) / 16 on.
+// A staged record: 64 bases from three before its first window, their reverse
+// complement from 31 - K bases on with its words in reverse order, its label.
+// Window o's base before it and its K bases are then two 32-bit funnel shifts
+// by -2 o - 4 of three words from the word that bit 5 of 2 o + 2 names on, and
+// its reverse strand's the same of the second sequence by 2 o + 2.
 struct RunsRow {
     uint32_t fw[4], rc[4], lab;
 };
 struct RunsStage {
     RunsRow row[kBinRec];
-    uint32_t map[kBinCap];  // window: its row's byte offset | 2 x its place in the record << 16 | 'N' flags
+    uint32_t map[kBinCap];  // window: its row's byte offset | 2 + 2 x its place in the record << 16 | 'N' flags
 };
 static_assert(sizeof(RunsRow) * kBinRec <= 0x10000, "16-bit offsets");
 // a window's flags: no base before it or after it.  Bits 24 and 27 (in side, out side) where its strand is the
@@ -852,11 +930,15 @@ union RunsLds {
     } out;
 };
 
-// Bound by vector instructions: FIGURES
-// 4096 windows, a lane for 4, is what two workgroups per CU and 64 registers hold.
+// Bound by vector instructions (83 % of the cycles): about 280 per 64 windows,
+// against 380 with the windows' places found by bit scans and a probe loop per
+// window, and 300 with 64-bit shifts per window (1.44e9 windows, k = 31: 16.9
+// -> 12.6 ms; 512 lanes of 8 windows: 18.6).  4096 windows, a lane for 4, is
+// what two workgroups per CU and 64 registers hold.
 // CHECK: only note which live labels there are (the first-run quirk's test).
 // PART: the scan holds part of the buckets; only the records' windows in them
-// are laid out (4 scans of 2 M reads: FIGPART).
+// are laid out (4 scans of 2 M reads of 150 bases: 6.8 -> 3.4 ms against
+// expanding all of them).
 template <bool CHECK, bool PART>
 __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
 {
@@ -886,21 +968,22 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     if (tid < 2) s_red[tid] = 0;
     if (tid == 0) s_nkey = 0;
     __syncthreads();
+    uint32_t o = inc - nl;
+    if (wave > 0 && wave * kWave < d.nrec)  // lane w of the sum: windows of the waves up to w
+        o += (uint32_t)__builtin_amdgcn_readlane((int)wave_incl(s_sum[lane % kWaves]), (int)wave - 1);
     if (have) {  // the records' windows laid end to end
-        uint32_t o = inc - nl;
-        for (uint32_t w = 0; w < wave; w++) o += s_sum[w];
         RunsRow &row = U.st.row[tid];
         const uint64_t rh = revcomp(fl, 32), rl = revcomp(fh, 32);
         const int sh = 2 * (31 - K);  // 0 .. 22
-        const uint64_t a = fh >> 2, b = (fh << 62) | (fl >> 2), c = (rh << sh) | ((rl >> 1) >> (63 - sh)), e = rl << sh;
+        const uint64_t a = fh >> 4, b = (fh << 60) | (fl >> 4), c = (rh << sh) | ((rl >> 1) >> (63 - sh)), e = rl << sh;
         row.fw[0] = (uint32_t)(a >> 32);
         row.fw[1] = (uint32_t)a;
         row.fw[2] = (uint32_t)(b >> 32);
         row.fw[3] = (uint32_t)b;
-        row.rc[0] = (uint32_t)(c >> 32);
-        row.rc[1] = (uint32_t)c;
-        row.rc[2] = (uint32_t)(e >> 32);
-        row.rc[3] = (uint32_t)e;
+        row.rc[3] = (uint32_t)(c >> 32);
+        row.rc[2] = (uint32_t)c;
+        row.rc[1] = (uint32_t)(e >> 32);
+        row.rc[0] = (uint32_t)e;
         row.lab = rc.z;
         const uint32_t f = (rc.y >> 13) & 3, at = tid * (uint32_t)sizeof(RunsRow);
         const uint32_t pn = (f & kPrevN) ? kMapPrevN : 0u, nn = (f & kNextN) ? kMapNextN : 0u;
@@ -908,10 +991,10 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
             for (uint32_t m = rc.w << ((32 - L) & 31); m;) {
                 const uint32_t q = (uint32_t)__builtin_clz(m);
                 m &= ~(0x80000000u >> q);
-                U.st.map[o++] = at | (q << 17) | (q == 0 ? pn : 0u) | (q + 1 == L ? nn : 0u);
+                U.st.map[o++] = at | ((q + 1) << 17) | (q == 0 ? pn : 0u) | (q + 1 == L ? nn : 0u);
             }
         } else {
-            uint32_t e = at | pn;
+            uint32_t e = at | (2u << 16) | pn;
             for (uint32_t q = 0; q + 1 < L; q++) {
                 U.st.map[o + q] = e;
                 e = (e & 0x3FFFFF) + (2u << 16);
@@ -932,14 +1015,14 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         lab[i] = 0;
         key[i] = 0;
         if (j < d.nwin) {
-            const uint32_t m = U.st.map[j], w = (m >> 16) & 63;
-            const char *const row = (const char *)&U.st + (m & 0xFFFF);
-            const uint32_t *const yw = (const uint32_t *)(row + ((w >> 3) & 4));
-            const uint32_t *const zw = (const uint32_t *)(row + 16 + (((60 - w) >> 3) & 4));
-            lab[i] = *(const uint32_t *)(row + 32);
-            const uint32_t y1 = yw[1], z1 = zw[1], zs = w + 2, ys = 0u - zs;
+            const uint32_t m = U.st.map[j], zs = m >> 16, ys = 0u - 2 - zs;  // (a shift takes the low five bits)
+            const uint32_t *const row = (const uint32_t *)((const char *)&U.st + (m & 0xFFFF));
+            const uint32_t *const yw = row + ((m >> 21) & 1);
+            const uint32_t *const zw = yw + 4;
+            lab[i] = row[8];
+            const uint32_t y1 = yw[1], z1 = zw[1];
             const uint32_t yh = __builtin_amdgcn_alignbit(yw[0], y1, ys), yl = __builtin_amdgcn_alignbit(y1, yw[2], ys);
-            const uint32_t zh = __builtin_amdgcn_alignbit(zw[0], z1, zs), zl = __builtin_amdgcn_alignbit(z1, zw[2], zs);
+            const uint32_t zh = __builtin_amdgcn_alignbit(zw[2], z1, zs), zl = __builtin_amdgcn_alignbit(z1, zw[0], zs);
             // y: base before, K bases ...; z: complement of the base after, reverse complement of the K bases ...
             const uint64_t F = (((uint64_t)yh << 32) | yl) & kmask, R = (((uint64_t)zh << 32) | zl) & kmask;
             const bool fwd = F < R;
@@ -1501,6 +1584,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     const uint64_t desc_bytes = nsteps * kStepRec * sizeof(uint64_t);
     if (npos == 0 || (desc_bytes > key_room(npos) && desc_bytes > (64ull << 20))) return 0;  // mostly reads without windows
     // wave steps per wave: about 8192 tiles (their table of counts stays small), at least one step
+    static_assert(4 * 128 <= kTileSteps, "a tile's steps");
     const int steps = (int)std::min<uint64_t>(128, (nsteps + 4 * 8192 - 1) / (4 * 8192));
     const uint32_t tiles = (uint32_t)((nsteps + 4 * (uint64_t)steps - 1) / (4 * (uint64_t)steps));
     const uint32_t chunks = (tiles + kColTiles - 1) / kColTiles;
@@ -1647,7 +1731,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     BinDesc *const d_bins = (BinDesc *)ctx->lab[1].p, *const d_big = d_bins + bin_cap;
     uint32_t *const d_wit = (uint32_t *)(d_big + bin_cap);
     uint4 *const rec_a = (uint4 *)ctx->keys[1].p, *const rec_b = (uint4 *)ctx->keys[0].p;
-    hipLaunchKernelGGL(bin_scatter_kernel, dim3(tiles), dim3(256), 0, ctx->stream, G, (const uint64_t *)S.desc,
+    hipLaunchKernelGGL(steps >= kScLongTile ? bin_scatter_kernel<6> : bin_scatter_kernel<3>, dim3(tiles), dim3(kScThreads), 0, ctx->stream, G, (const uint64_t *)S.desc,
                        (const uint32_t *)d_nrec, (const uint32_t *)d_rank, (const uint32_t *)d_cnt, steps, nsteps,
                        (const uint64_t *)(part ? S.inr : nullptr), rec_a);
     MP_HIP(hipGetLastError());
