@@ -58,6 +58,18 @@ __device__ __forceinline__ void block_add(uint32_t v, unsigned long long *ctr)
         if (t) atomicAdd(ctr, (unsigned long long)t);
     }
 }
+// inclusive prefix sum over the wave's lanes (all active): four shifts inside
+// the 16-lane rows, then the rows' totals, on the vector unit alone
+__device__ __forceinline__ uint32_t wave_incl(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);  // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2 and 3
+    return v;
+}
 // grid of at most 2048 workgroups of 256 lanes for a grid-stride loop over n items
 inline unsigned stride_grid(uint64_t n)
 {
