@@ -772,40 +772,55 @@ __global__ void compress_kernel(uint32_t *parent, const uint8_t *__restrict__ ba
     parent[i] = x;
 }
 
-// sizes[r] += reads x with parent[x] = r.  A component holding much of the
-// input (the 3-minimizer graph before its pair step, a 100 M-read scan's
-// largest component) would serialise millions of device atomics on one
-// address, so a workgroup first counts its 256 reads' roots in a small LDS
-// hash table (four probes; a root that finds no slot adds singly) and then
-// adds each root it saw once.
-constexpr uint32_t kSizeSlots = 512;
-__global__ __launch_bounds__(256) void sizes_kernel(const uint32_t *__restrict__ parent, uint32_t *__restrict__ sizes,
-                                                    uint64_t N)
+// sizes[r] = reads x with parent[x] = r, for roots r (0 for the others).  The
+// roots count themselves in the pass that clears the array.  A component that
+// holds much of the input (the 3-minimizer graph before its pair step, a 100
+// M-read scan's largest component) would serialise device atomics on one
+// address, some 40 ns each: a workgroup first counts its 8192 reads' roots in
+// an LDS hash table (four probes; a root that finds no slot adds singly) and
+// adds each root it saw once.  Per call, 4 M 3-minimizer reads, 2.2 M deep
+// ones: 0.07, 0.03 ms (256 reads and 512 slots per workgroup, roots counted like the
+// others: 0.40, 0.29 ms).
+constexpr uint32_t kSizeSlots = 4096, kSizeReads = 8;
+
+__global__ void sizes_clear_kernel(const uint32_t *__restrict__ parent, uint32_t *__restrict__ sizes, uint64_t N)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < N) sizes[i] = parent[i] == (uint32_t)i;
+}
+
+__global__ __launch_bounds__(1024) void sizes_kernel(const uint32_t *__restrict__ parent, uint32_t *__restrict__ sizes,
+                                                     uint64_t N)
 {
     __shared__ uint32_t s_key[kSizeSlots], s_cnt[kSizeSlots];
-    for (uint32_t j = threadIdx.x; j < kSizeSlots; j += blockDim.x) {
+    for (uint32_t j = threadIdx.x; j < kSizeSlots; j += 1024) {
         s_key[j] = ~0u;
         s_cnt[j] = 0;
     }
     __syncthreads();
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < N) {
-        const uint32_t v = parent[i];
-        const uint32_t h = (v * 2654435761u) >> 23;  // 9 bits
+    const uint64_t i0 = (uint64_t)blockIdx.x * (1024 * kSizeReads) + threadIdx.x;
+    uint32_t v[kSizeReads];
+#pragma unroll
+    for (uint32_t q = 0; q < kSizeReads; q++) v[q] = i0 + q * 1024 < N ? parent[i0 + q * 1024] : ~0u;
+#pragma unroll
+    for (uint32_t q = 0; q < kSizeReads; q++) {
+        if (i0 + q * 1024 >= N || v[q] == (uint32_t)(i0 + q * 1024)) continue;
+        const uint32_t h = (v[q] * 2654435761u) >> 20;  // 12 bits
         bool done = false;
         for (uint32_t p = 0; p < 4 && !done; p++) {
             const uint32_t slot = (h + p) & (kSizeSlots - 1);
-            const uint32_t old = atomicCAS(&s_key[slot], ~0u, v);
-            if (old == ~0u || old == v) {
+            uint32_t old = s_key[slot];
+            if (old == ~0u) old = atomicCAS(&s_key[slot], ~0u, v[q]);
+            if (old == ~0u || old == v[q]) {
                 atomicAdd(&s_cnt[slot], 1u);
                 done = true;
             }
         }
-        if (!done) atomicAdd(&sizes[v], 1u);
+        if (!done) atomicAdd(&sizes[v[q]], 1u);
     }
     __syncthreads();
-    for (uint32_t j = threadIdx.x; j < kSizeSlots; j += blockDim.x)
-        if (s_key[j] != ~0u) atomicAdd(&sizes[s_key[j]], s_cnt[j]);
+    for (uint32_t j = threadIdx.x; j < kSizeSlots; j += 1024)
+        if (s_cnt[j]) atomicAdd(&sizes[s_key[j]], s_cnt[j]);
 }
 
 __global__ __launch_bounds__(256) void root_weight_kernel(const uint32_t *__restrict__ parent,
@@ -1223,6 +1238,15 @@ __global__ __launch_bounds__(256) void sample_stats_kernel(const uint32_t *__res
 static inline unsigned nblk(uint64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
 // every read (except BAD ones, when bad is given) to its root
+static int component_sizes(mp_ctx *ctx, const uint32_t *parent, uint32_t *sizes, uint64_t N)
+{
+    hipLaunchKernelGGL(sizes_clear_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, parent, sizes, N);
+    hipLaunchKernelGGL(sizes_kernel, dim3((unsigned)((N + 1024 * kSizeReads - 1) / (1024 * kSizeReads))), dim3(1024), 0,
+                       ctx->stream, parent, sizes, N);
+    MP_HIP(hipGetLastError());
+    return 0;
+}
+
 static int compress_labels(mp_ctx *ctx, uint32_t *parent, const uint8_t *bad, uint64_t N)
 {
     if (N == 0) return 0;
@@ -1751,9 +1775,7 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
     hipEventRecord(ctx->ev[5], ctx->stream);
     // sizes after the last scan (metapart.c:4010-4021)
     MP_TRY(compress_labels(ctx, parent, (const uint8_t *)ctx->bad.p, N));
-    MP_TRY(fill_u32(ctx, sizes, 0, N));
-    hipLaunchKernelGGL(sizes_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)parent, sizes, N);
-    MP_HIP(hipGetLastError());
+    MP_TRY(component_sizes(ctx, parent, sizes, N));
     // Pair step (unionFindPeReads): pair (2j, 2j+1) joins its two components
     // unless both hold more than 1000 reads at that moment.  Sizes only grow,
     // so a pair whose components are both > 1000 now never joins, and the
@@ -1791,9 +1813,7 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
         hipLaunchKernelGGL(pair_graph_kernel, dim3(nblk(P)), dim3(256), 0, ctx->stream, (const uint32_t *)parent,
                            (const uint32_t *)sizes, gparent, P);
         MP_TRY(compress_labels(ctx, gparent, nullptr, N));
-        MP_TRY(fill_u32(ctx, gsize, 0, N));
-        hipLaunchKernelGGL(sizes_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)gparent, gsize,
-                           N);
+        MP_TRY(component_sizes(ctx, gparent, gsize, N));
         hipLaunchKernelGGL(pair_classify_kernel, dim3(stride_grid(P)), dim3(256), 0, ctx->stream,
                            (const uint32_t *)parent, (const uint32_t *)sizes, (const uint32_t *)gparent,
                            (const uint32_t *)gsize, ordered, P, (unsigned long long *)(d_small + 41));
@@ -1960,9 +1980,7 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
     // every BAD read was reset to itself by the pair step
     MP_TRY(fill_u32(ctx, ctx->bad.p, 0, (N + 3) / 4));
     MP_TRY(compress_labels(ctx, parent, (const uint8_t *)ctx->bad.p, N));
-    MP_TRY(fill_u32(ctx, sizes, 0, N));
-    hipLaunchKernelGGL(sizes_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)parent, sizes, N);
-    MP_HIP(hipGetLastError());
+    MP_TRY(component_sizes(ctx, parent, sizes, N));
     // partition plan over root ids in ascending order
     MP_TRY(ensure(ctx, ctx->wg_off, (N + 1) * sizeof(uint64_t)));
     MP_TRY(ensure(ctx, ctx->wg_cnt, N * sizeof(uint32_t)));
