@@ -630,7 +630,7 @@ __global__ __launch_bounds__(256) void union_kernel(GParams G, const uint64_t *_
 // old but are always members of the same set, and takes the coherent find and
 // its compare-and-swap only where they differ.  Against union_kernel's way on
 // the same lists: 12 M reads at 5x (96 % BAD) 3.4 -> 2.4 ms, 2.2 M reads at 46x
-// 3.9 -> 1.6, a batch of 24 samples 1.5 -> 0.56.
+// 3.9 -> 1.5, a batch of 24 samples 1.5 -> 0.53.
 constexpr int kLW = 16;
 static_assert(kLW % kUW == 0, "whole steps");
 
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(256) void union_list_kernel(const uint32_t *__restr
     const uint64_t w0 = (((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave) * kLW;
     if (w0 >= nw) return;
     const uint64_t lt = lanemask_lt(), upto = lane == 63 ? ~0ull : (2ull << lane) - 1;
-    uint32_t carry = 0;       // the last live label of the run that goes on, if any
+    uint32_t carry = 0;       // an ancestor of the last live label of the run that goes on, if any
     bool have = false;
     if (w0 > 0 && !(st_bits[w0] & 1)) {  // the wave's first run began before: its last live label (uniform)
         for (uint64_t q = w0; q-- > 0 && !have;) {
@@ -663,7 +663,7 @@ __global__ __launch_bounds__(256) void union_list_kernel(const uint32_t *__restr
             const int s = m ? 63 - __builtin_clzll(m) : 0;  // the run's start in this word, if it began here
             const uint64_t v = __ballot((int)lane >= s && !((badbits[l >> 5] >> (l & 31)) & 1));
             if (v) {
-                carry = __shfl(l, 63 - __builtin_clzll(v), kWave);
+                carry = __shfl(l, 63 - __builtin_clzll(v), kWave);  // itself
                 have = true;
             }
             if (m) break;
@@ -680,6 +680,9 @@ __global__ __launch_bounds__(256) void union_list_kernel(const uint32_t *__restr
         }
 #pragma unroll
         for (int u = 0; u < kUW; u++) bw[u] = badbits[lb[u] >> 5];
+        uint32_t up[kUW];  // the live labels' parents, looked up once for both joins that a label may be in
+#pragma unroll
+        for (int u = 0; u < kUW; u++) up[u] = (bw[u] >> (lb[u] & 31)) & 1 ? 0u : parent[lb[u]];
 #pragma unroll
         for (int u = 0; u < kUW; u++) {
             if (w0 + g + u >= nw) break;
@@ -689,19 +692,19 @@ __global__ __launch_bounds__(256) void union_list_kernel(const uint32_t *__restr
                 const uint64_t sm = st[u] & upto;
                 uint64_t cand = lv & lt;
                 if (sm) cand &= ~0ull << (63 - __builtin_clzll(sm));  // lanes of the same run
-                uint32_t a = __shfl(lb[u], cand ? 63 - __builtin_clzll(cand) : 0, kWave);
+                uint32_t a = __shfl(up[u], cand ? 63 - __builtin_clzll(cand) : 0, kWave);
                 bool join = live && cand != 0;
                 if (live && !cand && !sm && have) {  // the first live label here of a run from before
                     a = carry;
                     join = true;
                 }
-                if (join && a != lb[u]) uf_join(parent, a, lb[u]);
+                if (join && a != up[u]) uf_join(parent, a, up[u]);
             }
             // the run that goes on past this word
             const uint64_t s = st[u];
             const uint64_t tail = s ? lv & (~0ull << (63 - __builtin_clzll(s))) : lv;
             if (tail) {
-                carry = __shfl(lb[u], 63 - __builtin_clzll(tail), kWave);
+                carry = __shfl(up[u], 63 - __builtin_clzll(tail), kWave);
                 have = true;
             } else if (s) {
                 have = false;
@@ -756,7 +759,15 @@ __global__ void halve_kernel(uint32_t *parent, const uint8_t *__restrict__ bad, 
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N || (bad && bad[i])) return;
-    (void)uf_find(parent, (uint32_t)i);
+    // plain loads and stores: nothing is joined meanwhile, an old value is an ancestor too, and parents ascend
+    // (2.2 M deep reads, four calls: 0.36 ms with coherent ones, 0.05 so)
+    for (uint32_t x = (uint32_t)i;;) {
+        const uint32_t p = parent[x];
+        if (p == x) return;
+        const uint32_t gp = parent[p];
+        if (gp != p) parent[x] = gp;
+        x = gp;
+    }
 }
 
 __global__ void compress_kernel(uint32_t *parent, const uint8_t *__restrict__ bad, uint64_t N)
@@ -883,13 +894,16 @@ __device__ __forceinline__ bool pair_candidate(const uint32_t *parent, const uin
     return a != b && (sizes[a] <= MP_PAIR_GATE || sizes[b] <= MP_PAIR_GATE);
 }
 
-// components of the candidate-pair graph, rooted at their largest id
+// components of the candidate-pair graph, rooted at their largest id (ancestors
+// in the cache compared first, as in union_list_kernel: 4 M 3-minimizer reads
+// 1.4 -> 0.83 ms.  An eighth of the pairs first, compressed, then the others:
+// 0.2 better on 2.2 M deep reads, 0.3 worse on these)
 __global__ void pair_graph_kernel(const uint32_t *__restrict__ parent, const uint32_t *__restrict__ sizes,
                                   uint32_t *gparent, uint64_t P)
 {
     const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t a, b;
-    if (j < P && pair_candidate(parent, sizes, j, a, b)) uf_union(gparent, a, b);
+    if (j < P && pair_candidate(parent, sizes, j, a, b)) uf_join(gparent, a, b);
 }
 
 // 1 for a candidate pair inside a candidate-graph component of > 1000 reads;
