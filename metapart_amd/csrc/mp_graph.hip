@@ -950,12 +950,12 @@ __global__ __launch_bounds__(256) void pair_classify_kernel(const uint32_t *__re
 // costs: a root's parts lie in one 16-byte node; its lowest pair stands until a
 // join changes the root (only a join takes a root's lowest pair out of play:
 // pairs are dropped between roots that a join made one, or large); a pair that
-// is not the lowest is left out of the round's second kernel; and the list is
-// closed up every kPairStep rounds only.  450,000 waiting pairs of 4 M reads
-// take 41 + 32 -> 30 + 14 us a round, the first of them the two nodes a pair
-// from 64 MB.  (Pairs that wait for the bit of the lowest pair to be set, and
-// read no node meanwhile: 30 + 10, since most wait on a root that changes in
-// every round.)
+// is not the lowest is left out of the round's second kernel; the list is
+// closed up every kPairStep rounds only; and the pairs of a root that grows in
+// every round find its lowest in LDS first, as up to a thousand atomics on one
+// address take longer than all the rest.  450,000 waiting pairs of 4 M reads
+// take 22 + 5 us a round (30 + 14 with an atomic per pair and a count per block,
+// 41 + 32 with separate arrays too).
 struct __align__(16) PairTree {
     uint32_t up;    // forest over the roots: any root stays one, a large component's always does
     uint32_t size;  // reads, exact up to 1000
@@ -966,7 +966,6 @@ struct PairRounds {
     PairTree *t;
     uint4 *list[2];  // pairs in play: two roots, pair number, state
     uint32_t *n;     // pairs in play after every closing up
-    unsigned long long *unions;
 };
 constexpr uint32_t kPairMaxRounds = 256, kPairStep = 4;
 constexpr uint64_t kPairsForRounds = 100000;
@@ -1015,11 +1014,34 @@ __device__ __forceinline__ uint4 pair_root(const PairTree *t, uint32_t &x)
 }
 
 // first half of a round: roots as they are now, the lowest pair on every small one
-__global__ __launch_bounds__(256) void pair_mark_kernel(PairRounds R, uint32_t step)
+constexpr uint32_t kMarkPairs = 2, kMarkSlots = 4096;  // pairs a lane; the LDS table's slots
+
+__global__ __launch_bounds__(1024) void pair_mark_kernel(PairRounds R, uint32_t step)
 {
-    const uint32_t n = R.n[step], stride = gridDim.x * blockDim.x;
+    __shared__ uint32_t s_key[kMarkSlots], s_min[kMarkSlots];
+    const uint32_t n = R.n[step];
     uint4 *const list = R.list[step & 1];
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const uint32_t i0 = blockIdx.x * (1024 * kMarkPairs) + threadIdx.x;
+    if (i0 - threadIdx.x >= n) return;  // the block
+    for (uint32_t j = threadIdx.x; j < kMarkSlots; j += 1024) s_key[j] = s_min[j] = ~0u;
+    __syncthreads();
+    auto lower = [&](uint32_t root, uint32_t q) {
+        const uint32_t h = (root * 2654435761u) >> 20;  // 12 bits
+        for (uint32_t p = 0; p < 4; p++) {
+            const uint32_t slot = (h + p) & (kMarkSlots - 1);
+            uint32_t old = s_key[slot];
+            if (old == ~0u) old = atomicCAS(&s_key[slot], ~0u, root);
+            if (old == ~0u || old == root) {
+                atomicMin(&s_min[slot], q);
+                return;
+            }
+        }
+        atomicMin(&R.t[root].res, q);
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < kMarkPairs; k++) {
+        const uint32_t i = i0 + k * 1024;
+        if (i >= n) break;
         const uint4 o = list[i];
         if (o.w == kPairDead) continue;
         uint4 e = o;
@@ -1037,33 +1059,32 @@ __global__ __launch_bounds__(256) void pair_mark_kernel(PairRounds R, uint32_t s
         }
         // (a res read while others lower it is not below the true one)
         e.w = x.z < e.z ? kPairWait : lx || ly ? kPairLarge : y.z < e.z ? kPairWait : kPairSmall;
-        if (x.z > e.z) atomicMin(&R.t[e.x].res, e.z);
-        if (!lx && !ly && y.z > e.z) atomicMin(&R.t[e.y].res, e.z);
+        if (x.z > e.z) lower(e.x, e.z);
+        if (!lx && !ly && y.z > e.z) lower(e.y, e.z);
         if (e.x != o.x || e.y != o.y || e.w != o.w) list[i] = e;
     }
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < kMarkSlots; j += 1024)
+        if (s_key[j] != ~0u) atomicMin(&R.t[s_key[j]].res, s_min[j]);
 }
 
 // second half: the joins.  x is in no other join of the round, nor is a small y
 __global__ __launch_bounds__(256) void pair_join_kernel(PairRounds R, uint32_t step)
 {
-    const uint32_t n = R.n[step], stride = gridDim.x * blockDim.x;
+    const uint32_t n = R.n[step], i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
     uint4 *const list = R.list[step & 1];
-    uint32_t cnt = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint4 e = list[i];
-        if (e.w > kPairLarge || R.t[e.x].res != e.z || (e.w == kPairSmall && R.t[e.y].res != e.z)) continue;
-        cnt++;
-        list[i].w = kPairDead;
-        PairTree &x = R.t[e.x], &y = R.t[e.y];
-        x.up = e.y;
-        if (e.w == kPairSmall) {
-            y.size += x.size;
-            y.res = ~0u;
-        }
-        const uint32_t l = x.lab;
-        if (y.lab < l) atomicMax(&y.lab, l);
+    const uint4 e = list[i];
+    if (e.w > kPairLarge || R.t[e.x].res != e.z || (e.w == kPairSmall && R.t[e.y].res != e.z)) return;
+    list[i].w = kPairDead;
+    PairTree &x = R.t[e.x], &y = R.t[e.y];
+    x.up = e.y;
+    if (e.w == kPairSmall) {
+        y.size += x.size;
+        y.res = ~0u;
     }
-    block_add(cnt, R.unions);
+    const uint32_t l = x.lab;
+    if (y.lab < l) atomicMax(&y.lab, l);
 }
 
 __global__ __launch_bounds__(1024) void pair_close_kernel(PairRounds R, uint32_t step)
@@ -1080,17 +1101,24 @@ __global__ __launch_bounds__(1024) void pair_close_kernel(PairRounds R, uint32_t
 }
 
 // initial roots of the larger candidate-graph components take their trees'
-// labels, and a label its component's size as the loop's remaining pairs need it
-__global__ void pair_label_kernel(uint32_t *__restrict__ parent, const uint32_t *__restrict__ gparent,
-                                  const uint32_t *__restrict__ gsize, uint32_t *__restrict__ sizes,
-                                  const PairTree *__restrict__ t, uint64_t N)
+// labels (every root but the one that is the label was joined to another), and
+// a label its component's size as the loop's remaining pairs need it
+__global__ __launch_bounds__(256) void pair_label_kernel(uint32_t *__restrict__ parent, const uint32_t *__restrict__ gparent,
+                                                         const uint32_t *__restrict__ gsize, uint32_t *__restrict__ sizes,
+                                                         const PairTree *__restrict__ t, uint64_t N,
+                                                         unsigned long long *__restrict__ unions)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N || gsize[gparent[i]] <= MP_PAIR_GATE || parent[i] != (uint32_t)i) return;
-    uint32_t x = (uint32_t)i;
-    const uint4 v = pair_root(t, x);
-    parent[i] = v.w;
-    if (x == (uint32_t)i) sizes[v.w] = v.y;
+    uint32_t cnt = 0;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += stride) {
+        if (gsize[gparent[i]] <= MP_PAIR_GATE || parent[i] != (uint32_t)i) continue;
+        uint32_t x = (uint32_t)i;
+        const uint4 v = pair_root(t, x);
+        if (x == (uint32_t)i) sizes[v.w] = v.y;
+        cnt += v.w != (uint32_t)i;
+        parent[i] = v.w;
+    }
+    block_add(cnt, unions);
 }
 
 __global__ void pair_left_kernel(PairRounds R, uint32_t step, uint32_t *__restrict__ ordered)
@@ -1731,7 +1759,7 @@ static uint32_t hfind(PairNode *nd, uint32_t x)
 // The pairs flagged in `ordered` in rounds on the device, until none is left
 // or the rounds end: then *left pairs remain, flagged in `ordered` again, on
 // the labels so far (in the roots of parent, with their sizes).  A round takes
-// 15 us and 35 us per million pairs, the host 0.6 ms and 9 ms per million, so
+// 12 us and 35 us per million pairs, the host 0.6 ms and 9 ms per million, so
 // the rounds end where they have taken as long as the host would for what is
 // left: numbers that ascend along a chain of components settle one link a
 // round (in no order, half the pairs go in the first eight).
@@ -1748,7 +1776,6 @@ static int pair_rounds(mp_ctx *ctx, uint32_t *ordered, uint64_t P, unsigned long
     R.list[0] = (uint4 *)(pc + o_list);
     R.list[1] = R.list[0] + n0;
     R.n = (uint32_t *)(pc + o_n);
-    R.unions = d_unions;
     MP_TRY(fill_u32(ctx, R.n, 0, kSteps + 4));
     hipLaunchKernelGGL(pair_forest_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint32_t *)ctx->sizes.p, R.t, N);
     hipLaunchKernelGGL(pair_start_kernel, dim3((unsigned)((P + 1023) / 1024)), dim3(1024), 0, ctx->stream,
@@ -1756,22 +1783,22 @@ static int pair_rounds(mp_ctx *ctx, uint32_t *ordered, uint64_t P, unsigned long
     MP_HIP(hipGetLastError());
     uint32_t step = 0, n = (uint32_t)n0;
     while (n && step < kSteps && step * kPairStep < 48 + n / 2500) {
-        const unsigned grid = stride_grid(n);
+        const dim3 gm((n + 1024 * kMarkPairs - 1) / (1024 * kMarkPairs)), gj((n + 255) / 256), gc((n + 1023) / 1024);
         for (const uint32_t end = step + 2; step < end; step++) {
             for (uint32_t i = 0; i < kPairStep; i++) {
-                hipLaunchKernelGGL(pair_mark_kernel, dim3(grid), dim3(256), 0, ctx->stream, R, step);
-                hipLaunchKernelGGL(pair_join_kernel, dim3(grid), dim3(256), 0, ctx->stream, R, step);
+                hipLaunchKernelGGL(pair_mark_kernel, gm, dim3(1024), 0, ctx->stream, R, step);
+                hipLaunchKernelGGL(pair_join_kernel, gj, dim3(256), 0, ctx->stream, R, step);
             }
-            hipLaunchKernelGGL(pair_close_kernel, dim3((grid + 3) / 4), dim3(1024), 0, ctx->stream, R, step);
+            hipLaunchKernelGGL(pair_close_kernel, gc, dim3(1024), 0, ctx->stream, R, step);
         }
         MP_HIP(hipGetLastError());
         MP_HIP(hipMemcpyAsync(&n, R.n + step, sizeof(n), hipMemcpyDeviceToHost, ctx->stream));
         MP_HIP(hipStreamSynchronize(ctx->stream));
         if (step == 2 && n > n0 / 8 * 7) break;
     }
-    hipLaunchKernelGGL(pair_label_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (uint32_t *)ctx->parent.p,
+    hipLaunchKernelGGL(pair_label_kernel, dim3(stride_grid(N)), dim3(256), 0, ctx->stream, (uint32_t *)ctx->parent.p,
                        (const uint32_t *)ctx->gparent.p, (const uint32_t *)ctx->gsize.p, (uint32_t *)ctx->sizes.p,
-                       (const PairTree *)R.t, N);
+                       (const PairTree *)R.t, N, d_unions);
     if (n) {
         MP_TRY(fill_u32(ctx, ordered, 0, P));
         hipLaunchKernelGGL(pair_left_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream, R, step, ordered);
@@ -1837,9 +1864,9 @@ int finish_components(mp_ctx *ctx, uint64_t *W, mp_finish_stats *st)
         MP_HIP(hipStreamSynchronize(ctx->stream));
         n_ordered = n_host = cl[0];
         // the host takes 0.6 ms and 9 ms per million pairs, as one thread does
-        // on the largest component or 16 on all; the rounds about 1.2 ms and
-        // 1.1 per million (134 k pairs of 24 samples: 1.0 against 1.9 with 0.7
-        // of them on the host; 446 k of one component: 4.7 against 2.3)
+        // on the largest component or 16 on all; the rounds about 1.0 ms and
+        // 1.1 per million (134 k pairs of 24 samples: 1.0 ms on the host, 1.9 in
+        // rounds; 446 k of one component: 4.7 on the host, 1.8 in rounds)
         if (std::max(n_ordered / 16, std::min(n_ordered, cl[1] / 2)) >= kPairsForRounds)
             MP_TRY(pair_rounds(ctx, ordered, P, d_unions, &n_host));
         if (n_host) {  // the pairs left over, on the labels that the rounds left
