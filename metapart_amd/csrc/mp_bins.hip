@@ -71,15 +71,14 @@ struct BinDesc {
 };
 
 struct BinCtl {  // device counters of a scan, cleared before it
-    unsigned long long nvalid[kMaxSeg];  // windows without 'N' per sample (plain: [0], in the bucket range: [1])
+    unsigned long long nvalid[kMaxSeg];  // windows without 'N' per sample of a batch
     unsigned long long kmax1[kMaxSeg];   // 1 + the largest k-mer of every segment (0: none)
-    unsigned long long nrec;
     unsigned long long out;              // labels written (64-aligned per bin)
     unsigned long long big_win, big_max; // windows of the big bins: all, the largest
     uint32_t nbin, nbig, err;
     uint32_t pad;
     uint32_t found[kMaxSeg];             // live labels seen in the last segment (of the sample): kFoundOther, kFoundLast
-    unsigned long long stat[kStripes][16];  // [0] runs, [1] zeroed
+    unsigned long long stat[kStripes][16];  // [0] runs, [1] zeroed; of bin_scan [2] records, [3] windows, [4] of them in range
 };
 
 struct BinScan {
@@ -155,13 +154,21 @@ __device__ __forceinline__ void bin_of(uint32_t h, uint32_t nc, int cell_bits, u
 // one before (or that is not valid), at the step's first position, and at the
 // first position of a lane whose 16 windows are all valid without a start
 // (about 2 % more records; it bounds a record to 16 + 15 windows).
+// Bound by vector instructions.  A lane puts its windows' hashes and masks in
+// LDS and only lists its record starts; the records are then made 64 at a time
+// (a branch per window and lane before: 920 -> 670 instructions a step; 12 M
+// reads 3.25 -> 2.56 ms).  The tiles' totals go to 64 copies of the counters:
+// 529 k reads 0.36 -> 0.15 ms, of which 40,000 atomics on one line were most.
 template <int M, int W>
 __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
 {
-    __shared__ uint64_t s_rec[4][kStepRec];
+    __shared__ uint4 s_min[4][kWave][5];      // minimizer hashes of a lane's 16 windows (rows 80 bytes apart: no conflicts)
+    __shared__ uint4 s_lane[4][kWave];        // what else a record needs of its lane
+    __shared__ uint16_t s_start[4][kStepRec]; // the step's record starts: 16 lane + window
     __shared__ uint32_t s_cnt[kNC];
     __shared__ unsigned long long s_max[kMaxSeg];
-    __shared__ uint32_t s_nv[kMaxSeg];
+    __shared__ uint32_t s_nv[kMaxSeg];        // batch: windows per sample
+    __shared__ uint32_t s_all[3];             // records, windows, windows in range
     __shared__ uint32_t s_bnd[kMaxSeg + 1];
     __shared__ uint64_t s_first[kMaxSeg + 1];
     __shared__ uint32_t s_cb[kMaxSeg + 1];
@@ -172,7 +179,7 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
         s_max[j] = P.ctl->kmax1[j];
         s_nv[j] = 0;
     }
-    if (tid == 0) s_nv[1] = 0;
+    if (tid < 3) s_all[tid] = 0;
     for (uint32_t j = tid; j <= (uint32_t)P.T; j += 256) {
         if (batch) {
             s_first[j] = P.first[j];
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
     const uint64_t nh = (P.total + 127) / 16;  // halves that the streams hold at the least
     uint32_t over = 0, nv = 0, nin = 0;
     const uint32_t lo12 = P.lo << 12, span = P.inr ? (P.hi << 12) - lo12 : ~0u;  // of the top 16 bases
-    unsigned long long rec_total = 0;
+    uint32_t rec_total = 0;
     for (uint64_t ws = ws0; ws < ws1; ws++) {
         const uint64_t p0 = ws * kStepPos, h = p0 / 16 + lane;
         const bool have = h < nh;
@@ -258,7 +265,7 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
         uint32_t chg = 0;
         const uint32_t before = __shfl_up(a[15], 1, kWave);
 #pragma unroll
-        for (int j = 0; j < 16; j++) chg |= (a[j] != (j ? a[j - 1] : before) ? 1u : 0u) << (15 - j);
+        for (int j = 0; j < 16; j++) chg = chg + chg + (a[j] != (j ? a[j - 1] : before) ? 1u : 0u);
         const uint32_t Vb = __shfl_up(V, 1, kWave);
         const uint32_t Vn = __shfl_down(V, 1, kWave);
         const uint32_t Vo = lane < 60 ? V : 0u;
@@ -285,16 +292,12 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
         if (!fits) over = 1;
         if (fits) {
 #pragma unroll
-            for (int j = 0; j < 16; j++) {
-                if ((S >> (15 - j)) & 1) {
-                    const uint32_t rest = stop & ((1u << (15 - j)) - 1);
-                    const uint32_t L = rest ? (uint32_t)__builtin_clz(rest) - 16 - j : 16 - j + nxt;
-                    const uint32_t n7 = rest ? ((V >> (15 - (j + L))) & 1 ? 0u : kNextN) : nx7;
-                    const uint32_t p7 = (pv >> (15 - j)) & 1 ? 0u : kPrevN;
-                    const uint32_t rk = (exc >> 16) + (uint32_t)__popc(E >> (15 - j));
-                    const uint32_t misc = (16 * lane + j) | (L << 10) | ((p7 | n7) << 15) | (rk << 17);
-                    s_rec[wave][at++] = ((uint64_t)a[j] << 32) | misc;
-                }
+            for (int j = 0; j < 4; j++) s_min[wave][lane][j] = make_uint4(a[4 * j], a[4 * j + 1], a[4 * j + 2], a[4 * j + 3]);
+            s_lane[wave][lane] = make_uint4((stop << 16) | V, (pv << 16) | E, nxt | (nx7 << 8), exc >> 16);
+            for (uint32_t m = S; m;) {
+                const uint32_t j = (uint32_t)__builtin_clz(m) - 16;
+                m ^= 0x8000u >> j;
+                s_start[wave][at++] = (uint16_t)(16 * lane + j);
             }
         }
         wave_lds_fence();
@@ -306,8 +309,15 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
             rec_total += nr;
             uint64_t *out = P.desc + ws * kStepRec;
             for (uint32_t i = lane; i < nr; i += kWave) {
-                const uint64_t v = s_rec[wave][i];
-                const uint32_t misc = (uint32_t)v;
+                const uint32_t o = s_start[wave][i], j = o & 15;
+                const uint4 q = s_lane[wave][o >> 4];
+                const uint32_t hash = ((const uint32_t *)s_min[wave][o >> 4])[j];
+                const uint32_t qs = q.x >> 16, qv = q.x & 0xFFFF, rest = qs & ((0x8000u >> j) - 1);
+                const uint32_t end = rest ? (uint32_t)__builtin_clz(rest) - 16 : 16 + (q.z & 31);  // past its last window
+                const uint32_t n7 = rest ? ((qv >> (15 - end)) & 1 ? 0u : kNextN) : q.z >> 8;
+                const uint32_t p7 = (q.y >> (31 - j)) & 1 ? 0u : kPrevN;
+                const uint32_t rk = q.w + (uint32_t)__popc((q.y & 0xFFFF) >> (15 - j));
+                const uint32_t misc = o | ((end - j) << 10) | ((p7 | n7) << 15) | (rk << 17);
                 uint32_t c0 = 0, nc = kNC;
                 if (batch) {
                     const int s = last_le(s_first, P.T, rank + (misc >> 17) - 1);
@@ -316,7 +326,7 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
                     atomicAdd(&s_nv[s], (misc >> 10) & 31);
                 }
                 uint32_t coarse, cell;
-                bin_of((uint32_t)(v >> 32), nc, P.cell_bits, coarse, cell);
+                bin_of(hash, nc, P.cell_bits, coarse, cell);
                 coarse += c0;
                 atomicAdd(&s_cnt[coarse], 1u);
                 out[i] = (uint64_t)misc | ((uint64_t)coarse << 32) | ((uint64_t)cell << 42);
@@ -404,15 +414,15 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
         wave_lds_fence();
     }
     if (over) atomicOr(&P.ctl->err, 1u);
-    if (!batch) {
+    if (!batch)
         for (int o = kWave / 2; o > 0; o >>= 1) {
             nv += __shfl_down(nv, o, kWave);
             nin += __shfl_down(nin, o, kWave);
         }
-        if (lane == 0) {
-            atomicAdd(&s_nv[0], nv);
-            if (nin) atomicAdd(&s_nv[1], nin);
-        }
+    if (lane == 0) {
+        atomicAdd(&s_all[0], rec_total);
+        if (nv) atomicAdd(&s_all[1], nv);
+        if (nin) atomicAdd(&s_all[2], nin);
     }
     __syncthreads();
     for (uint32_t j = tid; j < kNC; j += 256) P.cnt[(uint64_t)blockIdx.x * kNC + j] = s_cnt[j];
@@ -420,8 +430,8 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
         if (s_max[j] > P.ctl->kmax1[j]) atomicMax(&P.ctl->kmax1[j], s_max[j]);
         if (batch && s_nv[j]) atomicAdd(&P.ctl->nvalid[j], (unsigned long long)s_nv[j]);
     }
-    if (!batch && tid < 2 && s_nv[tid]) atomicAdd(&P.ctl->nvalid[tid], (unsigned long long)s_nv[tid]);
-    if (lane == 0 && rec_total) atomicAdd(&P.ctl->nrec, rec_total);
+    // (a counter's copies: thousands of atomics on one address take longer than a small scan)
+    if (tid < 3 && s_all[tid]) atomicAdd(&P.ctl->stat[blockIdx.x % kStripes][2 + tid], (unsigned long long)s_all[tid]);
 }
 
 // ---------------------------------------------------------------- offsets of (tile, coarse bin)
@@ -610,7 +620,7 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
     __shared__ unsigned long long s_h[NM];  // records << 32 | windows per cell; then the cell's bin
     __shared__ uint64_t s_st[NM + 1];       // first record << 32 | first window of every bin; then its cursor
     __shared__ uint64_t s_w[16];
-    __shared__ uint32_t s_wb[16];
+    __shared__ uint32_t s_wb[16], s_place[2];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const uint32_t r0 = coarse[blockIdx.x], n = coarse[blockIdx.x + 1] - r0;
     if (n == 0) return;
@@ -691,10 +701,9 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
     }
     if (tid == 0) s_st[nb] = total;
     __syncthreads();
-    // the bins' entries: a place in the list per wave
+    // the bins' entries: places in the lists for all of them at once, then per wave
     const uint32_t smp = smp_of ? smp_of[blockIdx.x] : 0u;
-    for (uint32_t i0 = wave * kWave; i0 < nb; i0 += 1024) {
-        const uint32_t i = i0 + lane;
+    auto entry = [&](uint32_t i, bool &small, bool &large) {
         BinDesc d{0, 0, 0, smp};
         if (i < nb) {
             const uint64_t s = s_st[i], e = s_st[i + 1];
@@ -702,11 +711,33 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
             d.nrec = (uint32_t)(e >> 32) - (uint32_t)(s >> 32);
             d.nwin = (uint32_t)e - (uint32_t)s;
         }
-        const bool small = d.nwin && d.nwin <= kBinCap && d.nrec <= kBinRec, large = d.nwin && !small;
+        small = d.nwin && d.nwin <= kBinCap && d.nrec <= kBinRec;
+        large = d.nwin && !small;
+        return d;
+    };
+    if (tid < 2) s_place[tid] = 0;
+    __syncthreads();
+    uint32_t ns = 0, nl2 = 0;
+    for (uint32_t i0 = wave * kWave; i0 < nb; i0 += 1024) {
+        bool small, large;
+        (void)entry(i0 + lane, small, large);
+        ns += (uint32_t)__popcll(__ballot(small));
+        nl2 += (uint32_t)__popcll(__ballot(large));
+    }
+    if (lane == 0) {
+        if (ns) atomicAdd(&s_place[0], ns);
+        if (nl2) atomicAdd(&s_place[1], nl2);
+    }
+    __syncthreads();
+    if (tid < 2 && s_place[tid]) s_place[tid] = atomicAdd(tid ? &ctl->nbig : &ctl->nbin, s_place[tid]);
+    __syncthreads();
+    for (uint32_t i0 = wave * kWave; i0 < nb; i0 += 1024) {
+        bool small, large;
+        const BinDesc d = entry(i0 + lane, small, large);
         const uint64_t ms = __ballot(small), ml = __ballot(large);
         uint32_t at = 0, al = 0;
-        if (lane == 0 && ms) at = atomicAdd(&ctl->nbin, (uint32_t)__popcll(ms));
-        if (lane == 0 && ml) al = atomicAdd(&ctl->nbig, (uint32_t)__popcll(ml));
+        if (lane == 0 && ms) at = atomicAdd(&s_place[0], (uint32_t)__popcll(ms));
+        if (lane == 0 && ml) al = atomicAdd(&s_place[1], (uint32_t)__popcll(ml));
         at = __shfl(at, 0, kWave);
         al = __shfl(al, 0, kWave);
         if (small) bins[at + (uint32_t)__popcll(ms & lanemask_lt())] = d;
@@ -1687,11 +1718,16 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     std::unique_ptr<BinCtl> hc(new BinCtl);
     MP_HIP(hipMemcpyAsync(hc.get(), d_ctl, sizeof(BinCtl), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));  // also: seg is read by the copy above
-    uint64_t nv = 0;  // the scan's tuples
-    for (int i = 0; i < (batch ? T : 1); i++) nv += hc->nvalid[ranged ? 1 : i];
+    uint64_t nrec = 0, nwin = 0, nv = 0;  // records, windows, the scan's tuples
+    for (int i = 0; i < kStripes; i++) {
+        nrec += hc->stat[i][2];
+        nwin += hc->stat[i][3];
+        nv += hc->stat[i][ranged ? 4 : 3];
+    }
+    if (batch)
+        for (int i = 0; i < T; i++) nv += hc->nvalid[i];
     // a range that holds every window (one scan up to the last bucket that is not empty) needs no choice of windows
-    const bool part = ranged && nv < hc->nvalid[0];
-    const uint64_t nrec = hc->nrec;
+    const bool part = ranged && nv < nwin;
     if (hc->err || nv == 0 || nrec >= (1ull << 32) || nrec * sizeof(BinRec) > ctx->keys[0].bytes ||
         (nrec * sizeof(BinRec) > key_room(npos) && nrec * sizeof(BinRec) > (64ull << 20)))
         return 0;
