@@ -890,9 +890,9 @@ __device__ __forceinline__ void side_verdict(const uint32_t tl[4], uint32_t len,
 
 // a side's tallies by 2-bit code, as bin_runs keeps them (the in side's codes are the complement's), in the
 // order of the classes and back: class of a base is code ^ code >> 1, and the complement flips its bit 1
-__device__ __forceinline__ void code_verdict(uint32_t t0, uint32_t t1, bool out, uint32_t len, uint32_t &arg, bool &ratio)
+__device__ __forceinline__ void code_verdict(const uint32_t t[4], bool out, uint32_t len, uint32_t &arg, bool &ratio)
 {
-    const uint32_t a = t0 & 0xFFFF, b = t0 >> 16, c = t1 & 0xFFFF, d = t1 >> 16;
+    const uint32_t a = t[0], b = t[1], c = t[2], d = t[3];
     const uint32_t tl[4] = {out ? a : d, out ? b : c, out ? d : a, out ? c : b};
     uint32_t cls;
     side_verdict(tl, len, cls, ratio);
@@ -937,6 +937,7 @@ static_assert(sizeof(RunsRow) * kBinRec <= 0x10000, "16-bit offsets");
 constexpr uint32_t kMapPrevN = (1u << 27) | (1u << 28), kMapNextN = (1u << 24) | (1u << 31);
 struct RunsTable {
     unsigned long long key[kBinCap];
+    uint32_t gap[kBinCap];      // (the tallies' end)
     uint32_t meta[kBinCap];
 };
 union RunsLds {
@@ -944,7 +945,7 @@ union RunsLds {
     RunsTable tb;
     struct {
         uint32_t lab[kBinCap];      // labels in run order
-        uint32_t tal[kBinCap];      // 4 x 16-bit tallies of every branching side
+        uint32_t tal[2 * kBinCap];  // 4 tallies of every branching side (a run of two tuples at the least)
     } out;
 };
 
@@ -1023,16 +1024,15 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     __syncthreads();
     // every window's k-mer (from bit 61 down), neighbour codes and label
     uint64_t key[kPer];
-    uint32_t lab[kPer], st[kPer];  // st: slot | place in its run << 12 | codes << 24; ~0: no tuple
+    uint32_t lab[kPer], st[kPer];  // st: slot | place in its run << 12 | codes << 24
+    bool tup[kPer];                // a window there
     const int kz = 62 - 2 * K;     // zero bits below a key
     const uint64_t kmask = (~0ull >> 2) >> kz << kz;
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
         const uint32_t j = i * kRunThreads + tid;
-        st[i] = ~0u;
-        lab[i] = 0;
-        key[i] = 0;
-        if (j < d.nwin) {
+        tup[i] = j < d.nwin;
+        if (tup[i]) {
             const uint32_t m = U.st.map[j], zs = m >> 16, ys = 0u - 2 - zs;  // (a shift takes the low five bits)
             const uint32_t *const row = (const uint32_t *)((const char *)&U.st + (m & 0xFFFF));
             const uint32_t *const yw = row + ((m >> 21) & 1);
@@ -1063,7 +1063,7 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     uint32_t open = 0, fresh = 0;
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-        if (st[i] == ~0u) continue;
+        if (!tup[i]) continue;
         const uint64_t old = atomicCAS(&U.tb.key[st[i] & 0xFFF], kNoKey, (unsigned long long)key[i]);
         if (old == kNoKey) fresh |= 1u << i;
         else if (old != key[i]) open |= 1u << i;
@@ -1096,10 +1096,10 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         uint32_t old[kPer];
 #pragma unroll
         for (int i = 0; i < kPer; i++)
-            if (st[i] != ~0u) old[i] = atomicAdd(&U.tb.meta[st[i] & 0xFFF], 1u);
+            if (tup[i]) old[i] = atomicAdd(&U.tb.meta[st[i] & 0xFFF], 1u);
 #pragma unroll
         for (int i = 0; i < kPer; i++) {
-            if (st[i] == ~0u) continue;
+            if (!tup[i]) continue;
             const uint32_t s = st[i] & 0xFFF;
             const uint32_t seen = (1u << (16 + ((st[i] >> 24) & 7))) | (1u << (24 + (st[i] >> 27)));
             if (seen & ~old[i]) atomicOr(&U.tb.meta[s], seen);
@@ -1114,6 +1114,7 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     uint32_t add = 0, nz = 0, nlast = 0;
     const bool one = P.T == 1 || P.batch;
     const uint64_t lk = one ? P.ctl->kmax1[d.smp] : 0, last = lk ? (lk - 1) << kz : kNoKey;
+    const uint64_t wit = max((uint64_t)P.last_lo << 42, (uint64_t)1);  // witnesses: from the last segment on, not k-mer 0
 #pragma unroll
     for (int q = 0; q < kPer; q++) {
         cnt[q] = run[q] = at[q] = 0;
@@ -1122,12 +1123,11 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         if (x >= nkey) continue;
         const uint32_t s = s_list[x], m = U.tb.meta[s], c = m & kCntMask;
         const uint64_t k = U.tb.key[s];
-        const uint32_t b = (uint32_t)(k >> 42);
         at[q] = s;
         cnt[q] = c;
         const bool is_last = one ? k == last : (k >> kz) + 1 == last_of(P, k >> kz, d.smp);
-        const uint32_t mi = (m >> 16) & 15, mo = (m >> 24) & 15;
-        const bool bi = mi & (mi - 1), bo = mo & (mo - 1);  // more than one class
+        const uint32_t mc = (m >> 16) & 0x0F0F, m2 = mc & ((mc | 0x1010) - 0x0101);
+        const bool bi = m2 & 0xFF, bo = m2 >> 8;  // more than one class (the | keeps an empty side from borrowing)
         nlast += is_last;
         const bool zero = !is_last && bi && bo;
         nz += zero;
@@ -1135,7 +1135,7 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         if (!zero) {
             if (c >= 2 && k != 0) v |= kRunJoin;
             if (!is_last && (bi || bo)) v |= kRunSide | (bo ? kRunOut : 0u);
-            if (k != 0 && b >= P.last_lo) v |= !is_last ? kRunWit : CHECK ? kRunLast : 0u;
+            if (k >= wit) v |= !is_last ? kRunWit : CHECK ? kRunLast : 0u;
         }
         run[q] = v;
         add += ((v & kRunJoin) ? c : 0u) | ((v & kRunSide) ? 1u << 16 : 0u);
@@ -1175,13 +1175,13 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
         U.tb.meta[at[q]] = v;
     }
     if (!CHECK)
-        for (uint32_t j = tid; j < 2 * nside; j += kRunThreads) U.out.tal[j] = 0;
+        for (uint32_t j = tid; j < 4 * nside; j += kRunThreads) U.out.tal[j] = 0;
     __syncthreads();
     if constexpr (CHECK) {
         uint32_t f = 0;
 #pragma unroll
         for (int i = 0; i < kPer; i++) {
-            if (st[i] == ~0u) continue;
+            if (!tup[i]) continue;
             const uint32_t v = U.tb.meta[st[i] & 0xFFF];
             if ((v & (kRunWit | kRunLast)) && !P.bad[lab[i]]) f |= v & kRunWit ? kFoundOther : kFoundLast;
         }
@@ -1192,13 +1192,13 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
         ver[i] = 0;
-        if (st[i] == ~0u) continue;
+        if (!tup[i]) continue;
         const uint32_t v = U.tb.meta[st[i] & 0xFFF];
         ver[i] = v;
         if (v & kRunJoin) U.out.lab[(v & 0x1FFF) + ((st[i] >> 12) & 0xFFF)] = lab[i];
         if (v & kRunSide) {
             const uint32_t c = (st[i] >> ((v & kRunOut) ? 27 : 24)) & 7;
-            if (c < 4) atomicAdd(&U.out.tal[2 * ((v >> 16) & 0xFFF) + (c >> 1)], 1u << (16 * (c & 1)));
+            if (c < 4) atomicAdd(&U.out.tal[4 * ((v >> 16) & 0xFFF) + c], 1u);
         }
         if (i == 0 && wave < kBinWit) {
             const uint64_t wm = __ballot((v & kRunWit) != 0);
@@ -1208,11 +1208,11 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     if (nside) {
         __syncthreads();
         for (uint32_t h = tid; h < nside; h += kRunThreads) {
-            const uint32_t sl = s_list[h], t0 = U.out.tal[2 * h], t1 = U.out.tal[2 * h + 1];
+            const uint32_t sl = s_list[h];
             const uint32_t v = U.tb.meta[sl];
             uint32_t arg;
             bool ratio;
-            code_verdict(t0, t1, (v & kRunOut) != 0, s_list[kBinCap / 2 + h], arg, ratio);
+            code_verdict(&U.out.tal[4 * h], (v & kRunOut) != 0, s_list[kBinCap / 2 + h], arg, ratio);
             U.tb.meta[sl] = v | (ratio ? kRunRatio : 0u) | (arg << 29);
         }
     }
