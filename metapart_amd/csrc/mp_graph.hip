@@ -1759,10 +1759,12 @@ static uint32_t hfind(PairNode *nd, uint32_t x)
 // The pairs flagged in `ordered` in rounds on the device, until none is left
 // or the rounds end: then *left pairs remain, flagged in `ordered` again, on
 // the labels so far (in the roots of parent, with their sizes).  A round takes
-// 12 us and 35 us per million pairs, the host 0.6 ms and 9 ms per million, so
-// the rounds end where they have taken as long as the host would for what is
-// left: numbers that ascend along a chain of components settle one link a
-// round (in no order, half the pairs go in the first eight).
+// 12 us and 35 us per million pairs, the host 0.9 ms and 9 ms per million, and
+// pairs in no order are through in some 100 rounds (27 k of 1.35 M left after
+// 80: 0.2 ms of rounds or 0.9 on the host): the rounds end where they have
+// taken about as long as that and the host for what is left.  Numbers that
+// ascend along a chain of components settle one link a round (in no order, half
+// the pairs go in the first eight): those stop at once.
 static int pair_rounds(mp_ctx *ctx, uint32_t *ordered, uint64_t P, unsigned long long *d_unions, uint64_t *left)
 {
     const uint64_t N = ctx->N, n0 = *left;
@@ -1782,7 +1784,7 @@ static int pair_rounds(mp_ctx *ctx, uint32_t *ordered, uint64_t P, unsigned long
                        (const uint32_t *)ordered, (const uint32_t *)ctx->parent.p, P, R);
     MP_HIP(hipGetLastError());
     uint32_t step = 0, n = (uint32_t)n0;
-    while (n && step < kSteps && step * kPairStep < 48 + n / 2500) {
+    while (n && step < kSteps && step * kPairStep < 112 + n / 2500) {
         const dim3 gm((n + 1024 * kMarkPairs - 1) / (1024 * kMarkPairs)), gj((n + 255) / 256), gc((n + 1023) / 1024);
         for (const uint32_t end = step + 2; step < end; step++) {
             for (uint32_t i = 0; i < kPairStep; i++) {
