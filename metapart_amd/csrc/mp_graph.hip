@@ -1100,6 +1100,91 @@ __global__ __launch_bounds__(1024) void pair_close_kernel(PairRounds R, uint32_t
     }
 }
 
+// The last pairs' rounds in one workgroup, pairs in registers: a round is a few
+// memory latencies (5 us), not two launches of latency each (15 us).  What
+// other lanes write in the kernel is read past the CU's cache; every round ends
+// behind a device fence and a barrier.  A round settles a pair at the least, so
+// n rounds would do; `rounds` bounds them.
+constexpr uint32_t kTailLane = 8, kTailPairs = kTailLane * 1024, kTailRounds = 128;
+
+__global__ __launch_bounds__(1024) void pair_tail_kernel(PairRounds R, uint32_t step, uint32_t rounds)
+{
+    const uint32_t n = min(R.n[step], kTailPairs);
+    const uint4 *const list = R.list[step & 1];
+    auto node = [&](uint32_t x) {
+        const uint64_t *const p = (const uint64_t *)&R.t[x];
+        const uint64_t a = ld_agent(p), b = ld_agent(p + 1);
+        return make_uint4((uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32));
+    };
+    auto root = [&](uint32_t &x) {
+        uint4 v = node(x);
+        while (v.x != x) {
+            x = v.x;
+            v = node(x);
+        }
+        return v;
+    };
+    uint4 e[kTailLane];
+#pragma unroll
+    for (uint32_t k = 0; k < kTailLane; k++) {
+        const uint32_t i = k * 1024 + threadIdx.x;
+        e[k] = i < n ? list[i] : make_uint4(0, 0, 0, kPairDead);
+    }
+    for (uint32_t round = 0; round < rounds; round++) {
+#pragma unroll
+        for (uint32_t k = 0; k < kTailLane; k++) {
+            if (e[k].w == kPairDead) continue;
+            uint4 x = root(e[k].x), y = root(e[k].y);
+            const bool lx = x.y > MP_PAIR_GATE, ly = y.y > MP_PAIR_GATE;
+            if (e[k].x == e[k].y || (lx && ly)) {
+                e[k].w = kPairDead;
+                continue;
+            }
+            if (lx) {
+                const uint32_t r = e[k].x;
+                e[k].x = e[k].y;
+                e[k].y = r;
+                x = y;
+            }
+            const uint32_t q = e[k].z;
+            e[k].w = x.z < q ? kPairWait : lx || ly ? kPairLarge : y.z < q ? kPairWait : kPairSmall;
+            if (x.z > q) atomicMin(&R.t[e[k].x].res, q);
+            if (!lx && !ly && y.z > q) atomicMin(&R.t[e[k].y].res, q);
+        }
+        __threadfence();
+        __syncthreads();
+        bool join[kTailLane];
+#pragma unroll
+        for (uint32_t k = 0; k < kTailLane; k++)
+            join[k] = e[k].w <= kPairLarge && ld_agent(&R.t[e[k].x].res) == e[k].z &&
+                      (e[k].w == kPairLarge || ld_agent(&R.t[e[k].y].res) == e[k].z);
+        bool live = false;
+#pragma unroll
+        for (uint32_t k = 0; k < kTailLane; k++) {
+            if (join[k]) {  // x is in no other join of the round, nor is a small y
+                PairTree &x = R.t[e[k].x], &y = R.t[e[k].y];
+                const uint32_t l = ld_agent(&x.lab);
+                if (e[k].w == kPairSmall) {
+                    atomicAdd(&y.size, ld_agent(&x.size));
+                    __hip_atomic_store(&y.res, ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                atomicMax(&y.lab, l);
+                __hip_atomic_store(&x.up, e[k].y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                e[k].w = kPairDead;
+            }
+            live |= e[k].w != kPairDead;
+        }
+        __threadfence();
+        if (!__syncthreads_or(live)) break;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kTailLane; k++) {
+        const bool keep = e[k].w != kPairDead;
+        const uint32_t at = block_place(keep, &R.n[step + 1]);
+        if (keep) R.list[(step + 1) & 1][at] = e[k];
+    }
+}
+
 // initial roots of the larger candidate-graph components take their trees'
 // labels (every root but the one that is the label was joined to another), and
 // a label its component's size as the loop's remaining pairs need it
@@ -1797,6 +1882,14 @@ static int pair_rounds(mp_ctx *ctx, uint32_t *ordered, uint64_t P, unsigned long
         MP_HIP(hipMemcpyAsync(&n, R.n + step, sizeof(n), hipMemcpyDeviceToHost, ctx->stream));
         MP_HIP(hipStreamSynchronize(ctx->stream));
         if (step == 2 && n > n0 / 8 * 7) break;
+        if (n && n <= kTailPairs && step < kSteps) {
+            hipLaunchKernelGGL(pair_tail_kernel, dim3(1), dim3(1024), 0, ctx->stream, R, step, kTailRounds);
+            MP_HIP(hipGetLastError());
+            step++;
+            MP_HIP(hipMemcpyAsync(&n, R.n + step, sizeof(n), hipMemcpyDeviceToHost, ctx->stream));
+            MP_HIP(hipStreamSynchronize(ctx->stream));
+            break;
+        }
     }
     hipLaunchKernelGGL(pair_label_kernel, dim3(stride_grid(N)), dim3(256), 0, ctx->stream, (uint32_t *)ctx->parent.p,
                        (const uint32_t *)ctx->gparent.p, (const uint32_t *)ctx->gsize.p, (uint32_t *)ctx->sizes.p,
