@@ -1873,7 +1873,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
         if (open(true)) return 0;
     }
     hipEventRecord(ctx->ev[3], ctx->stream);
-    MP_TRY(union_label_runs(ctx, (const uint32_t *)ctx->lab[0].p, (const uint64_t *)ctx->runbits.p, hc->out));
+    MP_TRY(union_label_runs(ctx, (const uint32_t *)ctx->lab[0].p, (const uint64_t *)ctx->runbits.p, hc->out, N - nbad));
     hipEventRecord(ctx->ev[4], ctx->stream);
     MP_HIP(hipStreamSynchronize(ctx->stream));
     float ms = 0, a = 0, b = 0, u = 0;

@@ -647,11 +647,11 @@ __device__ __forceinline__ void uf_join(uint32_t *parent, uint32_t a, uint32_t b
 }
 
 __global__ __launch_bounds__(256) void union_list_kernel(const uint32_t *__restrict__ lab,
-                                                         const uint64_t *__restrict__ st_bits, uint64_t nw,
+                                                         const uint64_t *__restrict__ st_bits, uint64_t first, uint64_t nw,
                                                          const uint32_t *__restrict__ badbits, uint32_t *parent)
 {
     const uint32_t lane = __lane_id();
-    const uint64_t w0 = (((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave) * kLW;
+    const uint64_t w0 = first + (((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave) * kLW;
     if (w0 >= nw) return;
     const uint64_t lt = lanemask_lt(), upto = lane == 63 ? ~0ull : (2ull << lane) - 1;
     uint32_t carry = 0;       // an ancestor of the last live label of the run that goes on, if any
@@ -1734,7 +1734,7 @@ int refilter_reads(mp_ctx *ctx, unsigned long long *d_nbad)
     return 0;
 }
 
-int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, uint64_t n)
+int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, uint64_t n, uint64_t live)
 {
     const uint64_t N = ctx->N;
     if (n) {
@@ -1742,11 +1742,22 @@ int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, 
         uint64_t *badbits = (uint64_t *)ctx->scratch.p;
         hipLaunchKernelGGL(bad_bits_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, (const uint8_t *)ctx->bad.p, N,
                            badbits);
-        const uint64_t nw = n / 64, blocks = ((nw + kLW - 1) / kLW + 3) / 4;
-        if (!grid_fits(blocks, 256))
+        const uint64_t nw = n / 64;
+        auto blocks = [](uint64_t words) { return ((words + kLW - 1) / kLW + 3) / 4; };
+        if (!grid_fits(blocks(nw), 256))
             return ctx->fail(MP_EINVAL, "union over %llu labels exceeds one dispatch: use more scans", (unsigned long long)n);
-        hipLaunchKernelGGL(union_list_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, lab, st_bits, nw,
-                           (const uint32_t *)badbits, (uint32_t *)ctx->parent.p);
+        // where many live labels come to a read, a quarter of the runs first, and the labels to their roots: most
+        // joins of the others then end at the first look (2.2 M reads, 63 labels a read: 1.50 -> 1.13 ms; an eighth
+        // first 1.17).  Labels that an XCD's cache holds gain nothing (529 k reads: 0.088 and 0.095)
+        const uint64_t part = N >= (1u << 20) && (double)n * (double)live >= 16.0 * (double)N * (double)N ? nw / 4 : 0;
+        if (part) {
+            hipLaunchKernelGGL(union_list_kernel, dim3((unsigned)blocks(part)), dim3(256), 0, ctx->stream, lab, st_bits,
+                               (uint64_t)0, part, (const uint32_t *)badbits, (uint32_t *)ctx->parent.p);
+            MP_HIP(hipGetLastError());
+            MP_TRY(compress_labels(ctx, (uint32_t *)ctx->parent.p, (const uint8_t *)ctx->bad.p, N));
+        }
+        hipLaunchKernelGGL(union_list_kernel, dim3((unsigned)blocks(nw - part)), dim3(256), 0, ctx->stream, lab, st_bits, part,
+                           nw, (const uint32_t *)badbits, (uint32_t *)ctx->parent.p);
         MP_HIP(hipGetLastError());
     }
     return compress_labels(ctx, (uint32_t *)ctx->parent.p, (const uint8_t *)ctx->bad.p, N);

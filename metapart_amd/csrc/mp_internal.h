@@ -360,8 +360,8 @@ bool bins_apply(const mp_ctx *ctx, int T);
 int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uint64_t> *tpos, uint64_t *n_out, bool *done);
 // filtered reads to BAD ones; *d_nbad (device, zero before) takes their number
 int refilter_reads(mp_ctx *ctx, unsigned long long *d_nbad);
-// joins every run of the n labels (run starts in st_bits), then compresses
-int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, uint64_t n);
+// joins every run of the n labels (run starts in st_bits), then compresses; live: reads that are not BAD
+int union_label_runs(mp_ctx *ctx, const uint32_t *lab, const uint64_t *st_bits, uint64_t n, uint64_t live);
 // the zeroed runs of the sorted tuples in the current buffers (zbits), segments at device positions d_seg[0..nseg]
 int filter_zbits(mp_ctx *ctx, uint64_t n, const uint64_t *d_seg, int nseg);
 int filter_zbits_scan(mp_ctx *ctx, uint64_t n, const uint64_t *seg_bounds, int T);
