@@ -329,7 +329,7 @@ def main():
                                                    "that build the runs and evaluate the filter)"),
             "refilter": stage(float(sc["ms_filter"]), 2 * N, "filtered and BAD flags"),
             "union": stages["union"]}
-        roofline = {"bound": "lds", "kernel": "bin_runs_kernel (runs of equal k-mers in LDS tables, filter)",
+        roofline = {"bound": "valu", "kernel": "bin_runs_kernel (runs of equal k-mers in LDS tables, filter)",
                     "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS, "traffic": None,
                     "traffic_source": None, "bytes_per_launch": runs_bytes, "launch_ms": runs_ms, "tuples": n}
         sort = {"passes": passes, "by": "minimizer bins (no radix pass)", "algorithmic_bytes": runs_bytes, "ms": ms,

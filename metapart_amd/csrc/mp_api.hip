@@ -224,7 +224,7 @@ static uint64_t scan_tuple_room(mp_ctx *ctx)
     const uint64_t later_held = ctx->gparent.bytes + ctx->gsize.bytes + ctx->pairc.bytes + ctx->items[0].bytes +
                                 ctx->items[1].bytes + ctx->ilens[0].bytes + ctx->ilens[1].bytes + ctx->iaux[0].bytes +
                                 ctx->iaux[1].bytes + ctx->out.bytes;
-    // (measured: 48 B per read for the pair step, 66 B per read of items plus
+    // (64 B per read at most for the pair step, 12-16 B per read of items plus
     // the output for the writer; with the buffers' growth slack of 1/16)
     const uint64_t later_need = (128 * N + ctx->fq_bytes) / 16 * 17 + (1u << 20);
     const uint64_t reserve = later_need > later_held ? later_need - later_held : 0;

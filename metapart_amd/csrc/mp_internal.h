@@ -299,12 +299,12 @@ KeyLayout byte_layout();
 KeyLayout scan_layout(const mp_ctx *ctx);
 // kSortPasses x kSortRadix digit counts of the scan's tuples (host, passes of
 // pass_mask) and their number; fills *g for radix_sort_tuples.  all: the scan
-// holds every k-mer, so the counts of the last m-mer histogram serve.
+// holds every k-mer, so a batch's digit counts serve where there are any.
 int gen_histograms(mp_ctx *ctx, int s, uint64_t lo, uint64_t hi, uint32_t pass_mask, bool all, GenSource *g,
                    uint64_t *n_out);
 // Samples of a batch sorted each on its own (host arrays of ns + 1 entries):
 // sample s's tuples end up in [tpos[s], tpos[s+1]); the generating pass takes
-// its windows [wpos[s], wpos[s+1]) (and the m-mer histogram's per-tile digit
+// its windows [wpos[s], wpos[s+1]) (and count_batch_digits()'s per-tile digit
 // counts over tiles of each sample's windows).
 struct SortSegments {
     int ns = 0;

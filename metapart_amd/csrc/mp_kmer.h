@@ -185,7 +185,7 @@ struct GenSource {
     uint64_t h[kSortPasses * kSortRadix];     // digit counts of the tuples
     uint64_t npos;                            // k-mer windows of all reads
     // when set: digit counts of radix pass gcnt_pass per generating-pass tile
-    // ([tile][digit], from the m-mer histogram), so that pass needs no look-back
+    // ([tile][digit], a batch's digit counts), so that pass needs no look-back
     const uint32_t *gcnt = nullptr;
     uint64_t gcnt_tiles = 0;
     int gcnt_pass = -1;

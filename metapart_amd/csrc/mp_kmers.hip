@@ -1011,7 +1011,7 @@ int gen_histograms(mp_ctx *ctx, int s, uint64_t lo, uint64_t hi, uint32_t pass_m
     MP_HIP(hipMemcpyAsync(&g->npos, (const uint64_t *)ctx->pos_off.p + ctx->N, sizeof(uint64_t),
                           hipMemcpyDeviceToHost, ctx->stream));
     if (all && ctx->khist_valid && !(pass_mask & ~ctx->khist_mask)) {
-        // every k-mer is in the scan: the m-mer histogram counted these digits already
+        // every k-mer is in the scan: the batch's digit counts hold these already
         const int nc = ctx->khist_copies;
         std::vector<uint64_t> rep((size_t)nc * 8 * kSortRadix);
         MP_HIP(hipMemcpyAsync(rep.data(), ctx->khist.p, rep.size() * 8, hipMemcpyDeviceToHost, ctx->stream));

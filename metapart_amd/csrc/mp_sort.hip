@@ -1051,8 +1051,8 @@ int radix_sort_generic(mp_ctx *ctx, DevArray *keys, DevArray *lab, DevArray *adj
     std::vector<int> plist;
     for (int p = 0; p < kPasses; p++)
         if (run[p]) plist.push_back(p);
-    // the generating pass takes counted offsets too when the m-mer histogram
-    // counted its digits per tile (a scan over every k-mer, same tile size)
+    // the generating pass takes counted offsets too when its digits were counted
+    // per tile (a batch: a scan over every k-mer, same tile size)
     const bool gen_counted = counted && gen && gen->gcnt && gen_p == gen->gcnt_pass && gen->gcnt_tiles == gtiles &&
                              (ns > 0) == gen->gcnt_seg;
     if (ns > 0 && !gen_counted) return ctx->fail(MP_EINVAL, "a segmented sort takes counted offsets only");
