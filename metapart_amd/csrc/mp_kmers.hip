@@ -905,7 +905,7 @@ __global__ __launch_bounds__(kKBlock) void kmer_digit_hist_kernel(KParams P, uin
             for (int b = 0; b < 8; b++)
                 if ((pass_mask >> (b + 1)) & 1) atomicAdd(&h[b][kl.digit(canon, b)], 1u);
         };
-        if (staged) {  // two copies of the loop, as in hist_tile_kernel
+        if (staged) {  // two copies of the loop: no access tests which
             for_group_windows(
                 P.K, s_pref, s_base, nr, tid, kKBlock, [&](uint64_t w) -> uint64_t { return s_words[np + (w - wn0)]; },
                 [&](uint64_t w) -> uint64_t { return s_words[w - wp0]; }, body);
