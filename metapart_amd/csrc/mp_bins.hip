@@ -606,8 +606,11 @@ __global__ __launch_bounds__(kScThreads) void bin_scatter_kernel(KParams G, cons
 // ---------------------------------------------------------------- bins of a coarse bin
 // One workgroup per coarse bin: records and windows per cell in LDS, cells cut
 // into bins where the running window count passes a multiple of `aim`, the
-// records moved to their bin (a cursor per bin: a bin's records are written in
-// order, so its lines fill in L2).
+// records moved to their bin: where a lane can hold a bin's cursor (up to 1024
+// bins), in batches ordered by bin in LDS, so that what a batch holds of a bin
+// is written together (12 M reads 2.93 -> 2.43 ms, four scans of 2 M 1.29 ->
+// 1.16), else one by one.  Written were 2.3 times the bytes, as the bins' open
+// lines of an XCD's 32 workgroups are more than its cache.
 // PART: a record's windows are those in the bucket range.
 template <int NM, bool PART>
 __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict__ rec, const uint32_t *__restrict__ coarse,
@@ -617,8 +620,13 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
                                                          BinCtl *ctl)
 {
     constexpr int kPer = NM / 1024;
+    constexpr uint32_t kBatch = NM >= 8192 ? 4096 : 2048, kItems = kBatch / 1024;
+    constexpr size_t kRoom = (NM + 1) * sizeof(uint64_t) > kBatch * sizeof(uint4) ? (NM + 1) * sizeof(uint64_t) : kBatch * sizeof(uint4);
     __shared__ unsigned long long s_h[NM];  // records << 32 | windows per cell; then the cell's bin
-    __shared__ uint64_t s_st[NM + 1];       // first record << 32 | first window of every bin; then its cursor
+    __shared__ __align__(16) uint8_t s_room[kRoom];
+    __shared__ uint16_t s_bin[kBatch];
+    __shared__ uint32_t s_n[1024], s_at[1024], s_to[1024];
+    uint64_t *const s_st = (uint64_t *)s_room;  // first record << 32 | first window of every bin; then its cursor
     __shared__ uint64_t s_w[16];
     __shared__ uint32_t s_wb[16], s_place[2];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -749,6 +757,52 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
         }
     }
     __syncthreads();
+    if (nb <= 1024) {  // in batches ordered by bin
+        uint4 *const s_rec = (uint4 *)s_room;
+        uint32_t cur = tid < nb ? r0 + (uint32_t)(s_st[tid] >> 32) : 0u;
+        s_n[tid] = 0;
+        __syncthreads();
+        for (uint32_t q0 = 0; q0 < n; q0 += kBatch) {
+            uint4 x[kItems];
+            uint32_t at[kItems];  // bin | place in it << 10 (no record: ~0)
+#pragma unroll
+            for (uint32_t u = 0; u < kItems; u++) x[u] = rec[r0 + min(q0 + u * 1024 + tid, n - 1)];
+#pragma unroll
+            for (uint32_t u = 0; u < kItems; u++) {
+                at[u] = ~0u;
+                if (q0 + u * 1024 + tid >= n) continue;
+                const uint32_t bi = (uint32_t)s_h[(x[u].y >> 15) & cmask];
+                at[u] = bi | (atomicAdd(&s_n[bi], 1u) << 10);
+            }
+            __syncthreads();
+            const uint32_t mine = s_n[tid], inc2 = wave_incl(mine);
+            if (lane == kWave - 1) s_wb[wave] = inc2;
+            __syncthreads();
+            const uint32_t run2 = wave_incl(s_wb[lane % 16]), w = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+            const uint32_t first = inc2 - mine + (w ? (uint32_t)__builtin_amdgcn_readlane((int)run2, (int)w - 1) : 0u);
+            s_at[tid] = first;
+            s_to[tid] = cur - first;
+            cur += mine;
+            s_n[tid] = 0;
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < kItems; u++) {
+                if (at[u] == ~0u) continue;
+                const uint32_t bi = at[u] & 1023, p = s_at[bi] + (at[u] >> 10);
+                s_rec[p] = x[u];
+                s_bin[p] = (uint16_t)bi;
+            }
+            __syncthreads();
+            const uint32_t m = min(kBatch, n - q0);
+#pragma unroll
+            for (uint32_t u = 0; u < kItems; u++) {
+                const uint32_t p = u * 1024 + tid;
+                if (p < m) out[s_to[s_bin[p]] + p] = s_rec[p];
+            }
+            // (the next batch writes s_to, s_rec and s_bin only behind two more barriers)
+        }
+        return;
+    }
     uint32_t *const s_cur = (uint32_t *)s_st;  // word 2 i + 1 of entry i: its first record, counted up
     for (uint32_t i0 = tid; i0 < n; i0 += kU * 1024) {
         uint4 x[kU];
