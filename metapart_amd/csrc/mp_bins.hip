@@ -159,7 +159,12 @@ __device__ __forceinline__ void bin_of(uint32_t h, uint32_t nc, int cell_bits, u
 // (a branch per window and lane before: 920 -> 670 instructions a step; 12 M
 // reads 3.25 -> 2.56 ms).  The tiles' totals go to 64 copies of the counters:
 // 529 k reads 0.36 -> 0.15 ms, of which 40,000 atomics on one line were most.
-template <int M, int W>
+// A scan of part of the buckets makes only the records that hold a window in
+// them: in one scan of 64 that is every sixth, and what is left holds a window
+// at the least, so a bin of up to kBinRec windows never has more records than
+// bin_runs takes.
+// PART: the scan holds part of the buckets.
+template <int M, int W, bool PART>
 __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
 {
     __shared__ uint4 s_min[4][kWave][5];      // minimizer hashes of a lane's 16 windows (rows 80 bytes apart: no conflicts)
@@ -208,7 +213,7 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
     }
     const uint64_t nh = (P.total + 127) / 16;  // halves that the streams hold at the least
     uint32_t over = 0, nv = 0, nin = 0;
-    const uint32_t lo12 = P.lo << 12, span = P.inr ? (P.hi << 12) - lo12 : ~0u;  // of the top 16 bases
+    const uint32_t lo12 = P.lo << 12, span = PART ? (P.hi << 12) - lo12 : ~0u;  // of the top 16 bases
     uint32_t rec_total = 0;
     for (uint64_t ws = ws0; ws < ws1; ws++) {
         const uint64_t p0 = ws * kStepPos, h = p0 / 16 + lane;
@@ -289,11 +294,27 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
         uint32_t at = exc & 0xFFFF;
         const uint32_t nr = tot & 0xFFFF;
         const bool fits = nr <= kStepRec;
+        // the canonical k-mers' top 16 bases, by position; the windows in the bucket range
+        const uint32_t Y0 = rc32(X2), Y1 = rc32(X1), Y2 = rc32(X0);
+        const int zs = 2 * (33 - K);
+        const uint32_t Z0 = fun32(Y0, Y1, zs), Z1 = fun32(Y1, Y2, zs);
+        uint32_t I = 0xFFFF;
+        if constexpr (PART) {
+            I = 0;
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const uint32_t c = min(fun32(X0, X1, 2 * j), fun32(Z0, Z1, 2 * (15 - j)));
+                I = I + I + (c - lo12 < span ? 1u : 0u);
+            }
+            I &= Vo;
+            nin += (uint32_t)__popc(I);
+            if (lane < 60) P.inr[h ^ 3] = (uint16_t)I;
+        }
         if (!fits) over = 1;
         if (fits) {
 #pragma unroll
             for (int j = 0; j < 4; j++) s_min[wave][lane][j] = make_uint4(a[4 * j], a[4 * j + 1], a[4 * j + 2], a[4 * j + 3]);
-            s_lane[wave][lane] = make_uint4((stop << 16) | V, (pv << 16) | E, nxt | (nx7 << 8), exc >> 16);
+            s_lane[wave][lane] = make_uint4((stop << 16) | V, (pv << 16) | E, nxt | (nx7 << 8) | (PART ? I << 16 : 0u), exc >> 16);
             for (uint32_t m = S; m;) {
                 const uint32_t j = (uint32_t)__builtin_clz(m) - 16;
                 m ^= 0x8000u >> j;
@@ -301,12 +322,8 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
             }
         }
         wave_lds_fence();
-        if (lane == 0) {
-            P.nrec[ws] = fits ? nr : 0u;
-            P.erank[ws] = (uint32_t)rank;
-        }
+        uint32_t kept = fits && !PART ? nr : 0u;  // records with a window in range (counted below, by lane 0 in whole)
         if (fits) {
-            rec_total += nr;
             uint64_t *out = P.desc + ws * kStepRec;
             for (uint32_t i = lane; i < nr; i += kWave) {
                 const uint32_t o = s_start[wave][i], j = o & 15;
@@ -314,7 +331,16 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
                 const uint32_t hash = ((const uint32_t *)s_min[wave][o >> 4])[j];
                 const uint32_t qs = q.x >> 16, qv = q.x & 0xFFFF, rest = qs & ((0x8000u >> j) - 1);
                 const uint32_t end = rest ? (uint32_t)__builtin_clz(rest) - 16 : 16 + (q.z & 31);  // past its last window
-                const uint32_t n7 = rest ? ((qv >> (15 - end)) & 1 ? 0u : kNextN) : q.z >> 8;
+                uint32_t to = i;
+                if constexpr (PART) {  // a record without a window in range is left out (it ends in its lane or the next)
+                    const uint32_t in = ((q.z & 0xFFFF0000u) | (s_lane[wave][(o >> 4) + 1].z >> 16)) << j;
+                    const bool keep = in >> (32 - (end - j));
+                    const uint64_t m = __ballot(keep);
+                    to = kept + (uint32_t)__popcll(m & lanemask_lt());
+                    kept += (uint32_t)__popcll(m);
+                    if (!keep) continue;
+                }
+                const uint32_t n7 = rest ? ((qv >> (15 - end)) & 1 ? 0u : kNextN) : (q.z >> 8) & 3;
                 const uint32_t p7 = (q.y >> (31 - j)) & 1 ? 0u : kPrevN;
                 const uint32_t rk = q.w + (uint32_t)__popc((q.y & 0xFFFF) >> (15 - j));
                 const uint32_t misc = o | ((end - j) << 10) | ((p7 | n7) << 15) | (rk << 17);
@@ -329,36 +355,26 @@ __global__ __launch_bounds__(256, 4) void bin_scan_kernel(BinScan P)
                 bin_of(hash, nc, P.cell_bits, coarse, cell);
                 coarse += c0;
                 atomicAdd(&s_cnt[coarse], 1u);
-                out[i] = (uint64_t)misc | ((uint64_t)coarse << 32) | ((uint64_t)cell << 42);
+                out[to] = (uint64_t)misc | ((uint64_t)coarse << 32) | ((uint64_t)cell << 42);
             }
+        }
+        rec_total += kept;
+        if (lane == 0) {
+            P.nrec[ws] = kept;
+            P.erank[ws] = (uint32_t)rank;
         }
         // the largest k-mer of every segment: the top 16 bases first, the whole
         // k-mer only where they reach the largest seen
         {
             const int sh = 2 * K - 32;
-            const uint32_t Y0 = rc32(X2), Y1 = rc32(X1), Y2 = rc32(X0);
-            const int zs = 2 * (33 - K);
-            const uint32_t Z0 = fun32(Y0, Y1, zs), Z1 = fun32(Y1, Y2, zs);
             uint32_t cand = 0;
             if (!batch) {
                 nv += (uint32_t)__popc(Vo);
-                uint32_t I = 0xFFFF;
-                if (P.inr) {
-                    I = 0;
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        const uint32_t c = min(fun32(X0, X1, 2 * j), fun32(Z0, Z1, 2 * (15 - j)));
-                        I = I + I + (c - lo12 < span ? 1u : 0u);
-                    }
-                    I &= Vo;
-                    nin += (uint32_t)__popc(I);
-                    if (lane < 60) P.inr[h ^ 3] = (uint16_t)I;
-                }
                 cand = I;
             }
             if (P.T == 1 && !batch) {
                 const unsigned long long m1 = s_max[0];
-                const uint32_t thr = m1 ? (uint32_t)((m1 - 1) >> sh) : 0u, top = P.inr ? lo12 + span - thr : 0u - thr;
+                const uint32_t thr = m1 ? (uint32_t)((m1 - 1) >> sh) : 0u, top = PART ? lo12 + span - thr : 0u - thr;
                 // [thr, end of the range); thr = 0 (nothing seen yet) or the end at 2^32: all from thr on
                 bool any = false;
 #pragma unroll
@@ -1588,7 +1604,8 @@ __global__ __launch_bounds__(256) void bin_alive_kernel(const uint8_t *__restric
 template <int M, int W>
 static void launch_scan(mp_ctx *ctx, uint32_t tiles, const BinScan &P)
 {
-    hipLaunchKernelGGL((bin_scan_kernel<M, W>), dim3(tiles), dim3(256), 0, ctx->stream, P);
+    auto *const kernel = P.inr ? bin_scan_kernel<M, W, true> : bin_scan_kernel<M, W, false>;
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(256), 0, ctx->stream, P);
 }
 
 // M-mers of 13 bases (33 M canonical values, far more than there are cells);

@@ -51,6 +51,16 @@ def test_scans_and_segments_equal_radix(S, T):
 
 
 @pytest.mark.gpu
+def test_many_scans_keep_to_the_bins_table():
+    # 32 scans of 150 k shallow reads: a record holds a third of a window in the scan's range, and without those
+    # that hold none every bin fits bin_runs
+    print("gpu bins, 32 scans", flush=True)
+    buf = mp.synth(0, n_reads=150000, seed=78, read_len=150, n_genomes=40, genome_len_min=500000, genome_len_max=1000000)
+    a = _same(buf, 32, 31, 32, 1)
+    assert [s["sort_long_groups"] for s in a.scans] == [0] * 32
+
+
+@pytest.mark.gpu
 def test_records_at_read_and_step_ends():
     # reads of k - 1 .. k + 2 bases and of every length around a step's 960
     # positions, 'N' first, last, beside and between windows
