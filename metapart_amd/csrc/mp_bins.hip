@@ -53,6 +53,7 @@ constexpr uint32_t kBinRec = 1024;  // records of such a bin
 constexpr uint32_t kBinAim = kBinCap * 3 / 4;  // windows per bin aimed at, at most (fewer where records hold few)
 constexpr int kRunThreads = 1024;
 constexpr uint64_t kRunGrid = 1ull << 21;  // bins of a dispatch of bin_runs: fewer than 2^32 threads
+constexpr int kBigRec = 64;         // records that bin_runs_big expands at once
 constexpr int kBinWit = 8;          // witnesses per bin (bin_runs)
 constexpr int kMaxSeg = 256;        // segments (samples of a batch)
 constexpr int kStripes = 64;        // copies of the global counters, a cache line each
@@ -74,8 +75,10 @@ struct BinCtl {  // device counters of a scan, cleared before it
     unsigned long long nvalid[kMaxSeg];  // windows without 'N' per sample of a batch
     unsigned long long kmax1[kMaxSeg];   // 1 + the largest k-mer of every segment (0: none)
     unsigned long long out;              // labels written (64-aligned per bin)
-    unsigned long long big_win, big_max; // windows of the big bins: all, the largest
+    unsigned long long big_win;          // windows of the big bins
+    unsigned long long big_grp, big_most; // groups of kBigRec of their records: all, the largest bin's
     uint32_t nbin, nbig, err;
+    uint32_t next[2];                    // bin_runs_big, and its CHECK: bins taken
     uint32_t pad;
     uint32_t found[kMaxSeg];             // live labels seen in the last segment (of the sample): kFoundOther, kFoundLast
     unsigned long long stat[kStripes][16];  // [0] runs, [1] zeroed; of bin_scan [2] records, [3] windows, [4] of them in range
@@ -768,8 +771,10 @@ __global__ __launch_bounds__(1024) void bin_group_kernel(const uint4 *__restrict
         if (large) {
             const uint32_t q = al + (uint32_t)__popcll(ml & lanemask_lt());
             if (q < big_cap) big[q] = d;
+            const unsigned long long groups = (d.nrec + kBigRec - 1) / kBigRec;
             atomicAdd(&ctl->big_win, (unsigned long long)d.nwin);
-            atomicMax(&ctl->big_max, (unsigned long long)d.nwin);
+            atomicAdd(&ctl->big_grp, groups);
+            atomicMax(&ctl->big_most, groups);
         }
     }
     __syncthreads();
@@ -840,7 +845,6 @@ struct BinRuns {
     const BinDesc *bins;
     uint32_t nbin;
     int K;
-    uint32_t lo, hi;          // bucket range
     int T, batch;
     const uint32_t *bounds;   // T + 1 bucket boundaries (plain)
     uint32_t last_lo;         // first bucket of the last segment that holds tuples
@@ -850,6 +854,7 @@ struct BinRuns {
     uint64_t *st_bits;        // run starts among them (zero before)
     uint64_t out_cap;         // labels that lab_out holds
     uint32_t *wit;            // kBinWit labels per bin (~0: none)
+    uint64_t big_work;        // groups that a workgroup of bin_runs_big may visit
     BinCtl *ctl;
 };
 
@@ -857,13 +862,11 @@ struct BinRuns {
 struct Window {
     uint64_t key;
     uint32_t cls;   // in class | out class << 3 (0-3, 7 'N')
-    bool in;        // inside the bucket range
 };
 
 // K bases and their neighbours from the 64 staged bases (index 0: the base
 // before the record's first window), window o of the record
-__device__ __forceinline__ Window expand(uint64_t hi, uint64_t lo, uint32_t o, bool p7, bool n7, int K, uint32_t blo,
-                                         uint32_t bhi)
+__device__ __forceinline__ Window expand(uint64_t hi, uint64_t lo, uint32_t o, bool p7, bool n7, int K)
 {
     const uint64_t y = (hi << (2 * o)) | ((lo >> 1) >> (63 - 2 * o));
     const uint32_t pc = (uint32_t)(y >> 62);
@@ -878,8 +881,6 @@ __device__ __forceinline__ Window expand(uint64_t hi, uint64_t lo, uint32_t o, b
     const uint32_t cp = p7 ? 7u : pc ^ (pc >> 1), cn = n7 ? 7u : nc ^ (nc >> 1);
     const uint32_t rp = p7 ? 7u : cp ^ 2, rn = n7 ? 7u : cn ^ 2;
     w.cls = fwd ? cn | (cp << 3) : rp | (rn << 3);
-    const uint32_t b = (uint32_t)(w.key >> (2 * K - 20));
-    w.in = b >= blo && b < bhi;
     return w;
 }
 
@@ -1318,16 +1319,34 @@ __global__ __launch_bounds__(kRunThreads, 8) void bin_runs_kernel(BinRuns P)
     }
 }
 
-// A bin past the table: its windows in parts by the top bits of the k-mer's
-// hash, a part split again when its k-mers overfill the table; the windows of
-// a part go by once to count, once to place the labels and tally the branching
-// sides and once to mark (records expanded again each time, kBigRec at once).
-constexpr int kBigThreads = 1024, kBigRec = 64;
+// A bin past the table.  Its windows go by once to count, once to place the
+// labels and tally the branching sides and once to mark (records expanded again
+// each time, kBigRec at once), whole where its distinct k-mers fit the table, as
+// in a pile of few k-mers however deep, else in parts by the top bits of the
+// k-mer's hash, a part split again when its k-mers overfill the table.
+// A bin of many k-mers is visited once per part, which grows with its square:
+// at the first overfull table the groups still to come are reckoned from the
+// k-mers seen so far, and where they would pass P.big_work, or once a workgroup
+// has visited so many, the scan goes by radix passes instead.
+// PART: a record's windows in the bucket range alone are expanded.
+constexpr int kBigThreads = 1024;
 constexpr uint32_t kBigKeys = 2048;   // k-mers of a part; a group of records adds at most 64 x 31, which still fit
+constexpr uint32_t kBigPart = kBigKeys * 3 / 4;  // and on average
 constexpr int kBigDepth = 24;
+constexpr int kBigGrid = 256;         // workgroups, one a CU; each takes the next bin
+// What bin_runs_big may take is what the radix path does: a window of 25e6 in a
+// ms, and of those in large bins, whose k-mers of thousands of copies it sorts
+// group by group and evaluates by one lane, 200e3 at the most (measured 44e3
+// where 40 k reads are of one 500 bp genome, 15e3 for 100 k of 5 kb, 117e3 where
+// 2 % of 60 k reads are poly-G, 171e3 for 40 k amplicons with 200 pairs of
+// flanks).  A visit of a group takes 2.0 to 2.7 us.  Against radix passes
+// these take 93 -> 3.7, 803 -> 0.8 and 41 -> 1.2 ms; the amplicons (the table overfull
+// at once) go on to the radix path after 0.3.
+constexpr double kBigGroupMs = 0.0025;
+constexpr double kRadixWin = 25e6, kRadixDeep = 200e3;
 static_assert(kBigKeys + kBigRec * kMaxRun < kBinCap, "the table never fills");
 
-template <bool CHECK>
+template <bool CHECK, bool PART>
 __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
 {
     constexpr int kPer = kBinCap / kBigThreads;
@@ -1336,49 +1355,56 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
     __shared__ uint32_t s_cnt[kBinCap], s_meta[kBinCap], s_base[kBinCap];
     __shared__ uint32_t s_tal[kBigKeys + kBigRec * kMaxRun][4];
     __shared__ ulonglong2 s_seq[kBigRec];
-    __shared__ uint32_t s_lab[kBigRec], s_fl[kBigRec], s_off[kBigRec + 1];
-    __shared__ uint8_t s_map[kBigRec * kMaxRun + 1];
-    __shared__ uint32_t s_nkey, s_sumc[kWaves], s_sums[kWaves], s_red[2];
+    __shared__ uint32_t s_lab[kBigRec], s_fl[kBigRec];
+    __shared__ uint16_t s_map[kBigRec * kMaxRun];  // window: its record | its place in it << 6
+    __shared__ uint32_t s_nwin, s_nkey, s_bin, s_stop, s_sumc[kWaves], s_sums[kWaves], s_red[2];
     __shared__ uint64_t s_out;
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int K = P.K;
-    for (uint32_t bin = blockIdx.x; bin < P.nbin; bin += gridDim.x) {
+    uint64_t work = 0;  // groups visited
+    for (;;) {
+        __syncthreads();
+        if (tid == 0) s_bin = atomicAdd(&P.ctl->next[CHECK ? 1 : 0], 1u);
+        __syncthreads();
+        const uint32_t bin = s_bin;
+        if (bin >= P.nbin) break;
         const BinDesc d = P.bins[bin];
         if (tid < 2) s_red[tid] = 0;
-        // the windows of records [g, g + kBigRec) of the part, fn(window, label, slot valid) per lane
+        // the windows of records [g, g + kBigRec) of the part, fn(window, label, hash) per lane
         auto group = [&](uint32_t g, auto fn) {
             __syncthreads();
             const uint32_t nr = min((uint32_t)kBigRec, d.nrec - g);
             if (tid < kBigRec) {  // one wave
-                uint32_t L = 0;
+                uint32_t m = 0;  // its windows to expand, the first at bit 31
                 if (tid < nr) {
                     const uint4 rc = P.rec[d.rec0 + g + tid];
                     uint64_t hi, lo;
                     bases64(P.packed, (((uint64_t)rc.y << 32) | rc.x) & ((1ull << 40) - 1), hi, lo);
+                    const uint32_t L = (rc.y >> 8) & 31;
                     s_seq[tid] = make_ulonglong2(hi, lo);
                     s_lab[tid] = rc.z;
-                    s_fl[tid] = (rc.y >> 13) & 3;
-                    L = (rc.y >> 8) & 31;
+                    s_fl[tid] = ((rc.y >> 13) & 3) | (L << 2);
+                    m = (PART ? rc.w : ~0u) << (32 - L);
                 }
-                const uint32_t i = wave_incl(L);
-                s_off[tid] = i - L;
-                if (tid == kBigRec - 1) s_off[kBigRec] = i;
-                for (uint32_t o = i - L; o < i; o++) s_map[o] = (uint8_t)tid;
+                const uint32_t n = (uint32_t)__popc(m), i = wave_incl(n);
+                if (tid == kBigRec - 1) s_nwin = i;
+                for (uint32_t o = i - n; m; o++) {
+                    const uint32_t q = (uint32_t)__builtin_clz(m);
+                    m &= ~(0x80000000u >> q);
+                    s_map[o] = (uint16_t)(tid | (q << 6));
+                }
             }
             __syncthreads();
-            const uint32_t nw = s_off[kBigRec];
+            const uint32_t nw = s_nwin;
             for (uint32_t j = tid; j < nw; j += kBigThreads) {
-                const uint32_t r = s_map[j], o = j - s_off[r];
-                const bool last = j + 1 == s_off[r + 1];
+                const uint32_t e = s_map[j], r = e & 63, o = e >> 6, fl = s_fl[r];
                 const ulonglong2 sq = s_seq[r];
-                const Window x = expand(sq.x, sq.y, o, o == 0 && (s_fl[r] & kPrevN), last && (s_fl[r] & kNextN), K, P.lo,
-                                        P.hi);
-                if (x.in) fn(x, s_lab[r], key_hash(x.key));
+                const Window x = expand(sq.x, sq.y, o, o == 0 && (fl & kPrevN), o + 1 == fl >> 2 && (fl & kNextN), K);
+                fn(x, s_lab[r], key_hash(x.key));
             }
+            work++;
         };
         int depth = 0;
-        while ((d.nwin >> depth) > 2 * kBinCap) depth++;
-        const int depth0 = depth;
         uint32_t part = 0;
         for (;;) {
             auto mine = [&](uint32_t h) { return depth == 0 || (h * 0x9E3779B1u) >> (32 - depth) == part; };
@@ -1389,8 +1415,11 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
                 s_cnt[q * kBigThreads + tid] = 0;
                 s_meta[q * kBigThreads + tid] = 0;
             }
-            if (tid == 0) s_nkey = 0;
-            bool over = false;
+            if (tid == 0) {
+                s_nkey = 0;
+                s_stop = ld_agent(&P.ctl->err);  // another workgroup gave up
+            }
+            uint32_t seen_grp = 0;  // groups up to the one that overfilled the table
             for (uint32_t g = 0; g < d.nrec; g += kBigRec) {
                 group(g, [&](const Window &x, uint32_t, uint32_t h) {
                     if (!mine(h)) return;
@@ -1404,12 +1433,24 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
                         atomicOr(&s_meta[s], seen);
                 });
                 __syncthreads();
-                if (s_nkey > kBigKeys) {  // uniform: read after the barrier, next written after another
-                    over = true;
+                // uniform: s_stop is written before the part's first barrier, s_nkey next behind another
+                if (s_stop) return;
+                if (s_nkey > kBigKeys) {
+                    seen_grp = g / kBigRec + 1;
                     break;
                 }
+                if (work > P.big_work) break;
             }
-            if (over) {
+            uint64_t todo = work;
+            if (seen_grp && depth == 0) {  // parts by the k-mers seen per group, three visits of all groups each
+                const uint64_t all = (d.nrec + kBigRec - 1) / kBigRec;
+                todo += all * 3 * ((uint64_t)s_nkey * all / ((uint64_t)seen_grp * kBigPart) + 1);
+            }
+            if (todo > P.big_work) {  // uniform
+                if (tid == 0) atomicOr(&P.ctl->err, 16u);
+                return;
+            }
+            if (seen_grp) {
                 if (depth == kBigDepth) {  // one hash value holds too many k-mers: the radix path
                     if (tid == 0) atomicOr(&P.ctl->err, 4u);
                     return;
@@ -1551,17 +1592,13 @@ __global__ __launch_bounds__(kBigThreads) void bin_runs_big_kernel(BinRuns P)
                 }
             }
             // the next part: up from every right half, then the right sibling
-            while (depth > depth0 && (part & 1)) {
+            while (depth && (part & 1)) {
                 part >>= 1;
                 depth--;
             }
-            if (depth == depth0) {
-                if (++part >> depth0) break;
-            } else {
-                part |= 1;
-            }
+            if (!depth) break;
+            part |= 1;
         }
-        __syncthreads();
     }
 }
 
@@ -1839,9 +1876,10 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     MP_HIP(hipStreamSynchronize(ctx->stream));
     const uint64_t nbin = hc->nbin, nbig = hc->nbig;
     if (hc->err || nbin > bin_cap || nbig > bin_cap) return 0;
-    // windows piled up in a few bins keep few workgroups busy: about 0.5 M
-    // windows a ms and workgroup against 25 M a ms for the radix path
-    if (std::max(hc->big_max / 0.5e6, hc->big_win / (256 * 0.5e6)) > nv / 25e6 + 0.5) return 0;
+    // what bin_runs_big may take, and its three visits of every group at the least
+    const double big_ms = nv / kRadixWin + hc->big_win / kRadixDeep + 0.5;
+    const uint64_t big_work = (uint64_t)(big_ms / kBigGroupMs);
+    if (3 * std::max<uint64_t>(hc->big_most, hc->big_grp / kBigGrid) > big_work) return 0;
     // labels of the runs to join: every bin's (and every part's of a big bin) padded to whole bitmap words
     const uint64_t out_cap = nv + 64 * nbin + 256 * nbig + hc->big_win / 8 + 4096;
     MP_ROOM(ensure(ctx, ctx->lab[0], out_cap * sizeof(uint32_t)));
@@ -1853,8 +1891,6 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     R.packed = (const uint64_t *)ctx->packed.p;
     R.rec = rec_b;
     R.K = K;
-    R.lo = lo;
-    R.hi = batch ? (uint32_t)MP_NBUCKETS : hi;
     R.T = T;
     R.batch = batch ? 1 : 0;
     R.bounds = d_bnd;
@@ -1880,10 +1916,13 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
         R.bins = d_big;
         R.nbin = (uint32_t)nbig;
         R.wit = d_wit + nbin * kBinWit;
-        const unsigned gb = (unsigned)std::min<uint64_t>(nbig, 2048);
-        if (nbig && check) hipLaunchKernelGGL(bin_runs_big_kernel<true>, dim3(gb), dim3(kBigThreads), 0, ctx->stream, R);
-        if (nbig && !check) hipLaunchKernelGGL(bin_runs_big_kernel<false>, dim3(gb), dim3(kBigThreads), 0, ctx->stream, R);
-        MP_HIP(hipGetLastError());
+        R.big_work = check ? ~0ull : big_work;  // (a check repeats the first visits)
+        if (nbig) {
+            auto *const kernel = check ? (part ? bin_runs_big_kernel<true, true> : bin_runs_big_kernel<true, false>)
+                                       : (part ? bin_runs_big_kernel<false, true> : bin_runs_big_kernel<false, false>);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<uint64_t>(nbig, kBigGrid)), dim3(kBigThreads), 0, ctx->stream, R);
+            MP_HIP(hipGetLastError());
+        }
         return 0;
     };
     hipEventRecord(ctx->pev[2], ctx->stream);

@@ -105,6 +105,48 @@ def test_bins_past_the_table_and_a_few_live_reads():
     _same(np.concatenate([np.frombuffer(deep.tobytes(), dtype=np.uint8), live]), 1, 31, 1, 1, bins=None)
 
 
+def _poly_g(n, err, seed):
+    rng = np.random.default_rng(seed)
+    seqs = []
+    for _ in range(n):
+        x = np.full(150, ord("G"), dtype=np.uint8)
+        e = rng.random(150) < err
+        x[e] = np.frombuffer(b"ACGT", dtype=np.uint8)[rng.integers(0, 4, int(e.sum()))]
+        seqs.append(x.tobytes().decode())
+    return _fastq(seqs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(1, 1), (2, 3)])
+@pytest.mark.parametrize("deep", [False, True])
+def test_piled_up_bins(deep, S, T):
+    # a bin of many windows and few k-mers is visited a few times, not once per so many windows: 2 % poly-G reads
+    # among others, and a 500 bp genome at 12000x, take less than a quarter of the radix path's time
+    print("gpu bins piled up", deep, S, T, flush=True)
+    if deep:
+        buf = mp.synth(0, n_reads=40000, n_genomes=1, genome_len_min=500, genome_len_max=500, read_len=150,
+                       err_rate=0.01, seed=22)
+    else:
+        buf = np.concatenate([np.frombuffer(mp.synth(0, n_reads=60000, read_len=150, seed=8).tobytes(), dtype=np.uint8),
+                              _poly_g(1200, 0.003, 8)])
+    a = _same(buf, 6, 31, S, T)
+    b, _, _ = _run(buf, 6, 31, S, T, sort_digit_bits=7)
+    assert all(s["sort_long_groups"] > 0 for s in a.scans)
+    ms = [sum(s[f] for s in r.scans for f in ("ms_enumerate", "ms_sort", "ms_filter")) for r in (a, b)]
+    assert ms[0] < ms[1] / 4, ms
+
+
+@pytest.mark.gpu
+def test_a_pile_of_distinct_kmers_goes_to_the_radix_path():
+    # every read holds the 13-mer of the lowest minimizer hash between random bases: one bin of 266 k windows, as many k-mers
+    print("gpu bins pile of distinct k-mers", flush=True)
+    rng = np.random.default_rng(3)
+    mer = "".join("ACGT"[(0x2545F49 >> (24 - 2 * i)) & 3] for i in range(13))
+    bases = np.frombuffer(b"ACGT", dtype=np.uint8)[rng.integers(0, 4, (14000, 137))]
+    seqs = [r[:60].tobytes().decode() + mer + r[60:].tobytes().decode() for r in bases]
+    _same(_fastq(seqs), 2, 31, 1, 1, bins=False)
+
+
 @pytest.mark.gpu
 def test_other_letters_take_the_radix_path():
     print("gpu bins letters", flush=True)
