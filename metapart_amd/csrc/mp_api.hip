@@ -1,5 +1,6 @@
 // C-ABI entry points of libmetapart_amd (declared in include/metapart_amd.h).
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
@@ -209,32 +210,75 @@ int mp_load_reads_device(mp_ctx *ctx, const void *d_fq, uint64_t nbytes, const u
 // digit bytes and count tables, and the growth slack of the buffers.
 constexpr uint64_t kScanBytesPerTuple = 31;
 
-// Tuples a scan can hold within the budget: the bytes not held by anything
-// else, less a label snapshot and the room the pair step and the writer will
-// need, over kScanBytesPerTuple (MP_SCAN_PART_TUPLES lowers it, for tests).
-static uint64_t scan_tuple_room(mp_ctx *ctx)
+// the buffers of a scan's tuples
+static std::array<DevArray *, 11> tuple_arrays(mp_ctx *ctx)
 {
-    const uint64_t N = ctx->N;
-    const uint64_t tuple_held = ctx->keys[0].bytes + ctx->keys[1].bytes + ctx->lab[0].bytes + ctx->lab[1].bytes +
-                                ctx->adj[0].bytes + ctx->adj[1].bytes + ctx->zbits.bytes + ctx->runbits.bytes +
-                                ctx->dig.bytes + ctx->rts.bytes +
-                                ctx->status.bytes;
-    const uint64_t other = ctx->held - tuple_held;
-    const uint64_t label_bytes = ctx->labsnap.bytes ? 0 : N * sizeof(uint32_t) + 64;
+    return {{&ctx->keys[0], &ctx->keys[1], &ctx->lab[0], &ctx->lab[1], &ctx->adj[0], &ctx->adj[1], &ctx->zbits, &ctx->runbits,
+            &ctx->dig, &ctx->rts, &ctx->status}};
+}
+
+// the room that the pair step and the writer will need beyond what they hold
+static uint64_t later_room(const mp_ctx *ctx)
+{
     const uint64_t later_held = ctx->gparent.bytes + ctx->gsize.bytes + ctx->pairc.bytes + ctx->items[0].bytes +
                                 ctx->items[1].bytes + ctx->ilens[0].bytes + ctx->ilens[1].bytes + ctx->iaux[0].bytes +
                                 ctx->iaux[1].bytes + ctx->out.bytes;
     // (64 B per read at most for the pair step, 12-16 B per read of items plus
     // the output for the writer; with the buffers' growth slack of 1/16)
-    const uint64_t later_need = (128 * N + ctx->fq_bytes) / 16 * 17 + (1u << 20);
-    const uint64_t reserve = later_need > later_held ? later_need - later_held : 0;
+    const uint64_t later_need = (128 * ctx->N + ctx->fq_bytes) / 16 * 17 + (1u << 20);
+    return later_need > later_held ? later_need - later_held : 0;
+}
+
+// Bytes a scan's tuples can take within the budget: those not held by anything
+// else, less a label snapshot and the room the pair step and the writer will need.
+static uint64_t scan_byte_room(mp_ctx *ctx)
+{
+    uint64_t tuple_held = 0;
+    for (const DevArray *a : tuple_arrays(ctx)) tuple_held += a->bytes;
+    const uint64_t other = ctx->held - tuple_held;
+    const uint64_t label_bytes = ctx->labsnap.bytes ? 0 : ctx->N * sizeof(uint32_t) + 64;
     // the generating pass's look-back status covers every k-mer window, not only the scan's
     const uint64_t npos_status = ctx->total_bases / 16;
-    const uint64_t fixed = other + label_bytes + reserve + npos_status;
-    const uint64_t avail = ctx->budget > fixed ? ctx->budget - fixed : 0;
-    uint64_t cap = avail / kScanBytesPerTuple;
+    const uint64_t fixed = other + label_bytes + later_room(ctx) + npos_status;
+    return ctx->budget > fixed ? ctx->budget - fixed : 0;
+}
+
+// Tuples: over kScanBytesPerTuple (MP_SCAN_PART_TUPLES lowers it, for tests).
+static uint64_t scan_tuple_room(mp_ctx *ctx)
+{
+    uint64_t cap = scan_byte_room(ctx) / kScanBytesPerTuple;
     if (const char *e = getenv("MP_SCAN_PART_TUPLES")) cap = std::min<uint64_t>(cap, strtoull(e, nullptr, 10));
     return cap;
+}
+
+// A scan by minimizer bins holds other buffers than the radix passes, larger
+// ones where it holds few of the k-mers.  What they hold is dead after it (a
+// dump sorts the tuples anew), so they go where the budget is short: before the
+// radix path that takes a scan over, or a dump, if n tuples would not fit beside
+// what they have beyond those, and before the pair step and the writer.
+static int release_scan_buffers(mp_ctx *ctx)
+{
+    MP_HIP(hipStreamSynchronize(ctx->stream));
+    for (DevArray *a : tuple_arrays(ctx))
+        if (a != &ctx->status) release(ctx, *a);  // (its epochs go on)
+    release(ctx, ctx->binctl);
+    release(ctx, ctx->rstart);
+    ctx->rstart_valid = false;
+    return 0;
+}
+
+static int room_for_tuples(mp_ctx *ctx, uint64_t n)
+{
+    const uint64_t need[] = {8 * n, 8 * n, 4 * n, 4 * n, n, n, n / 8, n / 4, n, n / 4, n / 4};
+    uint64_t beyond = 0;
+    const auto arrays = tuple_arrays(ctx);
+    for (size_t i = 0; i < arrays.size(); i++) beyond += arrays[i]->bytes > need[i] ? arrays[i]->bytes - need[i] : 0;
+    return kScanBytesPerTuple * n + beyond <= scan_byte_room(ctx) ? 0 : release_scan_buffers(ctx);
+}
+
+static int room_for_later(mp_ctx *ctx)
+{
+    return !ctx->dump_lazy || ctx->held + later_room(ctx) <= ctx->budget ? 0 : release_scan_buffers(ctx);
 }
 
 // The two-sweep scan: bucket parts of at most cap tuples, cut where the
@@ -366,6 +410,7 @@ int mp_scan(mp_ctx *ctx, int s, uint64_t lo, uint64_t hi, const uint64_t *seg_bo
             return 0;
         }
         memset(&st, 0, sizeof(st));
+        MP_TRY(room_for_tuples(ctx, expected_tuples ? expected_tuples : n));
     }
     // every k-mer: the first radix pass generates the tuples from the reads;
     // 3-minimizer k-mers (a per-read window state machine) are enumerated
@@ -411,6 +456,7 @@ int mp_finish(mp_ctx *ctx, uint64_t *W, mp_finish_stats *stats)
     MP_HIP(hipSetDevice(ctx->device));
     mp_finish_stats st;
     memset(&st, 0, sizeof(st));
+    MP_TRY(room_for_later(ctx));
     MP_TRY(finish_components(ctx, W, &st));
     if (stats) *stats = st;
     ctx->finished = true;
@@ -646,6 +692,7 @@ int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_s
         job.T = ns;
         job.first = ctx->chunk_ids.data();
         MP_TRY(bins_scan(ctx, job, &st, &tpos, &n, &done));
+        if (!done) MP_TRY(room_for_tuples(ctx, n));
     }
     if (!done) {
         memset(&st, 0, sizeof(st));
@@ -682,6 +729,7 @@ int mp_batch_partition(mp_ctx *ctx, mp_sample_result *res, mp_scan_stats *scan_s
     mp_finish_stats fs;
     memset(&fs, 0, sizeof(fs));
     uint64_t W[MP_NPART + 1];
+    MP_TRY(room_for_later(ctx));
     MP_TRY(finish_components(ctx, W, &fs));
     ctx->finished = true;
     if (res) {
@@ -718,6 +766,7 @@ int mp_batch_write(mp_ctx *ctx, const char *out_dir, uint64_t *bytes_out)
     if (!ctx) return MP_EINVAL;
     if (!ctx->batch || !ctx->finished) return ctx->fail(MP_ESTATE, "no partitioned batch");
     MP_HIP(hipSetDevice(ctx->device));
+    MP_TRY(room_for_later(ctx));
     return write_partitions(ctx, out_dir, 1, nullptr, nullptr, bytes_out);
 }
 
@@ -728,6 +777,7 @@ int mp_write_partitions(mp_ctx *ctx, const char *out_prefix, int T, const uint64
     if (!ctx->finished) return ctx->fail(MP_ESTATE, "mp_write_partitions before mp_finish");
     if (ctx->C % T) return ctx->fail(MP_EINVAL, "T must divide the chunk count");
     MP_HIP(hipSetDevice(ctx->device));
+    MP_TRY(room_for_later(ctx));
     return write_partitions(ctx, out_prefix, T, W, il_start, bytes_out);
 }
 

@@ -1707,6 +1707,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     uint64_t npos = 0;  // windows, those with 'N' too
     MP_HIP(hipMemcpyAsync(&npos, (const uint64_t *)ctx->pos_off.p + N, sizeof(npos), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
+    *n_out = npos;
     const uint64_t desc_bytes = nsteps * kStepRec * sizeof(uint64_t);
     if (npos == 0 || (desc_bytes > key_room(npos) && desc_bytes > (64ull << 20))) return 0;  // mostly reads without windows
     // wave steps per wave: about 8192 tiles (their table of counts stays small), at least one step
@@ -1746,12 +1747,14 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     const bool ranged = !batch && !(lo == 0 && hi == MP_NBUCKETS);
     if (ranged) MP_ROOM(ensure(ctx, ctx->adj[1], nsteps * (kStepPos / 8) + 64));
     // a small scan holds the radix path's tuple buffers too, so that falling back to it, or a dump, allocates nothing
-    if (npos <= (1ull << 24))
+    if (npos <= (1ull << 24)) {
+        const uint64_t n = job.expected ? std::min(job.expected, npos) : npos;
         for (int b = 0; b < 2; b++) {
-            MP_ROOM(ensure(ctx, ctx->keys[b], (npos + 1) * sizeof(uint64_t)));
-            MP_ROOM(ensure(ctx, ctx->lab[b], (npos + 1) * sizeof(uint32_t)));
-            MP_ROOM(ensure(ctx, ctx->adj[b], npos + 16));
+            MP_ROOM(ensure(ctx, ctx->keys[b], (n + 1) * sizeof(uint64_t)));
+            MP_ROOM(ensure(ctx, ctx->lab[b], (n + 1) * sizeof(uint32_t)));
+            MP_ROOM(ensure(ctx, ctx->adj[b], n + 16));
         }
+    }
     uint8_t *const tb0 = (uint8_t *)ctx->rts.p;
     uint32_t *const d_cnt = (uint32_t *)tb0, *const d_csum = (uint32_t *)(tb0 + o_csum),
              *const d_coarse = (uint32_t *)(tb0 + o_coarse), *const d_nrec = (uint32_t *)(tb0 + o_nrec),

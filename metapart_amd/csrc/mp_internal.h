@@ -346,8 +346,8 @@ int snapshot_labels(mp_ctx *ctx, int s);
 // A scan by minimizer bins (mp_bins.hip): filter and union of the tuples in
 // buckets [lo, hi) without sorting them.  Plain: T segments at bounds[0..T].
 // A batch: T samples (first: T + 1 first read ids, host), each one segment;
-// *tpos takes their tuple offsets.  *done = false: nothing was joined and the
-// caller takes the radix path.
+// *tpos takes their tuple offsets.  *n_out: the tuples.  *done = false: nothing
+// was joined and the caller takes the radix path; *n_out: windows, at least as many.
 struct BinJob {
     int s = 0;
     uint64_t lo = 0, hi = 0;

@@ -61,6 +61,50 @@ def test_many_scans_keep_to_the_bins_table():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("reads,S", [(60000, 2), (60000, 8), (200000, 16)])
+def test_budgets_that_hold_the_radix_path_hold_the_bins(reads, S):
+    # budgets from what the radix path held up to where bins fit too: a scan the bins cannot hold goes by radix
+    # passes, and the pair step and the writer get their room, on a ctx's first run and on its second
+    print("gpu bins budget", reads, S, flush=True)
+    buf = mp.synth(0, n_reads=reads, read_len=150, seed=5, n_genomes=40, genome_len_min=50000, genome_len_max=300000)
+
+    def run(budget, **kw):
+        with mp.Context(k=31, hbm_budget=budget, **kw) as ctx:
+            for _ in range(2):
+                ctx.load(buf, mp.index_buffer(buf, 16))
+                r = mp.partition(ctx, S=S, want_parent=True)
+                assert not budget or ctx.device_bytes <= budget
+            return r, ctx.device_bytes
+
+    want, held = run(0, sort_digit_bits=7)
+    for f in (1.0, 1.05, 1.1, 1.2, 1.3, 2.0):
+        got, _ = run(int(held * f))
+        assert np.array_equal(got.parent, want.parent) and np.array_equal(got.W, want.W) and got.out_bytes == want.out_bytes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,reads,L,K", [(3, 300, 100, 31), (8, 4000, 150, 31), (4, 60000, 45, 31), (1, 200000, 100, 21)])
+def test_budgets_that_hold_a_radix_batch_hold_the_bins(n, reads, L, K):
+    print("gpu bins batch budget", n, reads, L, K, flush=True)
+    bufs = [mp.synth(0, n_reads=reads, read_len=L, seed=5 + i, n_genomes=10, genome_len_min=50000, genome_len_max=300000)
+            for i in range(n)]
+
+    def run(budget, **kw):
+        with mp.Context(k=K, hbm_budget=budget, **kw) as ctx:
+            for _ in range(2):
+                ctx.batch_load(bufs)
+                res, _, _ = ctx.batch_partition()
+                nb = ctx.batch_write(None)
+            return np.concatenate([ctx.batch_parent(i) for i in range(n)]), [list(map(int, r["W"])) for r in res], nb, \
+                ctx.device_bytes
+
+    want = run(0, sort_digit_bits=7)
+    for f in (1.0, 1.05, 1.1, 1.3, 2.0):
+        got = run(int(want[3] * f))
+        assert np.array_equal(got[0], want[0]) and got[1:3] == want[1:3]
+
+
+@pytest.mark.gpu
 def test_records_at_read_and_step_ends():
     # reads of k - 1 .. k + 2 bases and of every length around a step's 960
     # positions, 'N' first, last, beside and between windows
