@@ -201,7 +201,10 @@ int mp_get_bad(mp_ctx *ctx, uint8_t *bad);
 
 /* The last scan's sorted, filtered tuple array in the reference's 14-byte
  * layout (enumerateKmers.c:352-365: k-mer u64, adj u8, id/UINT32_MAX u8,
- * id%UINT32_MAX u32).  Debug and parity only. */
+ * id%UINT32_MAX u32).  After a scan that went by minimizer bins the first
+ * dump generates and sorts the tuples: it takes a radix scan's time and
+ * buffers, and may return MP_ENOMEM (labels, plan and output are unaffected).
+ * Debug and parity only. */
 int mp_dump_tuples(mp_ctx *ctx, uint8_t *dst, uint64_t cap, uint64_t *n);
 
 /* Partitioned FASTQ writer.  Builds the 16*T output streams on the device

@@ -488,6 +488,7 @@ static int sort_for_dump(mp_ctx *ctx)
 {
     uint64_t n = 0;
     int passes = 0;
+    MP_TRY(room_for_tuples(ctx, ctx->last_n));
     if (ctx->batch) {
         std::vector<uint64_t> tpos;
         float gen_ms = 0;

@@ -225,6 +225,30 @@ def test_dump_after_bins_equals_radix():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("reads,S,f", [(200000, 1, 1.05), (300000, 2, 1.05), (400000, 4, 1.1)])
+def test_dump_in_the_radix_paths_budget(reads, S, f):
+    # more windows than a scan holds the radix path's buffers for: a dump at the end sorts then, in a budget that the
+    # radix path's dump goes through in, and leaves labels and files as they are
+    print("gpu bins dump budget", reads, S, flush=True)
+    buf = mp.synth(0, n_reads=reads, read_len=150, seed=5, n_genomes=40, genome_len_min=50000, genome_len_max=300000)
+
+    def run(budget, **kw):
+        with mp.Context(k=31, hbm_budget=budget, **kw) as ctx:
+            ctx.load(buf, mp.index_buffer(buf, 16))
+            r = mp.partition(ctx, S=S, want_parent=True)
+            assert all(s["parts"] == 0 for s in r.scans)
+            d = ctx.dump_tuples()
+            assert np.array_equal(ctx.parent(), r.parent)
+            assert ctx.write_partitions(None, 1, r.W, None) == r.out_bytes
+            return r, d, ctx.device_bytes
+
+    want, dump, held = run(0, sort_digit_bits=7)
+    got, d, dev = run(int(held * f))
+    assert dev <= held * f
+    assert np.array_equal(d, dump) and np.array_equal(got.parent, want.parent) and got.out_bytes == want.out_bytes
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 3, 70, 256])
 def test_batch_equals_radix(n):
     print("gpu bins batch", n, flush=True)
