@@ -250,13 +250,11 @@ int tmp_free(mp_ctx *ctx, void *p);
 // Copies between pageable host memory and the device through the ctx's two
 // pinned buffers (mp_util.hip).  The upload is stream-ordered (src may be
 // reused at return), the downloads are complete at return.  Small copies go
-// the runtime's way.
+// the runtime's way, and all where no pinned memory is to be had.
 int copy_to_device(mp_ctx *ctx, uint8_t *dst, const char *src, uint64_t nbytes);
 int copy_to_host(mp_ctx *ctx, void *dst, const void *src, uint64_t nbytes);
 // n 32-bit labels as 64-bit ones
 int labels_to_host(mp_ctx *ctx, uint64_t *dst, const uint32_t *src, uint64_t n);
-// the device bytes [src, src + nbytes) in order, at most kStageBytes at a time
-int stream_to_host(mp_ctx *ctx, const void *src, uint64_t nbytes, const std::function<int(const char *, uint64_t)> &sink);
 
 // Exclusive scan of n u32 or u64 values into out (n+1 entries: out[n] = total).
 int scan_u32(mp_ctx *ctx, const uint32_t *in, uint64_t *out, uint64_t n);

@@ -220,13 +220,16 @@ int scan_u64(mp_ctx *ctx, const uint64_t *in, uint64_t *out, uint64_t n) { retur
 // do not).
 constexpr uint64_t kStagedUp = 32ull << 20, kStagedDown = 16ull << 20, kStagedLabels = 1ull << 20;
 
-static int stage_buffers(mp_ctx *ctx)
+// the ctx's pinned buffers and their events; false where there are none to be had: the copy goes the runtime's way
+static bool stage_buffers(mp_ctx *ctx)
 {
-    for (int b = 0; b < 2; b++) {
-        if (!ctx->stage[b]) MP_HIP(hipHostMalloc(&ctx->stage[b], kStageBytes, hipHostMallocDefault));
-        if (!ctx->stage_ev[b]) MP_HIP(hipEventCreateWithFlags(&ctx->stage_ev[b], hipEventDisableTiming));
-    }
-    return 0;
+    for (int b = 0; b < 2; b++)
+        if ((!ctx->stage[b] && hipHostMalloc(&ctx->stage[b], kStageBytes, hipHostMallocDefault) != hipSuccess) ||
+            (!ctx->stage_ev[b] && hipEventCreateWithFlags(&ctx->stage_ev[b], hipEventDisableTiming) != hipSuccess)) {
+            (void)hipGetLastError();
+            return false;
+        }
+    return true;
 }
 
 // f(a, b) over [0, n) on up to `threads` host threads, the caller among them;
@@ -250,11 +253,10 @@ template <typename F> static void host_parallel(unsigned threads, uint64_t n, F 
 
 int copy_to_device(mp_ctx *ctx, uint8_t *dst, const char *src, uint64_t nbytes)
 {
-    if (nbytes < kStagedUp) {
+    if (nbytes < kStagedUp || !stage_buffers(ctx)) {
         MP_HIP(hipMemcpyAsync(dst, src, nbytes, hipMemcpyHostToDevice, ctx->stream));
         return 0;
     }
-    MP_TRY(stage_buffers(ctx));
     for (uint64_t off = 0, c = 0; off < nbytes; off += kStageBytes, c++) {
         const int b = (int)(c & 1);
         const uint64_t len = std::min(kStageBytes, nbytes - off);
@@ -268,9 +270,10 @@ int copy_to_device(mp_ctx *ctx, uint8_t *dst, const char *src, uint64_t nbytes)
     return 0;
 }
 
-int stream_to_host(mp_ctx *ctx, const void *src, uint64_t nbytes, const std::function<int(const char *, uint64_t)> &sink)
+// the device bytes [src, src + nbytes) in order through the ctx's pinned buffers, at most kStageBytes at a time
+static int stream_to_host(mp_ctx *ctx, const void *src, uint64_t nbytes,
+                          const std::function<int(const char *, uint64_t)> &sink)
 {
-    MP_TRY(stage_buffers(ctx));
     for (int b = 0; b < 2; b++)  // an upload that is still reading them
         if (ctx->stage_used[b]) MP_HIP(hipEventSynchronize(ctx->stage_ev[b]));
     // four pieces at the least, so that a small copy overlaps its host side too
@@ -296,7 +299,7 @@ int stream_to_host(mp_ctx *ctx, const void *src, uint64_t nbytes, const std::fun
 
 int copy_to_host(mp_ctx *ctx, void *dst, const void *src, uint64_t nbytes)
 {
-    if (ctx->arena || nbytes < kStagedDown) {  // the allocation-free entry point pins nothing
+    if (ctx->arena || nbytes < kStagedDown || !stage_buffers(ctx)) {  // the allocation-free entry point pins nothing
         MP_HIP(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, ctx->stream));
         MP_HIP(hipStreamSynchronize(ctx->stream));
         return 0;
@@ -311,7 +314,7 @@ int copy_to_host(mp_ctx *ctx, void *dst, const void *src, uint64_t nbytes)
 
 int labels_to_host(mp_ctx *ctx, uint64_t *dst, const uint32_t *src, uint64_t n)
 {
-    if (n < kStagedLabels) {
+    if (n < kStagedLabels || !stage_buffers(ctx)) {
         std::vector<uint32_t> p(n);
         MP_HIP(hipMemcpyAsync(p.data(), src, n * 4, hipMemcpyDeviceToHost, ctx->stream));
         MP_HIP(hipStreamSynchronize(ctx->stream));

@@ -1,6 +1,10 @@
 """Copies through the pinned buffers: uploads at the line from which they are
 staged and at whole and odd numbers of buffers, counts and labels down, each
-against the same data by a direct copy."""
+against the same data by a direct copy; and all of them without pinned memory."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -58,3 +62,36 @@ def test_labels(n):
         ctx.batch_partition()
         want = ctx.batch_parent(0)  # 32-bit, a direct copy
     assert len(got) == n and np.array_equal(got, want)
+
+
+@pytest.mark.gpu
+def test_copies_without_pinned_memory(tmp_path):
+    # a process whose hipHostMalloc has no memory to give: uploads, counts and labels of the staged sizes go the
+    # runtime's way
+    print("gpu copies without pinned memory", flush=True)
+    shim = tmp_path / "shim.c"
+    shim.write_text("#include <stddef.h>\nint hipHostMalloc(void **p, size_t n, unsigned f) { *p = 0; return 2; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "shim.so"), str(shim)], check=True)
+    prog = """if 1:
+        import ctypes, sys
+        ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+        import numpy as np
+        import metapart_amd as mp
+        buf = mp.synth(0, n_reads=%d, seed=6, read_len=30)
+        assert buf.nbytes > 32 << 20
+        with mp.Context(k=27) as ctx:
+            ctx.load(buf, mp.index_buffer(buf, 5))
+            counts = ctx.count(want_counts=True)[3]
+            r = mp.partition(ctx, S=1, T=1, want_parent=True, build_output=False)
+        np.savez(sys.argv[2], counts=counts.sum(axis=0, dtype=np.uint64), parent=r.parent)
+    """ % (MB + 2)
+    out = str(tmp_path / "out.npz")
+    subprocess.run([sys.executable, "-c", prog, str(tmp_path / "shim.so"), out], check=True, timeout=100,
+                   cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    got = np.load(out)
+    buf = mp.synth(0, n_reads=MB + 2, seed=6, read_len=30)
+    with mp.Context(k=27) as ctx:
+        ctx.load(buf, mp.index_buffer(buf, 5))
+        counts = ctx.count(want_counts=True)[3]
+        r = mp.partition(ctx, S=1, T=1, want_parent=True, build_output=False)
+    assert np.array_equal(got["counts"], counts.sum(axis=0, dtype=np.uint64)) and np.array_equal(got["parent"], r.parent)
