@@ -2001,7 +2001,6 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     st->ms_sort_local = r;
     st->ms_filter = b;
     st->ms_union = u;
-    st->sort_passes = 2;
     st->sort_long_groups = nbig;
     st->evaluated_runs = runs_n;
     st->zeroed_runs = zeroed;

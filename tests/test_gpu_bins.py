@@ -44,6 +44,22 @@ def test_every_k_equals_radix(K):
 
 
 @pytest.mark.gpu
+def test_a_scan_by_bins_reports_no_radix_pass():
+    print("gpu bins stats", flush=True)
+    buf = mp.synth(0, n_reads=6000, seed=12, read_len=100)
+    with mp.Context(k=31) as ctx:
+        ctx.load(buf, mp.index_buffer(buf, 4))
+        r = mp.partition(ctx, build_output=False)
+        ctx.batch_load([buf, buf])
+        _, st, _ = ctx.batch_partition()
+    for s in (r.scans[0], st.as_dict()):
+        for f in ("sort_passes", "ms_sort_pass_avg", "ms_sort_hist", "ms_sort_gen", "sort_local_moved", "ms_sort_count",
+                  "sort_graph", "parts"):
+            assert s[f] == 0, f
+        assert s["ms_sort_local"] > 0
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("S,T", [(2, 1), (3, 2), (1, 16)])
 def test_scans_and_segments_equal_radix(S, T):
     print("gpu bins scans, segments", S, T, flush=True)
