@@ -196,15 +196,29 @@ def test_piled_up_bins(deep, S, T):
     assert ms[0] < ms[1] / 4, ms
 
 
+def _amplicons(n, seed):
+    """n reads that hold the 13-mer of the lowest minimizer hash between random bases: one bin of 19 n windows, as many k-mers"""
+    mer = "".join("ACGT"[(0x2545F49 >> (24 - 2 * i)) & 3] for i in range(13))
+    bases = np.frombuffer(b"ACGT", dtype=np.uint8)[np.random.default_rng(seed).integers(0, 4, (n, 137))]
+    return _fastq([r[:60].tobytes().decode() + mer + r[60:].tobytes().decode() for r in bases])
+
+
 @pytest.mark.gpu
 def test_a_pile_of_distinct_kmers_goes_to_the_radix_path():
-    # every read holds the 13-mer of the lowest minimizer hash between random bases: one bin of 266 k windows, as many k-mers
     print("gpu bins pile of distinct k-mers", flush=True)
-    rng = np.random.default_rng(3)
-    mer = "".join("ACGT"[(0x2545F49 >> (24 - 2 * i)) & 3] for i in range(13))
-    bases = np.frombuffer(b"ACGT", dtype=np.uint8)[rng.integers(0, 4, (14000, 137))]
-    seqs = [r[:60].tobytes().decode() + mer + r[60:].tobytes().decode() for r in bases]
-    _same(_fastq(seqs), 2, 31, 1, 1, bins=False)
+    _same(_amplicons(14000, 3), 2, 31, 1, 1, bins=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(1, 2), (2, 1), (2, 3)])
+def test_scans_given_up_after_marks(S, T):
+    # the same pile beside 200 k reads of several copies: three visits of it fit what the large bins may take, its
+    # parts do not, so the scan is given up after reads were marked, and a later scan puts their flags back
+    print("gpu bins given up", S, T, flush=True)
+    buf = mp.synth(0, n_reads=200000, read_len=150, seed=31, n_genomes=20, genome_len_min=100000, genome_len_max=200000)
+    both = np.concatenate([np.frombuffer(buf.tobytes(), dtype=np.uint8), _amplicons(12000, 4)])
+    a = _same(both, 6, 31, S, T, bins=False)
+    assert all(s["bad_labels"] > 0 for s in a.scans)
 
 
 @pytest.mark.gpu
@@ -280,3 +294,56 @@ def test_batch_equals_radix(n):
                         [getattr(st, f) for f in FIELDS], np.concatenate([ctx.batch_parent(i) for i in range(n)])))
     assert got[0][0] == got[1][0] and got[0][1] == got[1][1]
     assert np.array_equal(got[0][2], got[1][2])
+
+
+@pytest.fixture(scope="module")
+def big():
+    """8.3 M reads of 150 bases, more than 1.2e9 bases, from 60 genomes at some 7x, their record starts known"""
+    buf = mp.synth(0, n_reads=8300000, read_len=150, seed=41, n_genomes=60, genome_len_min=2000000, genome_len_max=4000000)
+    yield buf
+    buf.free()
+
+
+def _front(buf, reads):
+    """whole records from the front: `reads` of them, to an even number"""
+    step = buf.nbytes // 8300000 + 2  # the longest record, or more
+    v = buf.view()[:reads * step]
+    return v[:int(np.flatnonzero(v == 10)[4 * reads - 1]) + 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", list(range(25, 32)))
+def test_wide_minimizers_equal_radix(K, big):
+    # more than 200 M bases: 15-base minimizers, whole scans and scans of part of the buckets
+    print("gpu bins wide minimizers", K, flush=True)
+    buf = _front(big, 1400000)
+    for S, T in ((1, 1 + K % 4), (2 + K % 2, 1)):
+        a = _same(buf, 12, K, S, T)
+        assert sum(s["tuples"] for s in a.scans) == 1400000 * (151 - K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(1, 1), (2, 2)])
+def test_large_inputs_equal_radix(S, T, big):
+    # 13 cell bits, tiles of so many steps that records move in the larger batches
+    print("gpu bins large", S, T, flush=True)
+    a = _same(big.view(), 16, 31, S, T)
+    assert sum(s["tuples"] for s in a.scans) == 8300000 * 120
+
+
+@pytest.mark.gpu
+def test_large_batch_equals_radix(big):
+    print("gpu bins large batch", flush=True)
+    v = big.view()
+    cut = [0] + [len(_front(big, n)) for n in (2, 700000, 5000000)] + [big.nbytes]
+    bufs = [v[a:b] for a, b in zip(cut, cut[1:])]
+    got = []
+    for kw in ({}, {"sort_digit_bits": 7}):
+        with mp.Context(k=31, **kw) as ctx:
+            ctx.batch_load(bufs)
+            res, st, _ = ctx.batch_partition()
+            assert (st.ms_sort_gen == 0) == (not kw)
+            got.append(([[r[f] for f in ("reads", "tuples", "components", "largest")] + list(map(int, r["W"])) for r in res],
+                        [getattr(st, f) for f in FIELDS], [ctx.batch_parent(i) for i in range(len(bufs))]))
+    assert got[0][:2] == got[1][:2]
+    assert all(np.array_equal(a, b) for a, b in zip(got[0][2], got[1][2]))
