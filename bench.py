@@ -46,6 +46,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+VALU_PEAK_GOPS = 1024 * 2.4 / 4  # wave instructions: 1024 SIMDs at 2.4 GHz, four cycles each
+RUNS_VALU_PER_64 = 294  # of bin_runs per 64 windows (counters: 11.04e9 at 2.4e9 windows)
 TUPLE_BYTES = 13  # u64 k-mer + u32 label + u8 adj
 
 
@@ -322,7 +324,8 @@ def main():
             if sort_ms > 0 else 0.0}
     if by_bins:
         ms = float(sc["ms_enumerate"]) + sort_ms
-        gbs = runs_bytes / (runs_ms * 1e-3) / 1e9 if runs_ms > 0 else 0.0
+        insts = n / 64 * RUNS_VALU_PER_64
+        rate = insts / (runs_ms * 1e-3) / 1e9 if runs_ms > 0 else 0.0
         stages = {
             "bin_records": stage(float(sc["ms_enumerate"]), bases * 3 // 8, "2-bit and 'N' streams read"),
             "bin_runs": stage(runs_ms, runs_bytes, "0.375 B per base read, 4 B per tuple written at most (the kernels "
@@ -330,7 +333,8 @@ def main():
             "refilter": stage(float(sc["ms_filter"]), 2 * N, "filtered and BAD flags"),
             "union": stages["union"]}
         roofline = {"bound": "valu", "kernel": "bin_runs_kernel (runs of equal k-mers in LDS tables, filter)",
-                    "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS, "traffic": None,
+                    "achieved": rate, "peak": VALU_PEAK_GOPS, "unit": "G vector instructions/s",
+                    "frac": rate / VALU_PEAK_GOPS, "instructions_source": "profiles/bins_c2_20M.md", "traffic": None,
                     "traffic_source": None, "bytes_per_launch": runs_bytes, "launch_ms": runs_ms, "tuples": n}
         sort = {"passes": passes, "by": "minimizer bins (no radix pass)", "algorithmic_bytes": runs_bytes, "ms": ms,
                 "hbm_frac": runs_bytes / (ms * 1e-3) / 1e12 / (HBM_PEAK_GBS / 1e3) if ms > 0 else 0.0}

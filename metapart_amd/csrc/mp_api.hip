@@ -419,8 +419,7 @@ int mp_scan(mp_ctx *ctx, int s, uint64_t lo, uint64_t hi, const uint64_t *seg_bo
         MP_TRY(enumerate_scan(ctx, s, lo, hi, &n));
     } else {
         gen.reset(new GenSource());
-        const bool all = lo == 0 && expected_tuples != 0 && expected_tuples == ctx->kmer_total;
-        MP_TRY(gen_histograms(ctx, s, lo, hi, scan_pass_mask(ctx->cfg.k), all, gen.get(), &n));
+        MP_TRY(gen_histograms(ctx, s, lo, hi, scan_pass_mask(ctx->cfg.k), false, gen.get(), &n));
     }
     hipEventRecord(ctx->ev[1], ctx->stream);
     if (expected_tuples && n != expected_tuples)

@@ -32,7 +32,8 @@
 // What this path leaves to the radix sort (mp_sort.hip), see bins_apply():
 // k below 20 or 32 (the reference's forward code quirk), 3-minimizer scans,
 // reads with letters whose neighbour class the 2-bit code cannot give, scans
-// in bucket parts, and inputs whose windows pile up in a few minimizers.
+// in bucket parts, and inputs whose windows pile up in a few minimizers with
+// too many k-mers for bin_runs_big to be the faster way.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -57,6 +58,7 @@ constexpr int kBigRec = 64;         // records that bin_runs_big expands at once
 constexpr int kBinWit = 8;          // witnesses per bin (bin_runs)
 constexpr int kMaxSeg = 256;        // segments (samples of a batch)
 constexpr int kStripes = 64;        // copies of the global counters, a cache line each
+constexpr uint64_t kCellBases = 1200000000;  // bases from which a coarse bin has 8192 cells instead of 2048
 
 struct BinRec {  // a super-k-mer: consecutive windows of one read with one minimizer
     uint64_t a;      // first window's base (40 bits) | windows << 40 (5) | flags << 45 (2) | cell << 47 (13)
@@ -514,7 +516,10 @@ __global__ __launch_bounds__(kNC) void bin_col_apply_kernel(uint32_t *__restrict
 // write 96 bytes of a bin at once: 140 M records of 12 M reads 3.18 -> 1.85 ms,
 // 2.10 with 3072.  A tile of few steps holds little more than one such batch,
 // and there two workgroups of 3072 on a CU overlap better: 4 scans of 2 M reads
-// (40 steps, some 4000 records a tile) 2.28 -> 1.10 ms, 1.35 with 6144.
+// (40 steps, some 4000 records a tile) 2.28 -> 1.10 ms, 1.35 with 6144.  One
+// scan, records made and moved, 3072 against 6144: 210 Mb 0.59, 0.63 ms, 450 Mb
+// 1.21, 1.11, 900 Mb 2.38, 2.21, 1.8 Gb 4.78, 4.43; four scans 2.27, 2.52; 4.27,
+// 4.42; 8.46, 8.40; 16.6, 16.8.
 constexpr int kScThreads = 1024;
 constexpr int kTileSteps = 512;  // wave steps of a tile at most
 constexpr int kScLongTile = 32;  // wave steps per wave of a tile from which the batch is 6144
@@ -1646,7 +1651,13 @@ static void launch_scan(mp_ctx *ctx, uint32_t tiles, const BinScan &P)
 }
 
 // M-mers of 13 bases (33 M canonical values, far more than there are cells);
-// shorter ones below k = 22, so that a window keeps 10 of them
+// shorter ones below k = 22, so that a window keeps 10 of them.  wide: of 15
+// (0.5 G values), which spread the minimizers of a large input over more cells
+// and make some more records.  Records, grouping and runs of one scan of 150-base
+// reads, 13 against 15 bases: 210 Mb 2.47, 2.51 ms (k = 25 2.66, 2.82), 450 Mb
+// 5.02, 4.95 (5.45, 5.74), 1.2 Gb 16.4, 15.0 (17.9, 16.7); four scans of 1.2 Gb
+// 26.7, 27.1.  They cross between 0.2 and 1.2 Gb, later for smaller k.
+constexpr uint64_t kWideBases = 200000000;
 static int scan_launch(mp_ctx *ctx, uint32_t tiles, bool wide, const BinScan &P)
 {
     switch (wide && P.K >= 25 ? 100 + P.K : P.K) {
@@ -1715,7 +1726,9 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     const int steps = (int)std::min<uint64_t>(128, (nsteps + 4 * 8192 - 1) / (4 * 8192));
     const uint32_t tiles = (uint32_t)((nsteps + 4 * (uint64_t)steps - 1) / (4 * (uint64_t)steps));
     const uint32_t chunks = (tiles + kColTiles - 1) / kColTiles;
-    const int cell_bits = tb > 1200000000ull ? 13 : 11;  // cells of a few hundred windows
+    // cells of a few hundred windows.  One scan, 11 against 13 bits: 450 Mb 4.99, 4.96 ms, 750 Mb 8.4, 7.9, 1.2 Gb
+    // 15.0, 13.1, 1.8 Gb 24.0, 21.1 (four scans 9.9, 10.0; 16.5, 16.3; 27.3, 26.7; 43.1, 41.0): they cross at 450 Mb
+    const int cell_bits = tb > kCellBases ? 13 : 11;
     struct Cleanup {  // the snapshot serves the kernels of this scan (and a later dump, which sets it again)
         mp_ctx *c;
         ~Cleanup() { c->use_labsnap = false; }
@@ -1820,7 +1833,7 @@ int bins_scan(mp_ctx *ctx, const BinJob &job, mp_scan_stats *st, std::vector<uin
     S.erank = d_rank;
     S.cnt = d_cnt;
     S.ctl = d_ctl;
-    MP_TRY(scan_launch(ctx, tiles, tb > 200000000ull, S));
+    MP_TRY(scan_launch(ctx, tiles, tb > kWideBases, S));
     hipLaunchKernelGGL(bin_col_sum_kernel, dim3(chunks), dim3(kNC), 0, ctx->stream, (const uint32_t *)d_cnt, tiles, d_csum);
     hipLaunchKernelGGL(bin_col_scan_kernel, dim3(1), dim3(kNC), 0, ctx->stream, d_csum, chunks, d_coarse);
     hipLaunchKernelGGL(bin_col_apply_kernel, dim3(chunks), dim3(kNC), 0, ctx->stream, d_cnt, tiles,

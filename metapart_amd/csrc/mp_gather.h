@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kGLanes) void gather_kernel(const uint8_t *__restri
                 if (beg(mid) <= y) lo = mid; else hi = mid - 1;
             }
             // the unit's bytes come from item j, then (past an item end) from the
-            // next non-empty item, both read as 16 aligned-load bytes at once;
+            // next non-empty item, each read as 16 bytes at its own alignment;
             // a unit over three or more items takes its remaining bytes singly
             uint32_t j = lo;
             const uint32_t eA = min(beg(j + 1) - y, valid);

@@ -1364,7 +1364,7 @@ __global__ __launch_bounds__(256) void sample_stats_kernel(const uint32_t *__res
 
 static inline unsigned nblk(uint64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-// every read (except BAD ones, when bad is given) to its root
+// sizes[r] of every root r (sizes_kernel)
 static int component_sizes(mp_ctx *ctx, const uint32_t *parent, uint32_t *sizes, uint64_t N)
 {
     hipLaunchKernelGGL(sizes_clear_kernel, dim3(nblk(N)), dim3(256), 0, ctx->stream, parent, sizes, N);
@@ -1374,6 +1374,7 @@ static int component_sizes(mp_ctx *ctx, const uint32_t *parent, uint32_t *sizes,
     return 0;
 }
 
+// every read (except BAD ones, when bad is given) to its root
 static int compress_labels(mp_ctx *ctx, uint32_t *parent, const uint8_t *bad, uint64_t N)
 {
     if (N == 0) return 0;

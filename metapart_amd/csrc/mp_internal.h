@@ -176,7 +176,6 @@ struct mp_ctx {
     mp::DevArray khist;   // a batch's counts of the k-mer bytes its radix passes read, per sample
     bool khist_valid = false;
     uint32_t khist_mask = 0;  // passes (bit 1 + byte) khist counts
-    uint64_t kmer_total = 0;  // k-mers of the loaded reads (last m-mer histogram)
     // writer
     mp::DevArray out, items[2], ilens[2], iaux[2];
     // pinned host staging of large uploads (two buffers, one copy in flight)

@@ -488,7 +488,6 @@ static int count_plain_partitioned(mp_ctx *ctx, const KParams &K, const uint64_t
     H.toff = (const uint64_t *)ctx->wg_off.p;
     ctx->khist_valid = false;  // a radix sort of these reads counts its own digits
     ctx->gcnt_valid = false;
-    ctx->kmer_total = 0;
     if (H.total == 0) return 0;
     hipLaunchKernelGGL(hist_tiles_kernel, dim3(1), dim3(256), 0, ctx->stream, H, d_tile0);
     hipLaunchKernelGGL(hist_pos_kernel<0>, dim3((unsigned)NT), dim3(kHLanes), 0, ctx->stream, H);
@@ -501,7 +500,6 @@ static int count_plain_partitioned(mp_ctx *ctx, const KParams &K, const uint64_t
     MP_HIP(hipMemcpyAsync(bounds.data(), d_bounds, 8 * (nparts + 1), hipMemcpyDeviceToHost, ctx->stream));
     MP_HIP(hipStreamSynchronize(ctx->stream));
     const uint64_t total = bounds[nparts];
-    ctx->kmer_total = total;
     if (total == 0) return 0;
     // the low bits stage in the second tuple buffer, unused until the first scan's sort
     MP_TRY(ensure(ctx, ctx->keys[1], total * sizeof(uint16_t) + 64));
